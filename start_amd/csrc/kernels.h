@@ -50,6 +50,8 @@ struct RunK {
     double s0, s1;       // E = s0 * E_0 + s1 * E_1
     uint32_t key;        // folded into the variate key
     uint32_t first;      // load index of the run's first particle
+    float log2_conc;     // log2(conc), +inf outside [1e-35, 1e35]
+    int32_t pad;
     int64_t node_base;   // run * n_nodes
     int64_t tri_base;    // run * n_tris
 };
@@ -122,13 +124,14 @@ constexpr int kMaxPushSlots = 4;
 
 struct StepParams {
     double dt;
-    double lo[3], hi[3];
+    double lo[3], hi[3];      // expanded bounding box
     uint64_t seed;
     const RunK* runs;         // run table (one entry for a single simulation)
     int32_t model;
     int32_t em_push;
     int32_t charge;
-    int32_t nspecies;
+    int32_t bbox_covers;      // the expanded bounding box holds every node (with room for FP32 rounding)
+    float log2_dt;            // log2(dt) + log2(1.001 * 2^32), +inf for dt outside [1e-35, 1e35]
     const int64_t* n_active;  // live particles lead the arrays after a sort
     double* zero_charge;      // node-charge buffers of the next launch, cleared here
     int64_t charge_len;       // n_runs * n_nodes

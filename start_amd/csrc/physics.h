@@ -39,6 +39,9 @@ struct SpeciesK {
     // push increments per tet; -1 computed in the kernel; -2 charge 0 (the
     // increment is E*q, a signed zero)
     int32_t push_slot;
+    // estimate of the collision probability in the log domain, without the gas
+    // concentration and the time step: log2(P / (n dt)) = coll_a + coll_b log2(|v|^2)
+    float coll_a, coll_b;
     int32_t pad;
 };
 
@@ -78,6 +81,19 @@ __host__ __device__ inline void variates(uint64_t seed, uint32_t run, uint32_t p
     uint64_t b = ((uint64_t)w[2] << 21) | (w[3] >> 11);
     ua = (double)a * two_m53;
     ub = (double)b * two_m53;
+}
+
+// The first word of a step's draw 0: u1 = (word 0 and 21 bits of word 1) 2^-53.
+// The empty asm keeps the compiler from hoisting the twenty round keys out of
+// a step loop, where they would be spilled scalar registers read back one lane
+// at a time.
+__device__ inline uint32_t variate_word(uint64_t seed, uint32_t run, uint32_t pid, uint32_t step)
+{
+    uint32_t w[4], lo = (uint32_t)seed, hi = (uint32_t)(seed >> 32) ^ run;
+    asm volatile("" : "+s"(lo));
+    asm volatile("" : "+v"(pid));
+    philox4x32_10(pid, 0u, step, 0u, lo, hi, w);
+    return w[0];
 }
 
 // x rounded to FP32 stochastically: to the farther of the two neighbouring

@@ -431,6 +431,15 @@ int sort_now(start_ctx* c)
     return START_OK;
 }
 
+// log2 of a factor of the collision probability for the kernels' FP32
+// estimate: -inf for 0 (the probability is 0), +inf ("always ask the exact
+// test") outside the range in which the FP32 bound holds.
+double log2_factor(double v)
+{
+    if (v == 0.0) return -INFINITY;
+    return v >= 1e-35 && v <= 1e35 ? log2(v) : INFINITY;
+}
+
 // Species constants with the reference's expressions (HSModel.cpp:8-12,
 // VHSModel.cpp:12-22, VSSModel.cpp:32), evaluated once.
 SpeciesK species_constants(const start_species_desc& s, const start_gas_desc& g)
@@ -449,6 +458,16 @@ SpeciesK species_constants(const start_species_desc& s, const start_gas_desc& g)
     k.mass_ct = t_mass / (t_mass + p_mass);
     k.inv_alpha = g.alpha != 0.0 ? 1. / g.alpha : 0.0;
     k.push_slot = s.charge == 0.0 ? -2 : -1;
+    // P / (n dt) = sigma |v|, sigma = sigma_hs (HS) or pi vhs_c (two_kt / (m_r |v|^2))^vhs_exp
+    if (g.model == START_MODEL_HS) {
+        k.coll_a = (float)log2_factor(k.sigma_hs);
+        k.coll_b = 0.5f;
+    } else {
+        const double e = k.vhs_exp, a = log2_factor(kPi * k.vhs_c);
+        const bool sane = std::isfinite(a) && k.m_r >= 1e-35 && k.m_r <= 1e35 && e >= -1.0 && e <= 1.0;
+        k.coll_a = sane ? (float)(a + e * log2(k.two_kt / k.m_r)) : INFINITY;
+        k.coll_b = sane ? (float)(0.5 - e) : 0.5f;
+    }
     k.pad = 0;
     return k;
 }
@@ -565,6 +584,7 @@ int check_kernel_errors(start_ctx* c)
 
 int upload_runs(start_ctx* c)
 {
+    for (RunK& r : c->runs) r.log2_conc = (float)log2_factor(r.conc);
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     if (c->d_runs) (void)hipFree(c->d_runs);
     c->d_runs = nullptr;
@@ -671,7 +691,17 @@ StepParams step_params(const start_ctx* c)
     S.model = c->prm.gas.model;
     S.em_push = c->prm.em_push;
     S.charge = c->prm.charge_every_step;
-    S.nspecies = (int32_t)c->species.size();
+    S.log2_dt = (float)(log2_factor(c->prm.dt) + (32.0 + log2(1.001)));
+    // an owned position is inside the expanded bbox if that holds every node;
+    // the mixed path compares FP32 sums, within 4 ulps of the true position
+    bool covers = true;
+    for (int k = 0; k < 3; ++k) {
+        const double m = !c->mixed ? 0.0
+                                   : 1e-6 * std::max(std::max(fabs(c->hm.bbox_lo[k]), fabs(c->hm.bbox_hi[k])),
+                                                     std::max(fabs(c->hm.node_lo[k]), fabs(c->hm.node_hi[k])));
+        covers = covers && c->hm.bbox_lo[k] + m <= c->hm.node_lo[k] && c->hm.node_hi[k] + m <= c->hm.bbox_hi[k];
+    }
+    S.bbox_covers = covers ? 1 : 0;
     S.n_active = c->d_nactive;
     S.charge_len = c->charge_len();
     S.settle = c->record ? c->d_settle : nullptr;
@@ -1182,6 +1212,7 @@ int start_create(start_ctx** out, const start_mesh_desc* mesh, const start_param
     r0.s0 = 1.0;
     r0.s1 = 0.0;
     r0.key = params->run;
+    r0.log2_conc = (float)log2_factor(r0.conc);
     c->runs.assign(1, r0);
     std::vector<float> g32;
     if (c->mixed) {

@@ -1,13 +1,13 @@
 // Step kernels of the particle path (gfx950).
 //
-// One step = prologue (clear node charge, reset work list)
-//          -> step_main   one thread per particle: skip rules, push, move,
-//                         collision, certified same-tet relocation, charge
-//          -> step_resolve one thread per deferred particle: exact tet walk
-//                         along the step segment, surface hit and settle,
-//                         grid search for degenerate cases, charge.
-// The rare exact work (tet crossings, faces, hits) is compacted into a work
-// list so the streaming kernel stays short and free of divergent branches.
+// One launch = step_main    one thread per particle: skip rules, push, move,
+//                           collision, certified relocation, charge, for the
+//                           steps fused in the launch
+//           -> step_resolve one thread per deferred particle: exact tet walk
+//                           along the step segment, surface hit and settle,
+//                           grid search for degenerate cases, charge.
+// The rare exact work (segments through edges and vertices, end points on
+// faces) is compacted into a work list so the streaming kernel stays short.
 #include <type_traits>
 
 #include "kernels.h"
@@ -334,54 +334,76 @@ __device__ inline void scatter4(double* __restrict__ node_charge, const int4& nv
 // particles sorted by tet a 256-particle block touches ~100-150 nodes instead
 // of issuing 1,024 global atomics.
 template <int Bits>
-__device__ inline void lds_charge_add(int32_t* hk, double* hv, double* __restrict__ node_charge, int32_t node,
-                                      double val)
+__device__ inline uint32_t hash_slot(int32_t node)
 {
-    uint32_t h = ((uint32_t)node * 2654435761u) >> (32 - Bits);
-    // (left to the compiler to unroll: a rolled loop made the FP64 streaming
-    // kernel 7% slower)
-    // (reading the slot before the compare-and-swap, to skip it for nodes
-    // already present, made the kernel 17-35% slower)
-    for (int probe = 0; probe < 32; ++probe) {
-        int32_t prev = atomicCAS(&hk[h], -1, node);
+    return ((uint32_t)node * 2654435761u) >> (32 - Bits);
+}
+
+// The probes after the first, for a node whose first slot holds another one.
+// A rolled loop: unrolled 32-fold at every insertion it was three quarters of
+// the kernel's 17,000 instructions, and its nested branches spilled about
+// 2,000 SGPRs.
+template <int Bits>
+__device__ inline void lds_charge_probe(int32_t* hk, double* hv, double* __restrict__ node_charge, int32_t node,
+                                        uint32_t h, double val)
+{
+#pragma unroll 1
+    for (int probe = 1; probe < 32; ++probe) {
+        h = (h + 1) & ((1u << Bits) - 1u);
+        const int32_t prev = atomicCAS(&hk[h], -1, node);
         if (prev == -1 || prev == node) {
             lds_add_f64(&hv[h], val);
             return;
         }
-        h = (h + 1) & ((1u << Bits) - 1u);
     }
     global_add_f64(&node_charge[node], val);  // crowded table: straight to memory
 }
 
-// Node window: a block's tet-sorted particles touch nodes within a few
-// thousand ids of the lowest one (the node numbering of a structured mesh
-// puts a cell's nodes one layer, (nx+1)(ny+1) ids, apart), so nodes in
-// [wbase, wbase + Win) are summed in a plain LDS array by an LDS FP64 add,
-// without the hash's compare-and-swap; the others go to the hash.
-template <int Bits, int Win>
-__device__ inline void lds_window_add(int32_t* hk, double* hv, double* wv, int32_t wbase,
-                                      double* __restrict__ node_charge, int32_t node, double val)
-{
-    if (Win > 0) {
-        const uint32_t off = (uint32_t)(node - wbase);
-        if (off < (uint32_t)Win) {
-            lds_add_f64(&wv[off], val);
-            return;
-        }
-    }
-    lds_charge_add<Bits>(hk, hv, node_charge, node, val);
-}
-
-// base: offset of the run's node-charge array (0 for a single simulation)
+// The four contributions of one tet.  Node window (Win > 0): a block's
+// tet-sorted particles touch nodes within a few thousand ids of the lowest one
+// (the node numbering of a structured mesh puts a cell's nodes one layer,
+// (nx+1)(ny+1) ids, apart), so nodes in [wbase, wbase + Win) are summed in a
+// plain LDS array without the hash's compare-and-swap; the others go to the
+// hash.  The four compare-and-swaps are issued together (their results are a
+// full LDS latency away) and only a node that finds its first slot taken
+// probes on.  base: offset of the run's node-charge array (0 for a single
+// simulation).
 template <int Bits, int Win>
 __device__ inline void lds_scatter4(int32_t* hk, double* hv, double* wv, int32_t wbase,
-                                    double* __restrict__ node_charge, const int4& nv, int32_t base, double q,
-                                    const double lam[4])
+                                    double* __restrict__ node_charge, const int4& nv, int32_t base,
+                                    const double val[4])
 {
-    lds_window_add<Bits, Win>(hk, hv, wv, wbase, node_charge, base + nv.x, q * lam[0]);
-    lds_window_add<Bits, Win>(hk, hv, wv, wbase, node_charge, base + nv.y, q * lam[1]);
-    lds_window_add<Bits, Win>(hk, hv, wv, wbase, node_charge, base + nv.z, q * lam[2]);
-    lds_window_add<Bits, Win>(hk, hv, wv, wbase, node_charge, base + nv.w, q * lam[3]);
+    const int32_t node[4] = {base + nv.x, base + nv.y, base + nv.z, base + nv.w};
+    bool todo[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        todo[q] = true;
+        if (Win > 0) {
+            const uint32_t off = (uint32_t)(node[q] - wbase);
+            if (off < (uint32_t)Win) {
+                lds_add_f64(&wv[off], val[q]);
+                todo[q] = false;
+            }
+        }
+    }
+    if (Win > 0 && !(todo[0] || todo[1] || todo[2] || todo[3])) return;
+    uint32_t h[4];
+    int32_t prev[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        h[q] = hash_slot<Bits>(node[q]);
+        prev[q] = node[q];
+        if (Win == 0 || todo[q]) prev[q] = atomicCAS(&hk[h[q]], -1, node[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const bool here = prev[q] == -1 || prev[q] == node[q];
+        if (here && (Win == 0 || todo[q])) lds_add_f64(&hv[h[q]], val[q]);
+        todo[q] = !here;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (todo[q]) lds_charge_probe<Bits>(hk, hv, node_charge, node[q], h[q], val[q]);
 }
 
 // ---------------------------------------------------------------------------
@@ -475,7 +497,7 @@ __device__ inline void bary_at(const DevMesh& M, int32_t t, float x, float y, fl
 // bbox test of the frozen rule on the stored position
 __device__ inline bool in_bbox_at(const DevMesh& M, const StepParams& S, int32_t t, double x, double y, double z)
 {
-    return x >= S.lo[0] && x <= S.hi[0] && y >= S.lo[1] && y <= S.hi[1] && z >= S.lo[2] && z <= S.hi[2];
+    return (x >= S.lo[0]) & (x <= S.hi[0]) & (y >= S.lo[1]) & (y <= S.hi[1]) & (z >= S.lo[2]) & (z <= S.hi[2]);
 }
 __device__ inline bool in_bbox_at(const DevMesh& M, const StepParams& S, int32_t t, float x, float y, float z)
 {
@@ -486,8 +508,8 @@ __device__ inline bool in_bbox_at(const DevMesh& M, const StepParams& S, int32_t
         ay += a2.z;
         az += a2.w;
     }
-    return ax >= (float)S.lo[0] && ax <= (float)S.hi[0] && ay >= (float)S.lo[1] && ay <= (float)S.hi[1] &&
-           az >= (float)S.lo[2] && az <= (float)S.hi[2];
+    return (ax >= (float)S.lo[0]) & (ax <= (float)S.hi[0]) & (ay >= (float)S.lo[1]) & (ay <= (float)S.hi[1]) &
+           (az >= (float)S.lo[2]) & (az <= (float)S.hi[2]);
 }
 
 template <typename R>
@@ -547,55 +569,57 @@ struct LdsSink {
     double* wv;
     int32_t wbase;
     double* nc;
-    __device__ void add4(const int4& nv, int32_t base, double q, const double lam[4])
+    __device__ void add4(const int4& nv, int32_t base, const double val[4])
     {
-        lds_scatter4<Bits, Win>(hk, hv, wv, wbase, nc, nv, base, q, lam);
+        lds_scatter4<Bits, Win>(hk, hv, wv, wbase, nc, nv, base, val);
     }
 };
 struct GlobalSink {
     double* nc;
-    __device__ void add4(const int4& nv, int32_t base, double q, const double lam[4])
+    __device__ void add4(const int4& nv, int32_t base, const double val[4])
     {
-        scatter4(nc + base, nv, q, lam);
+        scatter4(nc + base, nv, 1.0, val);
     }
 };
-// Per-particle accumulation across the steps of a launch: a particle that
-// stays in one tet adds q*lambda into four registers, and its sums go to the
-// inner sink only when it changes tet or the launch ends.  base is the offset
-// of the particle's run in the node-charge buffer.
+// Per-particle accumulation across the steps of a launch: while the particle
+// stays in one tet the charge weights lambda are summed in four registers; the
+// sums, times the particle's charge q, go to the inner sink only when it
+// changes tet or the launch ends.  base is the offset of the particle's run in
+// the node-charge buffer; t < 0 or q = 0: nothing is scattered.
 template <typename Inner>
 struct RegSink {
     Inner inner;
-    int32_t cur;
-    int32_t base;
     double a0, a1, a2, a3;
-    __device__ void flush(const DevMesh& M)
+    __device__ void add(double w, const double lam[4])
     {
-        if (cur >= 0) {
-            double v[4] = {a0, a1, a2, a3};
-            inner.add4(M.tnode[cur], base, 1.0, v);
-        }
-        cur = -1;
+        a0 = __builtin_fma(w, lam[0], a0);
+        a1 = __builtin_fma(w, lam[1], a1);
+        a2 = __builtin_fma(w, lam[2], a2);
+        a3 = __builtin_fma(w, lam[3], a3);
+    }
+    __device__ void flush(const DevMesh& M, int32_t t, int32_t base, double q)
+    {
+        if (t >= 0 && q != 0.0) flush_nodes(M.tnode[t], base, q);
         a0 = a1 = a2 = a3 = 0.0;
     }
-    __device__ void add(const DevMesh& M, int32_t t, double q, const double lam[4])
+    __device__ void flush_nodes(const int4& nv, int32_t base, double q)
     {
-        if (t != cur) {
-            flush(M);
-            cur = t;
-        }
-        a0 += q * lam[0];
-        a1 += q * lam[1];
-        a2 += q * lam[2];
-        a3 += q * lam[3];
+        const double v[4] = {q * a0, q * a1, q * a2, q * a3};
+        inner.add4(nv, base, v);
+        a0 = a1 = a2 = a3 = 0.0;
     }
     // The flush at the end of a tile, where every lane of the wavefront is
     // active: lanes of one run of equal (tet, run offset) -- neighbours in the
     // tet-sorted order -- sum their four weights into the run's first lane
     // (segmented Hillis-Steele over the wavefront), which alone goes to the
     // inner sink.  One LDS insertion per run instead of one per particle.
-    __device__ void flush_wave(const DevMesh& M)
+    __device__ void flush_wave(const DevMesh& M, int32_t cur, int32_t base, double q)
     {
+        if (q == 0.0) cur = -1;
+        a0 *= q;
+        a1 *= q;
+        a2 *= q;
+        a3 *= q;
         const int lane = threadIdx.x & 63;
         const int32_t up_t = __shfl_up(cur, 1), up_b = __shfl_up(base, 1);
         const bool head = lane == 0 || up_t != cur || up_b != base;
@@ -614,7 +638,7 @@ struct RegSink {
             }
         }
         if (!head) cur = -1;  // summed into the run's first lane
-        flush(M);
+        flush(M, cur, base, 1.0);
     }
     // flush_wave with the node window of an LDS sink, when no charge has gone
     // to LDS yet in this tile (single-step launches): the window starts at the
@@ -626,8 +650,13 @@ struct RegSink {
     // tet, runs longer than four are rare; the full six rounds cost more
     // cross-lane moves than the inserts they save (measured: 63.5 against
     // 65.8 us per single-step FP64 launch on the large box).
-    __device__ void flush_wave_window(const DevMesh& M, int32_t* s_wbase)
+    __device__ void flush_wave_window(const DevMesh& M, int32_t cur, int32_t base, double q, int32_t* s_wbase)
     {
+        if (q == 0.0) cur = -1;
+        a0 *= q;
+        a1 *= q;
+        a2 *= q;
+        a3 *= q;
         const int lane = threadIdx.x & 63;
         const int32_t up_t = __shfl_up(cur, 1), up_b = __shfl_up(base, 1);
         const bool head = lane == 0 || up_t != cur || up_b != base;
@@ -660,11 +689,9 @@ struct RegSink {
         __syncthreads();
         inner.wbase = __builtin_amdgcn_readfirstlane(*s_wbase);
         if (cur >= 0) {
-            double v[4] = {a0, a1, a2, a3};
-            inner.add4(nv, base, 1.0, v);
+            const double v[4] = {a0, a1, a2, a3};
+            inner.add4(nv, base, v);
         }
-        cur = -1;
-        a0 = a1 = a2 = a3 = 0.0;
     }
 };
 
@@ -681,43 +708,68 @@ __device__ __noinline__ bool collides_exact64(int model, double sigma_hs, double
 }
 
 template <typename R>
-__device__ inline bool collides(const StepParams& S, const SpeciesK& k, double conc, R vx, R vy, R vz, double u1)
+__device__ inline bool collides(int model, double dt, const SpeciesK& k, double conc, R vx, R vy, R vz, double u1)
 {
     R vm = m_sqrt<R>(vx * vx + vy * vy + vz * vz);
-    if (S.model == 1) {  // HS: no transcendental, evaluate directly
+    if (model == 1) {  // HS: no transcendental, evaluate directly
         CollideK<R> ck{(R)k.sigma_hs, (R)0, (R)0, (R)0, (R)0, (R)0, (R)0, (R)0};
-        return (R)u1 < collision_probability<R>(1, ck, (R)conc, (R)S.dt, vm);
+        return (R)u1 < collision_probability<R>(1, ck, (R)conc, (R)dt, vm);
     }
     float vmf = (float)vm;
     CollideK<float> cf{(float)k.sigma_hs, (float)k.vhs_c, (float)k.two_kt, (float)k.m_r, (float)k.vhs_exp,
                        0.0f, 0.0f, 0.0f};
-    float p32 = collision_probability<float>(S.model, cf, (float)conc, (float)S.dt, vmf);
+    float p32 = collision_probability<float>(model, cf, (float)conc, (float)dt, vmf);
     if (!std::is_same<R, double>::value) return (float)u1 < p32;
     double p = (double)p32;
     if (!(p > 1e-30 && p < 1e30))  // outside the range the FP32 bound covers
-        return collides_exact64(S.model, k.sigma_hs, k.vhs_c, k.two_kt, k.m_r, k.vhs_exp, conc, S.dt, (double)vm, u1);
+        return collides_exact64(model, k.sigma_hs, k.vhs_c, k.two_kt, k.m_r, k.vhs_exp, conc, dt, (double)vm, u1);
     if (u1 < p * (1.0 - 1e-4)) return true;
     if (u1 >= p * (1.0 + 1e-4)) return false;
-    return collides_exact64(S.model, k.sigma_hs, k.vhs_c, k.two_kt, k.m_r, k.vhs_exp, conc, S.dt, (double)vm, u1);
+    return collides_exact64(model, k.sigma_hs, k.vhs_c, k.two_kt, k.m_r, k.vhs_exp, conc, dt, (double)vm, u1);
 }
 
-// Post-collision velocity of a particle whose collision test passed (rare:
-// about once per 1e4 particle-steps), out of line to keep the streaming kernel
-// lean.  The variates u2, u3 are drawn here, not by the caller, so that few of
-// the caller's registers are live at the call; arguments and result by value
-// so nothing of the caller escapes to memory.  FP64 in both precisions:
-// evaluated in FP32, sin(chi) = sqrt((1 - cos)(1 + cos)) of a forward scatter
-// (cos near 1 from an FP64 variate rounded to FP32) loses most of its digits.
+// The collision of one step for the few draws may_collide() lets through
+// (about once per 1e3-1e4 particle-steps): the decision, then the
+// post-collision velocity; unchanged if there is none.  Out of line to keep
+// the streaming kernel lean; the variates are drawn here so that few of the
+// caller's registers are live at the call; arguments and result by value so
+// nothing of the caller escapes to memory.  The scattering is FP64 in both
+// precisions: evaluated in FP32, sin(chi) = sqrt((1 - cos)(1 + cos)) of a
+// forward scatter (cos near 1 from an FP64 variate rounded to FP32) loses most
+// of its digits.
 struct V3 {
     double x, y, z;
 };
-__device__ __noinline__ V3 collide_velocity(int model, const SpeciesK* k, uint64_t seed, uint32_t key, uint32_t vid,
-                                            uint32_t step, double vx, double vy, double vz)
+template <typename R>
+__device__ __noinline__ V3 collide_step(int model, double dt, const SpeciesK* k, double conc, uint64_t seed,
+                                        uint32_t key, uint32_t vid, uint32_t step, double vx, double vy, double vz)
 {
-    double u2, u3;
-    variates(seed, key, vid, step, 1u, u2, u3);
-    scatter_velocity(model, k->mass_cp, k->mass_ct, k->inv_alpha, u2, u3, vx, vy, vz);
+    double u1, u2, u3;
+    variates(seed, key, vid, step, 0u, u1, u2);
+    if (collides<R>(model, dt, *k, conc, (R)vx, (R)vy, (R)vz, u1)) {
+        variates(seed, key, vid, step, 1u, u2, u3);
+        scatter_velocity(model, k->mass_cp, k->mass_ct, k->inv_alpha, u2, u3, vx, vy, vz);
+    }
     return V3{vx, vy, vz};
+}
+
+// Whether the collision test u1 < P of a step can pass, from the first variate
+// word w0 alone (u1 >= w0 2^-32) and an FP32 estimate of P in the log domain:
+// log2(P 2^32) = ca + cb log2(|v|^2), ca from the host's FP64 constants
+// (species, gas, time step; +inf where one of them is outside the range the
+// FP32 bound covers) plus 32 and log2(1.001).  The exponents stay below 200 in
+// magnitude, so ca, the product and the sum err by less than 5e-5 and v_log /
+// v_exp by an ulp: 1e-4 relative in P, a tenth of the margin.  "false" is
+// certain; "true" (P itself, and one draw in a thousand beyond it) goes to
+// collide_step, which decides as the reference does.  This replaces an FP32
+// pow, two square roots and the second variate word in every step.
+template <typename R>
+__device__ inline bool may_collide(uint32_t w0, float ca, float cb, R v2)
+{
+    const float v2f = (float)v2;
+    const float p = __builtin_amdgcn_exp2f(ca + cb * __builtin_amdgcn_logf(v2f));
+    // (below 1e-6 the FP32 probability of the mixed path leaves its range)
+    return !((float)w0 > p && (std::is_same<R, double>::value || v2f > 1e-6f));
 }
 
 // Barycentric classification with a certified threshold: strictly inside,
@@ -766,53 +818,61 @@ __device__ inline double walk_tol(double tau, const double l[4])
     return tau * fmax(1.0, 0.5 * s) * (1.0 + 1e-6);
 }
 
-__device__ inline int walk64(const DevMesh& M, int32_t t, const double* p0, const double* p1, int32_t& out)
+// The face of a tet through which the segment p0 -> p1 leaves it: l1 the
+// coordinates of p1 with their bound t1, l0() those of p0 (only needed when p1
+// lies beyond several faces).  kInHere: p1 is inside; kNoFace: not certain.
+enum { kInHere = -1, kNoFace = -2 };
+template <typename L0>
+__device__ inline int exit_face(double tau, const double l1[4], L0 l0_of)
 {
     constexpr double kE = 1.1102230246251565e-16;  // 2^-53
-    const double tau = M.tau;
+    const double t1 = walk_tol(tau, l1);
+    int nneg = 0, npos = 0, f1 = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        npos += l1[q] > t1;
+        if (l1[q] < -t1) {
+            ++nneg;
+            f1 = q;
+        }
+    }
+    if (npos + nneg < 4) return kNoFace;  // p1 too close to a face plane
+    if (nneg == 0) return kInHere;
+    if (nneg == 1) return f1;
+    double l0[4];
+    l0_of(l0);
+    const double t0 = walk_tol(tau, l0);
+    int exit_f = kNoFace;
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        bool first = l1[f] < -t1;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if (g == f) continue;
+            const double a = l0[f] * l1[g], b = l0[g] * l1[f];
+            const double err = t0 * (fabs(l1[f]) + fabs(l1[g]) + 2.0 * t1) +
+                               t1 * (fabs(l0[f]) + fabs(l0[g]) + 2.0 * t0) + 4.0 * kE * (fabs(a) + fabs(b));
+            first = first && (!(l1[g] < -t1) || a - b > err);
+        }
+        if (first && exit_f == kNoFace) exit_f = f;
+    }
+    return exit_f;
+}
+
+__device__ inline int walk64(const DevMesh& M, int32_t t, const double* p0, const double* p1, int32_t& out)
+{
     int32_t cur = t;
+#pragma unroll 1
     for (int hop = 0; hop < kWalkHops; ++hop) {
         double l1[4];
         bary_at(M, cur, p1[0], p1[1], p1[2], l1);
-        const double t1 = walk_tol(tau, l1);
-        int nneg = 0, npos = 0, f1 = 0;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            npos += l1[q] > t1;
-            if (l1[q] < -t1) {
-                ++nneg;
-                f1 = q;
-            }
-        }
-        if (npos + nneg < 4) return kWalkUnsure;  // p1 too close to a face plane of cur
-        if (nneg == 0) {
+        const int f = exit_face(M.tau, l1, [&](double* l0) { bary_at(M, cur, p0[0], p0[1], p0[2], l0); });
+        if (f == kNoFace) return kWalkUnsure;
+        if (f == kInHere) {
             out = cur;
             return kWalkInside;
         }
-        int exit_f = f1;
-        if (nneg > 1) {
-            double l0[4];
-            bary_at(M, cur, p0[0], p0[1], p0[2], l0);
-            const double t0 = walk_tol(tau, l0);
-            exit_f = -1;
-            for (int f = 0; f < 4 && exit_f < 0; ++f) {
-                if (!(l1[f] < -t1)) continue;
-                bool first = true;
-                for (int g = 0; g < 4; ++g) {
-                    if (g == f || !(l1[g] < -t1)) continue;
-                    const double a = l0[f] * l1[g], b = l0[g] * l1[f];
-                    const double err = t0 * (fabs(l1[f]) + fabs(l1[g]) + 2.0 * t1) +
-                                       t1 * (fabs(l0[f]) + fabs(l0[g]) + 2.0 * t0) + 4.0 * kE * (fabs(a) + fabs(b));
-                    if (!(a - b > err)) {
-                        first = false;
-                        break;
-                    }
-                }
-                if (first) exit_f = f;
-            }
-            if (exit_f < 0) return kWalkUnsure;
-        }
-        const int32_t code = nth(M.tnbr[cur], exit_f);
+        const int32_t code = nth(M.tnbr[cur], f);
         if (code <= -2) {
             out = -2 - code;
             return kWalkSurface;
@@ -825,8 +885,8 @@ __device__ inline int walk64(const DevMesh& M, int32_t t, const double* p0, cons
 
 enum StepOutcome { kDone = 0, kSettledNow = 1, kDeferNow = 2, kFrozenNow = 3 };
 
-// settle record for the adjoint (rare; out of line, scalar arguments)
-__device__ __noinline__ void record_settle(SettleRec* rec, uint32_t pidx, uint32_t step, double x0, double y0,
+// settle record for the adjoint
+__device__ inline void record_settle(SettleRec* rec, uint32_t pidx, uint32_t step, double x0, double y0,
                                            double z0)
 {
     SettleRec r;
@@ -906,200 +966,204 @@ __device__ __forceinline__ void track_hit(const DevMesh& M, const StepParams& S,
 // position in R (FP32 in the owner's frame in mixed mode), velocity FP64:
 // accumulated in FP32, a per-tet increment much smaller than |v| rounds the
 // same way step after step, and the velocity drifts linearly (about 6e-8 of
-// |v| per step)
+// |v| per step).  v2 = |v|^2 in R, kept with the velocity.
 template <typename R>
 struct PState {
     R x, y, z;
     double vx, vy, vz;
+    R v2;
     int32_t t, f;
+    __device__ void set_v2()
+    {
+        const R a = (R)vx, b = (R)vy, c = (R)vz;
+        v2 = a * a + b * b + c * c;
+    }
 };
 
-// One step of one particle (ParticleDynamicsProcessor.cpp:166-199 stage order,
-// then the relocation and charge of the next gather).  Relocations that the
-// barycentric maps cannot certify return kDeferNow with the state at x1 in the
-// frame of the unchanged owner; the caller resolves them exactly.
-// The owning tet's data is re-read each step (L1/L2 hits while the particle
-// stays in it) to keep the register footprint of the streaming kernel small.
-// The same index, through an empty asm statement (no instruction): the
-// compiler cannot reuse the per-lane addresses of the state loads at the start
-// of a step for the stores at its end, which kept eight 64-bit addresses live
-// across the FP64 step and spilled them to scratch; the stores recompute
-// theirs from the index and the kernel-argument bases instead.  (In the mixed
-// kernels the allocation without it measured faster.)
-__device__ __forceinline__ int64_t fresh_index(int64_t i)
+// sqrt(v2) < 10 without the root: the root is correctly rounded, so it is
+// below 10 exactly for v2 below the smallest number whose root rounds to 10.
+__device__ inline bool too_slow(double v2) { return v2 < 0x1.8ffffffffffffp+6; }
+__device__ inline bool too_slow(float v2) { return v2 < 0x1.8ffffep+6f; }
+
+// What stays the same over a particle's steps of a launch.
+struct PConst {
+    const SpeciesK* k;
+    const RunK* rk;
+    uint32_t vid;   // variate counter
+    uint32_t key;   // the run's part of the variate key
+    float ca, cb;   // may_collide
+};
+__device__ inline PConst particle_const(const StepParams& S, const SpeciesK* k, const RunK* rk, uint32_t vid)
 {
-    asm volatile("" : "+v"(i));
-    return i;
+    return PConst{k, rk, vid, rk->key, k->coll_a + rk->log2_conc + S.log2_dt, k->coll_b};
 }
 
-struct StepResult {
-    int outcome;
-    int32_t hit_tri;
+// face codes and nodes of a particle's tet
+struct TetRows {
+    int4 nbr, node;
 };
 
-template <typename R, bool kBatch, bool kWalk, typename Sink>
-__device__ __forceinline__ StepResult step_one(const DevMesh& M, const StepParams& S, const SpeciesK& k,
-                                               const RunK* __restrict__ rk, uint32_t vid, uint32_t step,
-                                               int remaining, PState<R>& s, Sink& sink)
+// The record of one tet as a particle's step uses it: the barycentric map
+// (FP64: v0 and A; mixed: A) and the push increment h of the particle in it.
+template <typename R>
+struct TetRec {
+    static constexpr int kLen = std::is_same<R, double>::value ? 12 : 9;
+    int32_t t;  // -1: nothing loaded
+    R g[kLen];
+    R hx, hy, hz;
+
+    // The record of tet (-1: none).  rows: null, or where the tet's face codes
+    // and nodes go (LDS; a lane that leaves the tet then needs no load before
+    // that of the next tet's record).
+    template <bool kBatch>
+    __device__ inline void load(const DevMesh& M, const StepParams& S, const SpeciesK& k,
+                                const RunK* __restrict__ rk, int32_t tet, TetRows* rows = nullptr)
+    {
+        if (tet >= 0) {
+            load_in<kBatch>(M, S, k, rk, tet, rows);
+        } else {  // outside the mesh: no push, and no point is certified inside
+            t = tet;
+#pragma unroll
+            for (int q = 0; q < kLen; ++q) g[q] = R(0);
+            hx = hy = hz = R(-0.0);
+        }
+    }
+    template <bool kBatch>
+    __device__ inline void load_in(const DevMesh& M, const StepParams& S, const SpeciesK& k,
+                                   const RunK* __restrict__ rk, int32_t tet, TetRows* rows = nullptr)
+    {
+        t = tet;
+        if constexpr (std::is_same<R, double>::value) {
+            const double* p = M.geo + 12 * (int64_t)tet;
+#pragma unroll
+            for (int q = 0; q < 12; ++q) g[q] = p[q];
+        } else {
+            const float4* a = reinterpret_cast<const float4*>(M.geo32) + 3 * (int64_t)tet;
+            const float4 a0 = a[0], a1 = a[1];
+            g[0] = a0.x;
+            g[1] = a0.y;
+            g[2] = a0.z;
+            g[3] = a0.w;
+            g[4] = a1.x;
+            g[5] = a1.y;
+            g[6] = a1.z;
+            g[7] = a1.w;
+            g[8] = a[2].x;
+        }
+        if (rows) {
+            rows->nbr = M.tnbr[tet];
+            rows->node = M.tnode[tet];
+        }
+        load_h<kBatch>(M, S, k, rk, tet);
+    }
+    // h = (((E*q)/m)*dt)/2 (Particle.cpp:199-207); -0 where the push is skipped,
+    // which leaves (v + h) + h = v bit for bit.  From the table of the species,
+    // or evaluated here with the same operations: per lane once per tet it
+    // enters, not once per step (three FP64 divisions).
+    template <bool kBatch>
+    __device__ inline void load_h(const DevMesh& M, const StepParams& S, const SpeciesK& k,
+                                  const RunK* __restrict__ rk, int32_t tet)
+    {
+        if (!kBatch && S.em_push && k.push_slot >= 0) {
+            load_push(M, k.push_slot, tet, hx, hy, hz);
+            return;
+        }
+        const R dt = (R)S.dt, qc = (R)k.charge, m = (R)k.mass;
+        R ex, ey, ez;
+        run_field<R, kBatch>(M, rk, tet, ex, ey, ez);
+        const bool push = S.em_push && dt != R(0) && !(ex == R(0) && ey == R(0) && ez == R(0));
+        ex = ex * qc;
+        ey = ey * qc;
+        ez = ez * qc;
+        if (kBatch || k.push_slot != -2) {  // (charge 0 in a single simulation: the signed zero E*q)
+            ex = ((ex / m) * dt) / R(2);
+            ey = ((ey / m) * dt) / R(2);
+            ez = ((ez / m) * dt) / R(2);
+        }
+        hx = push ? ex : R(-0.0);
+        hy = push ? ey : R(-0.0);
+        hz = push ? ez : R(-0.0);
+    }
+    __device__ inline void bary(R x, R y, R z, double lam[4]) const
+    {
+        if constexpr (std::is_same<R, double>::value) {
+            bary64(g, x, y, z, lam);
+        } else {
+            const float l1 = (g[0] * x + g[1] * y) + g[2] * z;
+            const float l2 = (g[3] * x + g[4] * y) + g[5] * z;
+            const float l3 = (g[6] * x + g[7] * y) + g[8] * z;
+            const float l0 = 1.0f - ((l1 + l2) + l3);
+            lam[0] = l0;
+            lam[1] = l1;
+            lam[2] = l2;
+            lam[3] = l3;
+        }
+    }
+};
+
+// Where a step's end point went (relocate): the position in its owner's frame,
+// the owner, the outcome, the triangle hit, and its coordinates in the owner.
+struct Lam {
+    double l[4];
+};
+template <typename R>
+struct Relocated {
+    R x, y, z;
+    int32_t t;
+    int32_t outcome;
+    int32_t hit_tri;
+    Lam lam;
+};
+// Relocation of a step whose end point x1 is not certified inside the owner t
+// by its coordinates `l` there: faces, neighbours, the multi-tet walk.  x0
+// strictly inside t.  Certified cases: x1 strictly inside the owner (by the
+// FP64 map), or strictly outside exactly one face f and strictly inside the
+// other three (the segment leaves through the open face f), or the walk's;
+// the rest (kDeferNow, x1 in the frame of t) needs the exact walk.
+// vneg: sign bits of the velocity (mixed only).
+template <typename R, bool kWalk>
+__device__ inline Relocated<R> relocate(const DevMesh& M, int32_t t, int32_t vneg, R x0, R y0, R z0, R x1, R y1,
+                                              R z1, Lam l)
 {
     const double tau = tau_of<R>(M);
-    // 2. |v| < 10 m/s and 3. outside the expanded bbox: frozen this step and
-    //    every later one (nothing changes its state); it still carries charge
-    const R vxr = (R)s.vx, vyr = (R)s.vy, vzr = (R)s.vz;
-    R vmod = m_sqrt<R>(vxr * vxr + vyr * vyr + vzr * vzr);
-    bool frozen = vmod < R(10) || !in_bbox_at(M, S, s.t, s.x, s.y, s.z);
-    double lam[4];
-    if (frozen) {
-        if (S.charge && s.t >= 0 && k.charge != 0.0) {
-            bary_at(M, s.t, s.x, s.y, s.z, lam);
-            sink.add(M, s.t, k.charge * (double)remaining, lam);
-        }
-        return StepResult{kFrozenNow, -1};
+    int fneg = 0;
+    int cls = classify(l.l, tau, fneg);
+    if (!std::is_same<R, double>::value && cls == kUncertain) {
+        // FP32 too close to a face: certify with the FP64 map at the FP64
+        // absolute position of the stored FP32 state
+        double p1[3];
+        abs_pos(M, t, x1, y1, z1, p1);
+        bary_at(M, t, p1[0], p1[1], p1[2], l.l);
+        cls = classify(l.l, M.tau, fneg);
     }
-    R dt = (R)S.dt;
-    // 4. push with the owning tet's field (ParticleDynamicsProcessor.cpp:179-180)
-    if (S.em_push && s.t >= 0) {
-        if (!kBatch && k.push_slot >= 0) {
-            // h = (((E*q)/m)*dt)/2 of this tet and species, evaluated per field
-            // and time step with the same operations (-0 where the push is
-            // skipped, which leaves v unchanged bit for bit)
-            R hx, hy, hz;
-            load_push(M, k.push_slot, s.t, hx, hy, hz);
-            s.vx = (s.vx + (double)hx) + (double)hx;
-            s.vy = (s.vy + (double)hy) + (double)hy;
-            s.vz = (s.vz + (double)hz) + (double)hz;
-        } else if (!kBatch && k.push_slot == -2) {
-            // charge 0: with m > 0 and dt > 0 the increment is the signed zero E*q
-            R ex, ey, ez;
-            load_E(M, s.t, ex, ey, ez);
-            if (dt != R(0) && !(ex == R(0) && ey == R(0) && ez == R(0))) {
-                const R q = (R)k.charge;
-                const double hx = (double)(ex * q), hy = (double)(ey * q), hz = (double)(ez * q);
-                s.vx = (s.vx + hx) + hx;
-                s.vy = (s.vy + hy) + hy;
-                s.vz = (s.vz + hz) + hz;
-            }
-        } else {
-            R ex, ey, ez;
-            run_field<R, kBatch>(M, rk, s.t, ex, ey, ez);
-            push<R>(ex, ey, ez, (R)k.charge, (R)k.mass, dt, s.vx, s.vy, s.vz);
+    if (cls == kInside) return Relocated<R>{x1, y1, z1, t, kDone, -1, l};
+    if (cls == kOneFace) {
+        const int32_t code = nth(M.tnbr[t], fneg);
+        if (code <= -2) return Relocated<R>{x1, y1, z1, t, kSettledNow, -2 - code};  // crosses this triangle first
+        // to the neighbour (or out through a face with no triangle)
+        double p1[3];
+        abs_pos(M, t, x1, y1, z1, p1);
+        R nx, ny, nz;
+        to_frame(M, code, p1, nx, ny, nz);
+        if (code == -1) return Relocated<R>{nx, ny, nz, -1, kDone, -1};
+        bary_at(M, code, nx, ny, nz, l.l);
+        int f2;
+        int c2 = classify(l.l, tau, f2);
+        if (!std::is_same<R, double>::value && c2 == kUncertain) {
+            double q[3];
+            abs_pos(M, code, nx, ny, nz, q);
+            bary_at(M, code, q[0], q[1], q[2], l.l);
+            c2 = classify(l.l, M.tau, f2);
         }
+        if (c2 == kInside) return Relocated<R>{nx, ny, nz, code, kDone, -1, l};
     }
-    // 6. move (Particle.cpp:157-165).  Mixed: the end point in the owner's
-    //    frame is rounded to FP32 stochastically, with 30 hashed bits of
-    //    (particle, step, seed).
-    R x1, y1, z1;
-    if constexpr (std::is_same<R, double>::value) {
-        x1 = s.x + s.vx * S.dt;
-        y1 = s.y + s.vy * S.dt;
-        z1 = s.z + s.vz * S.dt;
-    } else {
-        const uint32_t h = hash3(vid, step, (uint32_t)S.seed ^ rk->key);
-        x1 = round_stochastic((double)s.x + s.vx * S.dt, h & 0x3ffu);
-        y1 = round_stochastic((double)s.y + s.vy * S.dt, (h >> 10) & 0x3ffu);
-        z1 = round_stochastic((double)s.z + s.vz * S.dt, h >> 22);
-    }
-    if (x1 == s.x && y1 == s.y && z1 == s.z) {  // degenerate segment (:188-190)
-        if (S.charge && s.t >= 0 && k.charge != 0.0) {
-            bary_at(M, s.t, s.x, s.y, s.z, lam);
-            sink.add(M, s.t, k.charge, lam);
-        }
-        return StepResult{kDone, -1};
-    }
-    // 7. gas collision (ParticlePhysicsUpdater.cpp:20-24)
-    if (S.model != 0) {
-        double u1, u1b;
-        variates(S.seed, rk->key, vid, step, 0u, u1, u1b);
-        if (collides<R>(S, k, rk->conc, (R)s.vx, (R)s.vy, (R)s.vz, u1)) {
-            V3 nv = collide_velocity(S.model, &k, S.seed, rk->key, vid, step, s.vx, s.vy, s.vz);
-            s.vx = nv.x;
-            s.vy = nv.y;
-            s.vz = nv.z;
-        }
-    }
-    // 8. relocation and surface hit on the segment x -> x1.  Certified cases:
-    //    x1 strictly inside the owner, or strictly outside exactly one face f
-    //    and strictly inside the other three (the segment leaves through the
-    //    open face f).  The rest needs the exact walk.
-    bool certified = false;
-    if (s.t >= 0 && (s.f & kStrict)) {
-        bary_at(M, s.t, x1, y1, z1, lam);
-        int fneg = 0;
-        int cls = classify(lam, tau, fneg);
-        if (!std::is_same<R, double>::value && cls == kUncertain) {
-            // FP32 too close to a face: certify with the FP64 map at the FP64
-            // absolute position of the stored FP32 state
-            double p1[3];
-            abs_pos(M, s.t, x1, y1, z1, p1);
-            bary_at(M, s.t, p1[0], p1[1], p1[2], lam);
-            cls = classify(lam, M.tau, fneg);
-        }
-        if (cls == kInside) {
-            certified = true;
-        } else if (cls == kOneFace) {
-            int32_t code = nth(M.tnbr[s.t], fneg);
-            if (code <= -2) {
-                s.x = x1;  // crosses this surface triangle first
-                s.y = y1;
-                s.z = z1;
-                return StepResult{kSettledNow, -2 - code};
-            }
-            // to the neighbour (or out through a face with no triangle)
-            double p1[3];
-            abs_pos(M, s.t, x1, y1, z1, p1);
-            R nx, ny, nz;
-            to_frame(M, code, p1, nx, ny, nz);
-            if (code == -1) {
-                s.t = -1;
-                s.f &= ~kStrict;
-                s.x = nx;
-                s.y = ny;
-                s.z = nz;
-                return StepResult{kDone, -1};
-            }
-            bary_at(M, code, nx, ny, nz, lam);
-            int f2;
-            int c2 = classify(lam, tau, f2);
-            if (!std::is_same<R, double>::value && c2 == kUncertain) {
-                double q[3];
-                abs_pos(M, code, nx, ny, nz, q);
-                bary_at(M, code, q[0], q[1], q[2], lam);
-                c2 = classify(lam, M.tau, f2);
-            }
-            if (c2 == kInside) {
-                s.t = code;
-                x1 = nx;
-                y1 = ny;
-                z1 = nz;
-                certified = true;
-            }
-        }
-    }
-    if (s.t < 0) {
-        // outside the mesh: a segment wholly beyond one face of the nodes'
-        // bounding box meets no tet and no surface triangle (exact compares)
-        double p0[3], p1[3];
-        abs_pos(M, -1, s.x, s.y, s.z, p0);
-        abs_pos(M, -1, x1, y1, z1, p1);
-        bool away = false;
-#pragma unroll
-        for (int q = 0; q < 3; ++q)
-            away = away || (p0[q] < M.node_lo[q] && p1[q] < M.node_lo[q]) ||
-                   (p0[q] > M.node_hi[q] && p1[q] > M.node_hi[q]);
-        if (away) {
-            s.x = x1;
-            s.y = y1;
-            s.z = z1;
-            return StepResult{kDone, -1};
-        }
-    }
-    if (kWalk && !certified && s.t >= 0 && (s.f & kStrict)) {
+    if (kWalk) {
         // a segment through several tets: the certified FP64 walk
         double p0[3], p1[3];
-        abs_pos(M, s.t, s.x, s.y, s.z, p0);
-        abs_pos(M, s.t, x1, y1, z1, p1);
+        abs_pos(M, t, x0, y0, z0, p0);
+        abs_pos(M, t, x1, y1, z1, p1);
         int32_t where = -1;
-        int w = walk64(M, s.t, p0, p1, where);
+        int w = walk64(M, t, p0, p1, where);
         if (!std::is_same<R, double>::value && w == kWalkUnsure) {
             // FP32 end points lie on a lattice (~1e-9 m apart in a 1 cm tet),
             // and about 1e-7 of them land exactly on a face plane (one through
@@ -1108,42 +1172,32 @@ __device__ __forceinline__ StepResult step_one(const DevMesh& M, const StepParam
             // planes like x == y, which an equal move would keep it on) -- within
             // the FP32 state's own rounding -- and certified again; a point that
             // stays uncertain goes to the exact walk as before.
-            const R ux = s.vx < R(0) ? R(-INFINITY) : R(INFINITY);
-            const R uy = s.vy < R(0) ? R(-INFINITY) : R(INFINITY);
-            const R uz = s.vz < R(0) ? R(-INFINITY) : R(INFINITY);
+            const R ux = (vneg & 1) ? R(-INFINITY) : R(INFINITY);
+            const R uy = (vneg & 2) ? R(-INFINITY) : R(INFINITY);
+            const R uz = (vneg & 4) ? R(-INFINITY) : R(INFINITY);
             x1 = m_nextafter(x1, ux);
             y1 = m_nextafter(m_nextafter(y1, uy), uy);
             z1 = m_nextafter(m_nextafter(m_nextafter(z1, uz), uz), uz);
-            abs_pos(M, s.t, x1, y1, z1, p1);
-            w = walk64(M, s.t, p0, p1, where);
+            abs_pos(M, t, x1, y1, z1, p1);
+            w = walk64(M, t, p0, p1, where);
         }
         if (w == kWalkSurface) {
-            s.x = x1;  // crosses this surface triangle first
-            s.y = y1;
-            s.z = z1;
-            return StepResult{kSettledNow, where};
+            return Relocated<R>{x1, y1, z1, t, kSettledNow, where};  // crosses this surface triangle first
         }
         if (w != kWalkUnsure) {
             R nx, ny, nz;
             to_frame(M, w == kWalkOpen ? -1 : where, p1, nx, ny, nz);
-            if (w == kWalkOpen) {
-                s.t = -1;
-                s.f &= ~kStrict;
-                s.x = nx;
-                s.y = ny;
-                s.z = nz;
-                return StepResult{kDone, -1};
-            }
+            if (w == kWalkOpen) return Relocated<R>{nx, ny, nz, -1, kDone, -1};
             // the position as stored (FP32 in its owner's frame in mixed mode)
             // must itself be strictly inside the owner the walk found
-            bary_at(M, where, nx, ny, nz, lam);
+            bary_at(M, where, nx, ny, nz, l.l);
             int f2;
-            int c2 = classify(lam, tau, f2);
+            int c2 = classify(l.l, tau, f2);
             if (!std::is_same<R, double>::value && c2 == kUncertain) {
                 double q[3];
                 abs_pos(M, where, nx, ny, nz, q);
-                bary_at(M, where, q[0], q[1], q[2], lam);
-                c2 = classify(lam, M.tau, f2);
+                bary_at(M, where, q[0], q[1], q[2], l.l);
+                c2 = classify(l.l, M.tau, f2);
             }
             if (!std::is_same<R, double>::value) {
                 // Rounding the end point to FP32 in the new frame can put the
@@ -1157,35 +1211,145 @@ __device__ __forceinline__ StepResult step_one(const DevMesh& M, const StepParam
                     abs_pos(M, where, nx, ny, nz, q);
                     where = code;
                     to_frame(M, where, q, nx, ny, nz);
-                    bary_at(M, where, nx, ny, nz, lam);
-                    c2 = classify(lam, tau, f2);
+                    bary_at(M, where, nx, ny, nz, l.l);
+                    c2 = classify(l.l, tau, f2);
                     if (c2 == kUncertain) {
                         abs_pos(M, where, nx, ny, nz, q);
-                        bary_at(M, where, q[0], q[1], q[2], lam);
-                        c2 = classify(lam, M.tau, f2);
+                        bary_at(M, where, q[0], q[1], q[2], l.l);
+                        c2 = classify(l.l, M.tau, f2);
                     }
                 }
             }
-            if (c2 == kInside) {
-                s.t = where;
-                x1 = nx;
-                y1 = ny;
-                z1 = nz;
-                certified = true;
-            }
+            if (c2 == kInside) return Relocated<R>{nx, ny, nz, where, kDone, -1, l};
         }
     }
-    if (!certified) {
-        s.x = x1;
-        s.y = y1;
-        s.z = z1;
-        return StepResult{kDeferNow, -1};
+    return Relocated<R>{x1, y1, z1, t, kDeferNow, -1};
+}
+
+// Frozen this step and every later one of the launch (nothing changes its
+// state; it still carries charge): 2. |v| < 10 m/s or 3. outside the expanded
+// bbox (ParticleDynamicsProcessor.cpp:166-176).  Where the expanded bbox holds
+// every node, an owned point is inside it.
+template <typename R>
+__device__ inline bool is_frozen(const DevMesh& M, const StepParams& S, const PState<R>& s)
+{
+    return too_slow(s.v2) || ((s.t < 0 || !S.bbox_covers) && !in_bbox_at(M, S, s.t, s.x, s.y, s.z));
+}
+
+// 4. push with the owning tet's field (ParticleDynamicsProcessor.cpp:179-180);
+// rec: the owner's record.
+template <typename R>
+__device__ inline void push_in(PState<R>& s, const TetRec<R>& rec)
+{
+    s.vx = (s.vx + (double)rec.hx) + (double)rec.hx;
+    s.vy = (s.vy + (double)rec.hy) + (double)rec.hy;
+    s.vz = (s.vz + (double)rec.hz) + (double)rec.hz;
+    s.set_v2();
+}
+
+// 6. move (Particle.cpp:157-165): the end point in the owner's frame.  Mixed:
+// rounded to FP32 stochastically, with 30 hashed bits of (particle, step, seed).
+template <typename R>
+__device__ inline void end_point(const StepParams& S, uint32_t vid, uint32_t key, uint32_t step, const PState<R>& s,
+                                 R& x1, R& y1, R& z1)
+{
+    if constexpr (std::is_same<R, double>::value) {
+        x1 = s.x + s.vx * S.dt;
+        y1 = s.y + s.vy * S.dt;
+        z1 = s.z + s.vz * S.dt;
+    } else {
+        const uint32_t h = hash3(vid, step, (uint32_t)S.seed ^ key);
+        x1 = round_stochastic((double)s.x + s.vx * S.dt, h & 0x3ffu);
+        y1 = round_stochastic((double)s.y + s.vy * S.dt, (h >> 10) & 0x3ffu);
+        z1 = round_stochastic((double)s.z + s.vz * S.dt, h >> 22);
     }
+}
+
+// 7. gas collision (ParticlePhysicsUpdater.cpp:20-24) of a draw that may collide
+template <typename R>
+__device__ inline void collide(const StepParams& S, const PConst& c, uint32_t step, PState<R>& s)
+{
+    const V3 nv = collide_step<R>(S.model, S.dt, c.k, c.rk->conc, S.seed, c.key, c.vid, step, s.vx, s.vy, s.vz);
+    s.vx = nv.x;
+    s.vy = nv.y;
+    s.vz = nv.z;
+    s.set_v2();
+}
+
+// Outside the mesh: a segment wholly beyond one face of the nodes' bounding box
+// meets no tet and no surface triangle (exact compares).
+template <typename R>
+__device__ inline bool stays_outside(const DevMesh& M, const PState<R>& s, R x1, R y1, R z1)
+{
+    const double p0[3] = {(double)s.x, (double)s.y, (double)s.z}, p1[3] = {(double)x1, (double)y1, (double)z1};
+    bool away = false;
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+        away = away || (p0[q] < M.node_lo[q] && p1[q] < M.node_lo[q]) ||
+               (p0[q] > M.node_hi[q] && p1[q] > M.node_hi[q]);
+    return away;
+}
+
+// 8. relocation and surface hit on the segment from the state's position to x1.
+// Leaves the state at the end point (kDeferNow: in the frame of the unchanged
+// owner; the caller resolves it exactly) and, for kDone with an owner, the end
+// point's coordinates in lam.
+template <typename R, bool kWalk>
+__device__ inline int move_to(const DevMesh& M, PState<R>& s, bool strict, R x1, R y1, R z1, Lam& lam,
+                              int32_t& hit_tri)
+{
+    if (s.t >= 0 && strict) {
+        const int32_t vneg = (s.vx < 0.0 ? 1 : 0) | (s.vy < 0.0 ? 2 : 0) | (s.vz < 0.0 ? 4 : 0);
+        const Relocated<R> r = relocate<R, kWalk>(M, s.t, vneg, s.x, s.y, s.z, x1, y1, z1, lam);
+        s.x = r.x;
+        s.y = r.y;
+        s.z = r.z;
+        s.t = r.t;
+        lam = r.lam;
+        hit_tri = r.hit_tri;
+        return r.outcome;
+    }
+    const int outcome = s.t < 0 && stays_outside(M, s, x1, y1, z1) ? kDone : kDeferNow;
     s.x = x1;
     s.y = y1;
     s.z = z1;
-    if (S.charge && s.t >= 0 && k.charge != 0.0) sink.add(M, s.t, k.charge, lam);
-    return StepResult{kDone, -1};
+    return outcome;
+}
+
+// One step of one particle (ParticleDynamicsProcessor.cpp:166-199 stage order,
+// then the relocation and charge of the next gather), as the straggler kernel
+// takes it; step_tile runs the same stages with the common case first.
+template <typename R, bool kBatch, bool kWalk, typename Sink>
+__device__ inline int step_one(const DevMesh& M, const StepParams& S, const PConst& c, uint32_t step, int remaining,
+                               PState<R>& s, TetRec<R>& rec, Sink& sink, int32_t& hit_tri)
+{
+    Lam lam;
+    if (is_frozen(M, S, s)) {
+        if (s.t >= 0) {
+            bary_at(M, s.t, s.x, s.y, s.z, lam.l);
+            sink.add((double)remaining, lam.l);
+        }
+        return kFrozenNow;
+    }
+    if (s.t >= 0) {
+        if (s.t != rec.t) rec.template load<kBatch>(M, S, *c.k, c.rk, s.t);
+        push_in(s, rec);
+    }
+    R x1, y1, z1;
+    end_point(S, c.vid, c.key, step, s, x1, y1, z1);
+    const bool still = x1 == s.x && y1 == s.y && z1 == s.z;  // degenerate segment (:188-190)
+    if (!still && S.model != 0 && may_collide<R>(variate_word(S.seed, c.key, c.vid, step), c.ca, c.cb, s.v2))
+        collide(S, c, step, s);
+    int outcome = kDone;
+    if (s.t >= 0) rec.bary(x1, y1, z1, lam.l);
+    const int32_t t_before = s.t;
+    if (!still) {
+        outcome = move_to<R, kWalk>(M, s, (s.f & kStrict) != 0, x1, y1, z1, lam, hit_tri);
+        if (s.t < 0) s.f &= ~kStrict;
+    }
+    if (s.t != t_before) sink.flush(M, S.charge ? t_before : -1, (int32_t)c.rk->node_base, c.k->charge);
+    if (outcome == kDone && s.t >= 0) sink.add(1.0, lam.l);
+    return outcome;
 }
 
 // ---------------------------------------------------------------------------
@@ -1201,163 +1365,526 @@ __global__ void prologue_kernel(double* __restrict__ a, double* __restrict__ b, 
     }
 }
 
+// Arguments of the streaming kernels.
+template <typename R>
+struct StepArgs {
+    DevMesh M;
+    DevParticles<R> P;
+    StepParams S;
+    const SpeciesK* sp;
+    double* node_charge;
+    WorkItem* wl;
+    unsigned long long* cnt;
+    unsigned long long* tri_count;
+};
+// A particle that settled (flags, hit, counters, records) or deferred (work
+// list) in a step from px, py, pz in tet t_before; s: its state after it, which
+// the caller has stored.
+template <typename R, bool kTrack>
+__device__ inline void finish_rare(const StepArgs<R>& A, int outcome, uint32_t row, uint32_t li, const RunK* rk,
+                                   const PState<R>& s, int32_t t_before, R px, R py, R pz, uint32_t step, int32_t ks,
+                                   int32_t hit_tri)
+{
+    const StepParams& S = A.S;
+    if (outcome == kSettledNow) {
+        A.P.flags[row] = (s.f | kSettled) & ~kStrict;
+        A.P.hit[row] = hit_tri;
+        atomicAdd(&A.tri_count[rk->tri_base + hit_tri], 1ull);
+        S.settle_log[atomicAdd(&A.cnt[kCntSettled], 1ull)] = li;
+        if (S.settle || kTrack) {
+            double a[3];
+            abs_pos(A.M, t_before, px, py, pz, a);
+            if (S.settle) record_settle(S.settle, li, step, a[0], a[1], a[2]);
+            if (kTrack) track_hit<R>(A.M, S, li, a, s.t, s.x, s.y, s.z, hit_tri);
+        }
+        return;
+    }
+    // work list: one atomic for the lanes that defer together
+    const unsigned long long dm = __ballot(true);
+    const int lane = __lane_id();
+    const int leader = __ffsll((long long)dm) - 1;
+    unsigned int slot = 0u;
+    if (lane == leader)
+        slot = (unsigned int)atomicAdd(&A.cnt[kCntWork + 2 * S.work_slot], (unsigned long long)__popcll(dm));
+    slot = __shfl(slot, leader);
+    double a[3];
+    abs_pos(A.M, t_before, px, py, pz, a);
+    WorkItem it;
+    it.x0 = a[0];
+    it.y0 = a[1];
+    it.z0 = a[2];
+    it.i = (int32_t)row;
+    it.t0 = t_before;
+    it.k = ks;
+    it.pad = 0;
+    A.wl[slot + (unsigned)__popcll(dm & ((1ull << lane) - 1ull))] = it;
+}
+
+// What a rare step left: the owner, the outcome, and the charge weights lam,
+// to be counted `weight` times in t.
+struct RareStep {
+    Lam lam;
+    int32_t t;
+    int32_t outcome;
+    int32_t weight;
+};
+
+// Step ks of the launch for the lanes with `go` whose step is not the streaming
+// loop's common case: frozen particles, collisions, segments the loop does not
+// certify, surface hits.  The particle's state is in memory, before the step,
+// and is left there after it: nothing of the caller's is live here but the
+// charge sums, so that the walk's and the scattering's temporaries have the
+// registers.  (With the state kept in registers across it, parts of the loop's
+// own values went to scratch memory, which is 100 MB over the chip and misses
+// the L2: up to 11 ms for 200 steps of 1M particles.  Called out of line
+// it was slower too, for the calling convention's saves.)
+template <typename R, bool kBatch, bool kWalk, bool kTrack>
+__device__ __forceinline__ RareStep rare_step(const StepArgs<R>& A, uint32_t row, uint32_t step, int32_t ks, int32_t remaining,
+                                           bool go)
+{
+    RareStep r{{{0.0, 0.0, 0.0, 0.0}}, -1, kDone, 0};
+    if (!go) return r;
+    const DevMesh& M = A.M;
+    const StepParams& S = A.S;
+    const DevParticles<R>& P = A.P;
+    PState<R> s;
+    s.f = P.flags[row];
+    s.t = P.tet[row];
+    s.x = P.x[row];
+    s.y = P.y[row];
+    s.z = P.z[row];
+    s.vx = P.vx[row];
+    s.vy = P.vy[row];
+    s.vz = P.vz[row];
+    s.set_v2();
+    const SpeciesK& k = A.sp[(s.f >> kSpeciesShift) & 0xff];
+    const RunK* rk = kBatch ? S.runs + ((uint32_t)s.f >> kRunShift) : S.runs;
+    const uint32_t li = P.pidx[row];
+    r.t = s.t;
+    if (is_frozen(M, S, s)) {
+        if (s.t >= 0) {
+            bary_at(M, s.t, s.x, s.y, s.z, r.lam.l);
+            r.weight = remaining;
+        }
+        r.outcome = kFrozenNow;
+        return r;
+    }
+    const PConst c = particle_const(S, &k, rk, li - rk->first);
+    const R px = s.x, py = s.y, pz = s.z;
+    const int32_t t_before = s.t;
+    int32_t hit_tri = -1;
+    R x1, y1, z1;
+    {
+        TetRec<R> rec;
+        rec.template load<kBatch>(M, S, k, rk, s.t);
+        push_in(s, rec);
+        end_point(S, c.vid, c.key, step, s, x1, y1, z1);
+        rec.bary(x1, y1, z1, r.lam.l);
+    }
+    if (kTrack) track_start<R>(M, S, li, t_before, px, py, pz);
+    if (!(x1 == px && y1 == py && z1 == pz)) {  // (a degenerate segment ends here, :188-190)
+        if (S.model != 0 && may_collide<R>(variate_word(S.seed, c.key, c.vid, step), c.ca, c.cb, s.v2))
+            collide(S, c, step, s);
+        r.outcome = move_to<R, kWalk>(M, s, (s.f & kStrict) != 0, x1, y1, z1, r.lam, hit_tri);
+    }
+    r.t = s.t;
+    r.weight = r.outcome == kDone && s.t >= 0 ? 1 : 0;
+    P.x[row] = s.x;
+    P.y[row] = s.y;
+    P.z[row] = s.z;
+    P.vx[row] = s.vx;
+    P.vy[row] = s.vy;
+    P.vz[row] = s.vz;
+    if (s.t != t_before) P.tet[row] = s.t;
+    if (s.t < 0 && t_before >= 0) P.flags[row] = s.f & ~kStrict;
+    if (r.outcome != kDone)
+        finish_rare<R, kTrack>(A, r.outcome, row, li, rk, s, t_before, px, py, pz, step, ks, hit_tri);
+    return r;
+}
+
 // One tile of the streaming kernel: BS consecutive particles, one per thread,
-// S.nsteps steps with the state and the owning tet's data in registers.  A
+// S.nsteps steps with the state and the owning tet's record in registers.  A
 // particle whose relocation cannot be certified stops and goes to the work
 // list with the step it stopped at.  Called with a block-uniform tile.
 // kTrack: movement records on (S.trk_slot set), a kernel variant of its own so
 // that the streaming kernels without them carry none of their code.
-template <typename R, int BS, int HashBits, int Win, bool kBatch, bool kWalk, bool kTrack>
-__device__ __forceinline__ void step_tile(const DevMesh& M, const DevParticles<R>& P, const StepParams& S,
-                                          const SpeciesK* __restrict__ sp, double* __restrict__ node_charge,
-                                          WorkItem* __restrict__ wl, unsigned long long* __restrict__ cnt,
-                                          unsigned long long* __restrict__ tri_count, int64_t tile, int64_t n_active,
-                                          uint32_t step0, unsigned int* blk_processed, int32_t* hk, double* hv,
-                                          double* wv, int32_t* s_wbase)
+// What bounds a fused launch is VALU issue: a common step is about 150 vector
+// instructions, against 525 when every step read the record again, took an
+// FP32 pow and two square roots for the collision test and ran through the
+// code of the rare cases.  200 steps of 1M particles on 750k tets with their
+// read-back, FP64: 3.31 -> 1.17 ms; of 16 runs of 1e4 to 4e5 particles on
+// 162k tets, mixed: 6.37 -> 3.10 ms.  Where one lane of nearly every wave
+// changes tet in every step the latency of the next record bounds it and the
+// gain is small: 4% on a run of 1M particles through a 374k-tet chamber, and
+// the launches of 4,096 waves between two plates are slower, 380 -> 477 us per
+// 50 steps, because a quarter of the waves waits for a second round.
+// 3 waves per SIMD (168 registers): 4 waves put values of the loop into
+// scratch memory (1.47 ms), 2 waves hide too little of it (1.36 ms).
+template <typename R, int BS, int HashBits, bool kBatch, bool kWalk, bool kTrack>
+__device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, int64_t n_active, uint32_t step0,
+                                          unsigned int* blk_processed, int32_t* hk, double* hv, TetRows* s_rows)
 {
-    // The node window is used by single-step launches, whose charge all goes
-    // to LDS in the flush at the end of the tile (flush_wave_window); fused
-    // launches add to LDS while they step and use the hash alone.  (Laying a
-    // hash of twice the slots over the unused window for them was no faster.)
     constexpr int kSlots = 1 << HashBits;
-    const bool win = Win > 0 && S.nsteps == 1;
+    const DevMesh& M = A.M;
+    const StepParams& S = A.S;
+    const DevParticles<R>& P = A.P;
+    if (threadIdx.x == 0) *blk_processed = 0u;
+    if (S.charge) {
+        for (int h = threadIdx.x; h < kSlots; h += BS) {
+            hk[h] = -1;
+            hv[h] = 0.0;
+        }
+    }
+    __syncthreads();
+    // the tile's part of every array from a block-uniform base and the lane's
+    // 32-bit offset: no per-lane 64-bit address outlives its load or store
+    const int64_t i0 = tile * BS;
+    const int tid = threadIdx.x;
+    RegSink<LdsSink<HashBits, 0>> sink{LdsSink<HashBits, 0>{hk, hv, nullptr, 0, A.node_charge}, 0.0, 0.0, 0.0, 0.0};
+    // A lane is alive while its particle has steps to take.  A lane without a
+    // particle, or whose particle is done (frozen, settled, deferred: its state
+    // is in memory), goes through the arithmetic of the others; nothing of it
+    // is used.
+    PState<R> s;
+    s.f = kSettled;
+    s.t = -1;
+    s.x = s.y = s.z = R(0);
+    s.vx = s.vy = s.vz = 0.0;
+    auto read_state = [&]() {
+        s.t = (P.tet + i0)[tid];
+        s.x = (P.x + i0)[tid];
+        s.y = (P.y + i0)[tid];
+        s.z = (P.z + i0)[tid];
+        s.vx = (P.vx + i0)[tid];
+        s.vy = (P.vy + i0)[tid];
+        s.vz = (P.vz + i0)[tid];
+    };
+    int32_t t_mem = -1;  // the owner in memory (the loop only moves a particle from tet to tet)
+    auto write_state = [&]() {
+        (P.x + i0)[tid] = s.x;
+        (P.y + i0)[tid] = s.y;
+        (P.z + i0)[tid] = s.z;
+        (P.vx + i0)[tid] = s.vx;
+        (P.vy + i0)[tid] = s.vy;
+        (P.vz + i0)[tid] = s.vz;
+        if (s.t != t_mem) (P.tet + i0)[tid] = s.t;
+    };
+    uint32_t vid = 0;
+    if (i0 + tid < n_active) {
+        s.f = (P.flags + i0)[tid];
+        vid = (P.pidx + i0)[tid];
+        read_state();
+    }
+    bool alive = !(s.f & kSettled);
+    if (!alive) s.t = -1;
+    const SpeciesK& k = A.sp[alive ? (s.f >> kSpeciesShift) & 0xff : 0];
+    // one simulation: run 0 for every lane (scalar loads); a batch: the lane's run
+    const RunK* rk = kBatch ? S.runs + (alive ? (uint32_t)s.f >> kRunShift : 0u) : S.runs;
+    vid -= rk->first;
+    const bool strict = (s.f & kStrict) != 0;  // (a particle that leaves the mesh is told by its tet)
+    t_mem = s.t;
+    s.set_v2();
+    TetRec<R> rec;
+    TetRows* const rows = s_rows + tid;
+    rec.template load<kBatch>(M, S, k, rk, s.t, rows);
+    const PConst pc = particle_const(S, &k, rk, vid);
+    const int32_t base = kBatch ? (int32_t)rk->node_base : 0;
+    const double charge = k.charge;
+    const double tau = tau_of<R>(M);
+    const int nsteps = S.nsteps;
+    int ks = 0;
+    while (ks < nsteps && __ballot(alive) != 0) {
+        // The common case, alone in its loop: steps in which every live
+        // particle of the wavefront stays strictly inside its tet (all four
+        // coordinates of the end point above tau; their sum of magnitudes is
+        // then 1) with no collision to look at.  The loop is uniform and the
+        // common case touches no memory, so the state and the tet's record
+        // stay in registers.  A lane that crosses into a tet where it is
+        // certified, meets a surface or flies on outside the mesh is handled
+        // in place; a step with any other case in any lane leaves the loop.
+        bool rare;
+        for (;;) {
+            const uint32_t step = step0 + (uint32_t)ks;
+            const int32_t t0 = s.t;
+            rare = too_slow(s.v2);
+            if (!S.bbox_covers) rare = rare || !in_bbox_at(M, S, s.t, s.x, s.y, s.z);
+            PState<R> n = s;
+            R x1, y1, z1;
+            push_in(n, rec);
+            end_point(S, pc.vid, pc.key, step, n, x1, y1, z1);
+            bool draw = S.model != 0;
+            if (draw) draw = may_collide<R>(variate_word(S.seed, pc.key, pc.vid, step), pc.ca, pc.cb, n.v2);
+            Lam lam;
+            rec.bary(x1, y1, z1, lam.l);
+            bool inside = strict && lam.l[0] > tau && lam.l[1] > tau && lam.l[2] > tau && lam.l[3] > tau;
+            rare = rare || draw;
+            bool settles = false;
+            if (__ballot(alive && (rare || !inside)) != 0) {
+                if (alive && !rare && !inside) {
+                    if (s.t < 0) {
+                        inside = in_bbox_at(M, S, s.t, s.x, s.y, s.z) && stays_outside(M, s, x1, y1, z1);
+                    } else if (strict) {
+                        // From tet to tet along the segment.  (Mixed: one hop in
+                        // FP32; further ones go through the FP64 maps of
+                        // rare_step.)
+                        constexpr bool kFar = kWalk && std::is_same<R, double>::value;
+                        int fneg = 0;
+                        int f = kFar ? exit_face(tau, lam.l, [&](double* l0) { rec.bary(s.x, s.y, s.z, l0); })
+                                     : (classify(lam.l, tau, fneg) == kOneFace ? fneg : (int)kNoFace);
+                        if (f >= 0) {
+                            int32_t code = (&rows->nbr.x)[f];
+                            if (S.charge && charge != 0.0) sink.flush_nodes(rows->node, base, charge);
+                            R nx = x1, ny = y1, nz = z1;
+                            if constexpr (!std::is_same<R, double>::value) {
+                                double p1[3];
+                                abs_pos(M, s.t, x1, y1, z1, p1);
+                                to_frame(M, code, p1, nx, ny, nz);
+                            }
+#pragma unroll 1
+                            for (int hop = 0; code >= 0 && hop < (kFar ? 6 : 1); ++hop) {
+                                rec.template load_in<kBatch>(M, S, k, rk, code, rows);
+                                rec.bary(nx, ny, nz, lam.l);
+                                if (lam.l[0] > tau && lam.l[1] > tau && lam.l[2] > tau && lam.l[3] > tau) {
+                                    inside = true;
+                                    break;
+                                }
+                                f = kNoFace;
+                                if constexpr (kFar)
+                                    f = exit_face(tau, lam.l, [&](double* l0) { rec.bary(s.x, s.y, s.z, l0); });
+                                if (f < 0) break;
+                                code = (&rows->nbr.x)[f];
+                            }
+                            if (inside) {
+                                s.t = code;
+                                x1 = nx;
+                                y1 = ny;
+                                z1 = nz;
+                            } else if (f >= 0 && code <= -2) {
+                                settles = true;  // on triangle -2 - code
+                                s.f = code;
+                            }
+                        }
+                    }
+                }
+                rare = rare || !inside;
+            }
+            if (kTrack && alive && (!rare || settles)) track_start<R>(M, S, vid + rk->first, t0, s.x, s.y, s.z);
+            if (__builtin_expect(__ballot(settles) != 0, 0)) {
+                if (settles) {
+                    const R px = s.x, py = s.y, pz = s.z;
+                    const int32_t tri = -2 - s.f;
+                    s.f = (P.flags + i0)[tid];
+                    s.x = x1;  // in the frame of the owner it leaves
+                    s.y = y1;
+                    s.z = z1;
+                    s.vx = n.vx;
+                    s.vy = n.vy;
+                    s.vz = n.vz;
+                    write_state();
+                    finish_rare<R, kTrack>(A, kSettledNow, (uint32_t)(i0 + tid), vid + rk->first, rk, s, t0, px, py,
+                                           pz, step, ks, tri);
+                    atomicAdd(blk_processed, (unsigned int)ks + 1u);
+                    alive = false;
+                    s.t = -1;
+                    rec.template load<kBatch>(M, S, k, rk, -1, rows);
+                }
+            }
+            if (!rare) {
+                s.x = x1;
+                s.y = y1;
+                s.z = z1;
+                s.vx = n.vx;
+                s.vy = n.vy;
+                s.vz = n.vz;
+                s.v2 = n.v2;
+                sink.a0 += lam.l[0];
+                sink.a1 += lam.l[1];
+                sink.a2 += lam.l[2];
+                sink.a3 += lam.l[3];
+            }
+            rare = rare && alive;
+            if (__ballot(rare) != 0) break;
+            if (++ks == nsteps) break;
+        }
+        if (ks == nsteps) break;
+        // A step that is rare in some lanes (the others have taken it): every
+        // lane's state goes through memory.
+        if (alive) write_state();
+        const int32_t t_before = s.t;
+        const RareStep r = rare_step<R, kBatch, kWalk, kTrack>(
+            A, (uint32_t)(i0 + tid), step0 + (uint32_t)ks, ks,
+            nsteps - ks, rare);
+        asm volatile("" ::: "memory");
+        if (rare) {
+            const bool done = r.outcome != kDone;
+            if (S.charge && t_before >= 0 && (done || r.t != t_before)) {
+                if (r.outcome == kFrozenNow) sink.add((double)r.weight, r.lam.l);
+                sink.flush(M, t_before, base, charge);
+            }
+            if (!done) sink.add((double)r.weight, r.lam.l);
+            if (done) {
+                const unsigned int taken = (unsigned int)ks + (r.outcome == kFrozenNow ? 0u : 1u);
+                if (taken) atomicAdd(blk_processed, taken);
+                alive = false;
+            }
+            s.t = done ? -1 : r.t;
+        }
+        t_mem = s.t;
+        if (alive) read_state();
+        s.set_v2();
+        rec.template load<kBatch>(M, S, k, rk, s.t, rows);
+        ++ks;
+    }
+    if (alive) write_state();
+    if (!alive) sink.a0 = sink.a1 = sink.a2 = sink.a3 = 0.0;  // flushed when it stopped
+    if (S.charge) sink.flush_wave(M, s.t, base, charge);  // every lane is active here
+    // processed particle-steps: LDS per block, one atomic per tile spread over slots
+    const unsigned long long am = __ballot(alive);
+    if ((threadIdx.x & 63) == 0 && am) atomicAdd(blk_processed, (unsigned int)__popcll(am) * (unsigned int)nsteps);
+    __syncthreads();
+    if (threadIdx.x == 0 && *blk_processed)
+        atomicAdd(&A.cnt[kCntProcSlot0 + (tile & (kProcSlots - 1))], (unsigned long long)*blk_processed);
+    if (S.charge) {
+        for (int h = threadIdx.x; h < kSlots; h += BS) {
+            int32_t node = hk[h];
+            if (node >= 0) global_add_f64(&A.node_charge[node], hv[h]);
+        }
+    }
+    __syncthreads();  // the LDS table and counter are reused by the next tile
+}
+
+// One tile of a single-step launch of one simulation: each particle's step in
+// registers from load to store.  All charge goes to LDS in the flush at the
+// end of the tile, into a window of consecutive nodes (flush_wave_window).
+// HBM and the charge atomics bound it: 227 B per particle-step.  1M particles
+// on 750k tets: FP64 53.4 -> 52.6 us, mixed 57.8 -> 45.0 us; 4M particles FP64
+// 211 -> 183 us.  4 workgroups per CU, no scratch memory; a fifth (half the
+// hash, 96 registers) was slower, 55.5 and 193 us.
+template <typename R, int BS, int HashBits, int Win, bool kWalk>
+__device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, int64_t n_active, uint32_t step,
+                                            unsigned int* blk_processed, int32_t* hk, double* hv, double* wv,
+                                            int32_t* s_wbase)
+{
+    constexpr int kSlots = 1 << HashBits;
+    const DevMesh& M = A.M;
+    const StepParams& S = A.S;
+    const DevParticles<R>& P = A.P;
     if (threadIdx.x == 0) {
         *blk_processed = 0u;
-        if (Win > 0) *s_wbase = INT32_MAX;
+        *s_wbase = INT32_MAX;
     }
     if (S.charge) {
         for (int h = threadIdx.x; h < kSlots; h += BS) {
             hk[h] = -1;
             hv[h] = 0.0;
         }
-        if (win)
-            for (int h = threadIdx.x; h < Win; h += BS) wv[h] = 0.0;
+        for (int h = threadIdx.x; h < Win; h += BS) wv[h] = 0.0;
     }
     __syncthreads();
-    int64_t i = tile * BS + threadIdx.x;
-    RegSink<LdsSink<HashBits, Win>> sink{LdsSink<HashBits, Win>{hk, hv, wv, INT32_MAX, node_charge}, -1, 0, 0.0,
-                                         0.0, 0.0, 0.0};
-    int processed = 0;
-    bool deferred = false;
-    int defer_k = 0;
-    double x0abs[3] = {0.0, 0.0, 0.0};
-    int32_t t_defer = -1;
-    if (i < n_active) {
-        PState<R> s;
-        s.f = P.flags[i];
+    const int64_t i0 = tile * BS;
+    const int tid = threadIdx.x;
+    RegSink<LdsSink<HashBits, Win>> sink{LdsSink<HashBits, Win>{hk, hv, wv, INT32_MAX, A.node_charge}, 0.0, 0.0, 0.0,
+                                         0.0};
+    int32_t cur = -1;  // the tet the charge goes to
+    double charge = 0.0;
+    bool taken = false, rare = false, draw = false;
+    PState<R> s;
+    R x1 = R(0), y1 = R(0), z1 = R(0);
+    Lam lam;
+    lam.l[0] = lam.l[1] = lam.l[2] = lam.l[3] = 0.0;
+    const SpeciesK* kp = A.sp;
+    uint32_t vid = 0;
+    if (i0 + tid < n_active) {
+        s.f = (P.flags + i0)[tid];
+        s.t = (P.tet + i0)[tid];
+        s.x = (P.x + i0)[tid];
+        s.y = (P.y + i0)[tid];
+        s.z = (P.z + i0)[tid];
+        s.vx = (P.vx + i0)[tid];
+        s.vy = (P.vy + i0)[tid];
+        s.vz = (P.vz + i0)[tid];
+        vid = (P.pidx + i0)[tid] - S.runs->first;
         if (!(s.f & kSettled)) {
-            const SpeciesK& k = sp[(s.f >> kSpeciesShift) & 0xff];
-            // one simulation: run 0 for every lane (scalar loads); a batch: the lane's run
-            const RunK* rk = kBatch ? S.runs + ((uint32_t)s.f >> kRunShift) : S.runs;
-            sink.base = kBatch ? (int32_t)rk->node_base : 0;
-            s.x = P.x[i];
-            s.y = P.y[i];
-            s.z = P.z[i];
-            s.vx = P.vx[i];
-            s.vy = P.vy[i];
-            s.vz = P.vz[i];
-            s.t = P.tet[i];
-            const int32_t t_in = s.t, f_in = s.f;
-            // variate counter: collisions need it; the mixed path's stochastic
-            // rounding keys on it too
-            const uint32_t vid = (S.model != 0 || !std::is_same<R, double>::value) ? P.pidx[i] - rk->first : 0u;
-            bool moved = false;
-            for (int ks = 0; ks < S.nsteps; ++ks) {
-                const R px = s.x, py = s.y, pz = s.z;
-                const int32_t t_before = s.t;
-                StepResult r = step_one<R, kBatch, kWalk>(M, S, k, rk, vid, step0 + (uint32_t)ks, S.nsteps - ks, s, sink);
-                if (r.outcome == kFrozenNow) break;
-                ++processed;
-                moved = true;
-                if (kTrack) track_start<R>(M, S, P.pidx[i], t_before, px, py, pz);
-                if (r.outcome == kSettledNow) {
-                    s.f = (s.f | kSettled) & ~kStrict;
-                    P.hit[i] = r.hit_tri;
-                    atomicAdd(&tri_count[rk->tri_base + r.hit_tri], 1ull);
-                    S.settle_log[atomicAdd(&cnt[kCntSettled], 1ull)] = P.pidx[i];
-                    if (S.settle || kTrack) {
-                        double a[3];
-                        abs_pos(M, t_before, px, py, pz, a);
-                        if (S.settle) record_settle(S.settle, P.pidx[i], step0 + (uint32_t)ks, a[0], a[1], a[2]);
-                        if (kTrack) track_hit<R>(M, S, P.pidx[i], a, s.t, s.x, s.y, s.z, r.hit_tri);
-                    }
-                    break;
+            kp = A.sp + ((s.f >> kSpeciesShift) & 0xff);
+            charge = kp->charge;
+            s.set_v2();
+            TetRec<R> rec;
+            rec.template load<false>(M, S, *kp, S.runs, s.t);
+            if (is_frozen(M, S, s)) {
+                rec.bary(s.x, s.y, s.z, lam.l);
+                cur = s.t;
+            } else {
+                taken = true;
+                const PConst pc = particle_const(S, kp, S.runs, vid);
+                const double tau = tau_of<R>(M);
+                push_in(s, rec);
+                end_point(S, vid, pc.key, step, s, x1, y1, z1);
+                rec.bary(x1, y1, z1, lam.l);
+                if (S.model != 0) draw = may_collide<R>(variate_word(S.seed, pc.key, vid, step), pc.ca, pc.cb, s.v2);
+                rare = draw || !((s.f & kStrict) && lam.l[0] > tau && lam.l[1] > tau && lam.l[2] > tau &&
+                                 lam.l[3] > tau);
+                if (!rare) {
+                    (P.x + i0)[tid] = x1;
+                    (P.y + i0)[tid] = y1;
+                    (P.z + i0)[tid] = z1;
+                    (P.vx + i0)[tid] = s.vx;
+                    (P.vy + i0)[tid] = s.vy;
+                    (P.vz + i0)[tid] = s.vz;
+                    cur = s.t;
                 }
-                if (r.outcome == kDeferNow) {
-                    deferred = true;
-                    defer_k = ks;
-                    t_defer = t_before;
-                    abs_pos(M, t_before, px, py, pz, x0abs);
-                    break;
-                }
-            }
-            if (moved) {
-                const int64_t j = std::is_same<R, double>::value ? fresh_index(i) : i;
-                P.x[j] = s.x;
-                P.y[j] = s.y;
-                P.z[j] = s.z;
-                P.vx[j] = s.vx;
-                P.vy[j] = s.vy;
-                P.vz[j] = s.vz;
-                if (s.t != t_in) P.tet[j] = s.t;
-                if (s.f != f_in) P.flags[j] = s.f;
             }
         }
     }
-    if (S.charge) {  // every lane is active here
-        if (Win > 0 && S.nsteps == 1) sink.flush_wave_window(M, s_wbase);
-        else sink.flush_wave(M);
-    }
-    // work list: one atomic per wavefront, lanes take consecutive slots
-    unsigned long long dm = __ballot(deferred);
-    if (dm) {
-        int lane = threadIdx.x & 63;
-        int leader = __ffsll((long long)dm) - 1;
-        unsigned int base = 0u;
-        if (lane == leader)
-            base = (unsigned int)atomicAdd(&cnt[kCntWork + 2 * S.work_slot], (unsigned long long)__popcll(dm));
-        base = __shfl(base, leader);
-        if (deferred) {
-            WorkItem it;
-            it.x0 = x0abs[0];
-            it.y0 = x0abs[1];
-            it.z0 = x0abs[2];
-            it.i = (int32_t)i;
-            it.t0 = t_defer;
-            it.k = defer_k;
-            it.pad = 0;
-            wl[base + (unsigned)__popcll(dm & ((1ull << lane) - 1ull))] = it;
+    // collisions and segments that leave the tet
+    if (__ballot(rare) != 0) {
+        if (rare) {
+            const int32_t t_in = s.t;
+            const R px = s.x, py = s.y, pz = s.z;
+            int outcome = kDone;
+            int32_t hit_tri = -1;
+            if (!(x1 == px && y1 == py && z1 == pz)) {  // (a degenerate segment ends here, :188-190)
+                if (draw) collide(S, PConst{kp, S.runs, vid, S.runs->key, 0.0f, 0.0f}, step, s);
+                outcome = move_to<R, kWalk>(M, s, (s.f & kStrict) != 0, x1, y1, z1, lam, hit_tri);
+            }
+            const uint32_t row = (uint32_t)(i0 + tid);
+            P.x[row] = s.x;
+            P.y[row] = s.y;
+            P.z[row] = s.z;
+            P.vx[row] = s.vx;
+            P.vy[row] = s.vy;
+            P.vz[row] = s.vz;
+            if (s.t != t_in) {
+                P.tet[row] = s.t;
+                if (s.t < 0) P.flags[row] = s.f & ~kStrict;
+            }
+            if (outcome == kDone) cur = s.t;
+            else
+                finish_rare<R, false>(A, outcome, row, vid + S.runs->first, S.runs, s, t_in, px, py, pz, step, 0,
+                                      hit_tri);
         }
     }
-    // processed count: wavefront sum, LDS per block, one atomic per tile spread over slots
-    __syncthreads();
-    int wsum;
-    if (Win > 0) {  // single-step launches: 0 or 1 per lane
-        wsum = (int)__popcll(__ballot(processed != 0));
-    } else {
-        wsum = processed;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) wsum += __shfl_xor(wsum, off);
-    }
-    if ((threadIdx.x & 63) == 0 && wsum) atomicAdd(blk_processed, (unsigned int)wsum);
+    sink.a0 = lam.l[0];
+    sink.a1 = lam.l[1];
+    sink.a2 = lam.l[2];
+    sink.a3 = lam.l[3];
+    if (S.charge) sink.flush_wave_window(M, cur, 0, charge, s_wbase);  // every lane is active here
+    const unsigned long long am = __ballot(taken);
+    if ((threadIdx.x & 63) == 0 && am) atomicAdd(blk_processed, (unsigned int)__popcll(am));
     __syncthreads();
     if (threadIdx.x == 0 && *blk_processed)
-        atomicAdd(&cnt[kCntProcSlot0 + (tile & (kProcSlots - 1))], (unsigned long long)*blk_processed);
+        atomicAdd(&A.cnt[kCntProcSlot0 + (tile & (kProcSlots - 1))], (unsigned long long)*blk_processed);
     if (S.charge) {
         for (int h = threadIdx.x; h < kSlots; h += BS) {
-            int32_t node = hk[h];
-            if (node >= 0) global_add_f64(&node_charge[node], hv[h]);
+            const int32_t node = hk[h];
+            if (node >= 0) global_add_f64(&A.node_charge[node], hv[h]);
         }
         // window slots that received charge (untouched ones hold 0.0)
-        if (win) {
-            const int32_t wbase = sink.inner.wbase;
-            for (int h = threadIdx.x; h < Win; h += BS) {
-                const double v = wv[h];
-                if (v != 0.0) global_add_f64(&node_charge[wbase + h], v);
-            }
+        const int32_t wbase = sink.inner.wbase;
+        for (int h = threadIdx.x; h < Win; h += BS) {
+            const double v = wv[h];
+            if (v != 0.0) global_add_f64(&A.node_charge[wbase + h], v);
         }
     }
-    __syncthreads();  // the LDS table and counter are reused by the next tile
 }
 
 // Streaming kernel.  With persistent == 0 workgroup b takes tile b; otherwise
@@ -1366,12 +1893,10 @@ __device__ __forceinline__ void step_tile(const DevMesh& M, const DevParticles<R
 // sizes).  The charge of a tile is summed in LDS (node window and hash) and
 // flushed with one FP64 atomic per distinct node.
 template <typename R, int BS, bool kBatch, bool kPersistent, bool kWalk, bool kTrack = false, bool kWindow = false>
-__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) step_main(DevMesh M, DevParticles<R> P, StepParams S,
-                                                       const SpeciesK* __restrict__ sp,
-                                                       double* __restrict__ node_charge, WorkItem* __restrict__ wl,
-                                                       unsigned long long* __restrict__ cnt,
-                                                       unsigned long long* __restrict__ tri_count)
+__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kWindow ? 4 : 3))) step_main(StepArgs<R> A)
 {
+    const StepParams& S = A.S;
+    unsigned long long* const cnt = A.cnt;
     // kWindow (single-step launches of one simulation, 256 threads): a
     // 3,072-node window (24 KB) and a 1,024-slot hash (12 KB), 36 KB in all,
     // so that four workgroups (the 16 waves the 128-VGPR budget allows) share
@@ -1388,6 +1913,7 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) st
     __shared__ int32_t hk[1 << kBits];
     __shared__ double hv[1 << kBits];
     __shared__ double wv[kWin > 0 ? kWin : 1];
+    __shared__ TetRows s_rows[kWin > 0 ? 1 : BS];
     const uint32_t step0 = (uint32_t)cnt[kCntStep + S.work_slot];
     {
         // clear the next launch's charge buffers and counters, and give it its first step
@@ -1404,9 +1930,14 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) st
     const int64_t n_active = *S.n_active;
     if (!kPersistent) {
         if ((int64_t)blockIdx.x * BS < n_active)  // else the whole block is past the live particles
-            step_tile<R, BS, kBits, kWin, kBatch, kWalk, kTrack>(M, P, S, sp, node_charge, wl, cnt, tri_count,
-                                                                 blockIdx.x, n_active, step0, &blk_processed, hk, hv,
-                                                                 wv, &s_wbase);
+        {
+            if constexpr (kWindow)
+                single_tile<R, BS, kBits, kWin, kWalk>(A, blockIdx.x, n_active, step0, &blk_processed, hk, hv, wv,
+                                                       &s_wbase);
+            else
+                step_tile<R, BS, kBits, kBatch, kWalk, kTrack>(A, blockIdx.x, n_active, step0, &blk_processed, hk, hv,
+                                                               s_rows);
+        }
         return;
     }
     for (;;) {
@@ -1414,17 +1945,16 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) st
         __syncthreads();
         const int64_t tile = s_tile;
         if (tile * BS >= n_active) break;  // queue drained: every workgroup exits here
-        step_tile<R, BS, kBits, kWin, kBatch, kWalk, kTrack>(M, P, S, sp, node_charge, wl, cnt, tri_count, tile,
-                                                             n_active, step0, &blk_processed, hk, hv, wv, &s_wbase);
+        step_tile<R, BS, kBits, kBatch, kWalk, kTrack>(A, tile, n_active, step0, &blk_processed, hk, hv, s_rows);
     }
 }
 
 // Exact relocation of a deferred step: the state holds x1 in the frame of the
 // owner at the step start; x0abs is the absolute start.  Returns true when the
 // particle settled.
-template <typename R, typename Sink>
-__device__ inline bool finish_exact(const DevMesh& M, const StepParams& S, const SpeciesK& k, const double* x0abs,
-                                    PState<R>& s, Sink& sink, int32_t& hit_tri, int& exh, int& err)
+template <typename R>
+__device__ inline bool finish_exact(const DevMesh& M, const double* x0abs, PState<R>& s, int32_t& hit_tri, int& exh,
+                                    int& err)
 {
     double x1[3];
     abs_pos(M, s.t, s.x, s.y, s.z, x1);
@@ -1445,12 +1975,15 @@ __device__ inline bool finish_exact(const DevMesh& M, const StepParams& S, const
     }
     s.t = r.tet;
     s.f = strict ? (s.f | kStrict) : (s.f & ~kStrict);
-    if (S.charge && s.t >= 0 && k.charge != 0.0) {
-        double lam[4];
-        bary_at(M, s.t, s.x, s.y, s.z, lam);
-        sink.add(M, s.t, k.charge, lam);
-    }
     return false;
+}
+template <typename R, typename Sink>
+__device__ inline void add_here(const DevMesh& M, const PState<R>& s, Sink& sink)
+{
+    if (s.t < 0) return;
+    double lam[4];
+    bary_at(M, s.t, s.x, s.y, s.z, lam);
+    sink.add(1.0, lam);
 }
 
 // Straggler kernel: finishes each deferred relocation exactly, then runs the
@@ -1468,7 +2001,7 @@ __global__ void __launch_bounds__(64) step_resolve(DevMesh M, DevParticles<R> P,
     const uint32_t step0 = (uint32_t)cnt[kCntStep + S.work_slot];
     for (uint64_t w = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; w < nw;
          w += (uint64_t)gridDim.x * blockDim.x) {
-        RegSink<GlobalSink> sink{GlobalSink{node_charge}, -1, 0, 0.0, 0.0, 0.0, 0.0};
+        RegSink<GlobalSink> sink{GlobalSink{node_charge}, 0.0, 0.0, 0.0, 0.0};
         WorkItem it = wl[w];
         int64_t i = it.i;
         PState<R> s;
@@ -1482,33 +2015,42 @@ __global__ void __launch_bounds__(64) step_resolve(DevMesh M, DevParticles<R> P,
         s.vz = P.vz[i];
         const SpeciesK& k = sp[(s.f >> kSpeciesShift) & 0xff];
         const RunK* rk = S.runs + ((uint32_t)s.f >> kRunShift);
-        sink.base = (int32_t)rk->node_base;
+        const int32_t base = (int32_t)rk->node_base;
         int exh = 0, err = 0, nexact = 0;
         int32_t hit_tri = -1;
         double x0[3] = {it.x0, it.y0, it.z0};
         // (the step's start was recorded by the streaming kernel)
-        bool settled = finish_exact(M, S, k, x0, s, sink, hit_tri, exh, err);
+        bool settled = finish_exact(M, x0, s, hit_tri, exh, err);
+        if (!settled) add_here(M, s, sink);
         if (settled && S.trk_slot) track_hit<R>(M, S, P.pidx[i], x0, s.t, s.x, s.y, s.z, hit_tri);
         uint32_t settle_step = step0 + (uint32_t)it.k;  // step and start of the settling segment
         double sx = x0[0], sy = x0[1], sz = x0[2];
         if (!settled) {
-            const uint32_t vid = (S.model != 0 || !std::is_same<R, double>::value) ? P.pidx[i] - rk->first : 0u;
+            const PConst pc = particle_const(S, &k, rk, P.pidx[i] - rk->first);
+            TetRec<R> rec;
+            rec.t = -1;
+            s.set_v2();
             unsigned long long extra = 0;
             for (int ks = it.k + 1; ks < S.nsteps; ++ks) {
                 const R px = s.x, py = s.y, pz = s.z;
                 const int32_t t_before = s.t;
-                StepResult rr = step_one<R, true, kWalk>(M, S, k, rk, vid, step0 + (uint32_t)ks, S.nsteps - ks, s, sink);
-                if (rr.outcome == kFrozenNow) break;
+                int32_t tri = -1;
+                const int outcome =
+                    step_one<R, true, kWalk>(M, S, pc, step0 + (uint32_t)ks, S.nsteps - ks, s, rec, sink, tri);
+                if (outcome == kFrozenNow) break;
                 ++extra;
                 if (S.trk_slot) track_start<R>(M, S, P.pidx[i], t_before, px, py, pz);
-                if (rr.outcome == kDeferNow || rr.outcome == kSettledNow) {
+                if (outcome == kDeferNow || outcome == kSettledNow) {
                     double x0s[3];
                     abs_pos(M, t_before, px, py, pz, x0s);
-                    if (rr.outcome == kDeferNow) {
+                    if (outcome == kDeferNow) {
                         ++nexact;
-                        settled = finish_exact(M, S, k, x0s, s, sink, hit_tri, exh, err);
+                        // (the sums belong to the tet the step started in)
+                        sink.flush(M, S.charge ? t_before : -1, base, k.charge);
+                        settled = finish_exact(M, x0s, s, hit_tri, exh, err);
+                        if (!settled) add_here(M, s, sink);
                     } else {
-                        hit_tri = rr.hit_tri;
+                        hit_tri = tri;
                         settled = true;
                     }
                     if (settled && S.trk_slot) track_hit<R>(M, S, P.pidx[i], x0s, s.t, s.x, s.y, s.z, hit_tri);
@@ -1528,7 +2070,8 @@ __global__ void __launch_bounds__(64) step_resolve(DevMesh M, DevParticles<R> P,
             S.settle_log[atomicAdd(&cnt[kCntSettled], 1ull)] = P.pidx[i];
             if (S.settle) record_settle(S.settle, P.pidx[i], settle_step, sx, sy, sz);
         }
-        sink.flush(M);
+        // (a settling step left the owner as it was, with the sums of the steps before)
+        sink.flush(M, S.charge ? s.t : -1, base, k.charge);
         P.x[i] = s.x;
         P.y[i] = s.y;
         P.z[i] = s.z;
@@ -1906,12 +2449,13 @@ void launch_step(hipStream_t s, const DevMesh& M, const DevParticles<R>& P, cons
                  const SpeciesK* sp, double* node_charge, WorkItem* wl, unsigned long long* cnt,
                  unsigned long long* tri_count, const StepLaunch& L, hipEvent_t ev_mid)
 {
+    const StepArgs<R> A{M, P, S, sp, node_charge, wl, cnt, tri_count};
     if (P.n > 0 && S.trk_slot) {
         // movement records: the tracking variants (256-thread workgroups, one per tile)
         const unsigned grid = blocks_for(P.n, 256);
         switch ((L.batch ? 2 : 0) + (L.walk ? 1 : 0)) {
 #define SG_STEP_TRACK(B_, W_) \
-    step_main<R, 256, B_, false, W_, true><<<grid, 256, 0, s>>>(M, P, S, sp, node_charge, wl, cnt, tri_count)
+    step_main<R, 256, B_, false, W_, true><<<grid, 256, 0, s>>>(A)
         case 0: SG_STEP_TRACK(false, false); break;
         case 1: SG_STEP_TRACK(false, true); break;
         case 2: SG_STEP_TRACK(true, false); break;
@@ -1923,10 +2467,10 @@ void launch_step(hipStream_t s, const DevMesh& M, const DevParticles<R>& P, cons
         const unsigned grid = blocks_for(P.n, 256);
         if (L.walk)
             step_main<R, 256, false, false, true, false, true>
-                <<<grid, 256, 0, s>>>(M, P, S, sp, node_charge, wl, cnt, tri_count);
+                <<<grid, 256, 0, s>>>(A);
         else
             step_main<R, 256, false, false, false, false, true>
-                <<<grid, 256, 0, s>>>(M, P, S, sp, node_charge, wl, cnt, tri_count);
+                <<<grid, 256, 0, s>>>(A);
     } else if (P.n > 0) {
         const unsigned grid = L.persistent ? (unsigned)L.grid : blocks_for(P.n, L.block == 128 ? 128 : 256);
         // the multi-tet walk is instantiated for 256-thread workgroups only
@@ -1935,7 +2479,7 @@ void launch_step(hipStream_t s, const DevMesh& M, const DevParticles<R>& P, cons
                              : (L.block == 128 ? 4 : 0) + (L.batch ? 2 : 0) + (L.persistent ? 1 : 0);
         switch (v) {
 #define SG_STEP_MAIN(BS_, B_, P_, W_) \
-    step_main<R, BS_, B_, P_, W_><<<grid, BS_, 0, s>>>(M, P, S, sp, node_charge, wl, cnt, tri_count)
+    step_main<R, BS_, B_, P_, W_><<<grid, BS_, 0, s>>>(A)
         case 0: SG_STEP_MAIN(256, false, false, false); break;
         case 1: SG_STEP_MAIN(256, false, true, false); break;
         case 2: SG_STEP_MAIN(256, true, false, false); break;
