@@ -64,6 +64,11 @@ struct WorkItem {
     int32_t pad;
 };
 
+// Bounding box of a tet's nodes in FP32, rounded outwards.
+struct TetBox {
+    float lo[3], hi[3];
+};
+
 struct DevMesh {
     const double* nodes;   // 3M
     const double* geo;     // 12T
@@ -78,6 +83,7 @@ struct DevMesh {
     const float* H32;
     const int4* tnode;     // T
     const int4* tnbr;      // T
+    const TetBox* tbox;    // T
     const int32_t* tris;   // 3S
     const uint8_t* tri_degenerate;
     const int32_t* tgrid_start;

@@ -45,6 +45,7 @@ void launch_track_eligible(hipStream_t s, const DevMesh& M, const DevParticles<R
                            uint8_t* out);
 void launch_field(hipStream_t s, const DevMesh& M, const double* phi, double* E, float* E32);
 void launch_e32(hipStream_t s, const double* E, float* E32, int64_t nt);
+void launch_tet_boxes(hipStream_t s, const DevMesh& M, TetBox* box);
 void launch_push_table(hipStream_t s, const double* E, const float* E32, int64_t nt, const double* q,
                        const double* m, int32_t n_slots, double dt, double* H, float* H32);
 void launch_orient_batch(hipStream_t s, const double* pts, int64_t n, int32_t* out);
@@ -165,6 +166,7 @@ struct start_ctx {
     std::vector<uint8_t> present;  // species of the loaded population
     int4* d_tnode = nullptr;
     int4* d_tnbr = nullptr;
+    TetBox* d_tbox = nullptr;
     int32_t* d_tris = nullptr;
     uint8_t* d_tri_deg = nullptr;
     int32_t *d_tgs = nullptr, *d_tgl = nullptr, *d_sgs = nullptr, *d_sgl = nullptr;
@@ -241,6 +243,7 @@ struct start_ctx {
         M.H32 = d_H32;
         M.tnode = d_tnode;
         M.tnbr = d_tnbr;
+        M.tbox = d_tbox;
         M.tris = d_tris;
         M.tri_degenerate = d_tri_deg;
         M.tgrid_start = d_tgs;
@@ -1244,6 +1247,7 @@ int start_create(start_ctx** out, const start_mesh_desc* mesh, const start_param
     }
     chk(dalloc(&c->d_tnode, T));
     chk(dalloc(&c->d_tnbr, T));
+    chk(dalloc(&c->d_tbox, T));
     chk(dalloc(&c->d_tris, 3 * S));
     chk(dalloc(&c->d_tri_deg, S));
     chk(dalloc(&c->d_tgs, hm.tgrid_start.size()));
@@ -1277,6 +1281,9 @@ int start_create(start_ctx** out, const start_mesh_desc* mesh, const start_param
         chk(up(c->d_species, c->species.data(), sizeof(SpeciesK) * c->species.size()));
         chk(up(c->d_runs, c->runs.data(), sizeof(RunK)));
         chk(hipMemset(c->d_cnt, 0, sizeof(unsigned long long) * kCntTotal));
+        if (he == hipSuccess) launch_tet_boxes(c->stream, c->mesh_view(), c->d_tbox);
+        chk(hipGetLastError());
+        chk(hipStreamSynchronize(c->stream));
     }
     if (he != hipSuccess) {
         std::string msg = std::string("device set-up failed: ") + hipGetErrorString(he);
@@ -1293,7 +1300,7 @@ void start_destroy(start_ctx* c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     free_particles(c);
     void* ptrs[] = {c->d_nodes,     c->d_geo,       c->d_geo32,       c->d_E,         c->d_E32,      c->d_E1,
-                    c->d_E1_32,     c->d_tnode,     c->d_tnbr,        c->d_tris,      c->d_tri_deg,  c->d_tgs,
+                    c->d_E1_32,     c->d_tnode,     c->d_tnbr,        c->d_tbox,      c->d_tris,      c->d_tri_deg,  c->d_tgs,
                     c->d_tgl,       c->d_sgs,       c->d_sgl,         c->d_tri_count, c->d_node_charge,
                     c->d_species,   c->d_cnt,       c->d_nactive,     c->d_runs,      c->d_tet_vol,  c->d_node_vol,
                     c->d_tet_q,     c->d_adj_start, c->d_adj_list,    c->d_tet_n,     c->d_phi,
