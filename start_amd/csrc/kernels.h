@@ -108,6 +108,15 @@ struct DevParticles {
     int64_t n;
 };
 
+// Device columns of a read-back in load order (null: not wanted): x, y, z,
+// vx, vy, vz, owner, settled or not, hit triangle.
+struct ReadBack {
+    double* f[6];
+    int32_t* tet;
+    int32_t* settled;
+    int32_t* hit;
+};
+
 // Where and when a particle settled, indexed by load index (recorded on
 // request, for the adjoint of the push and hit map): the absolute position at
 // the start of the step whose segment met the surface, and that step.

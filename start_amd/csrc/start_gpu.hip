@@ -51,8 +51,11 @@ void launch_push_table(hipStream_t s, const double* E, const float* E32, int64_t
 void launch_orient_batch(hipStream_t s, const double* pts, int64_t n, int32_t* out);
 void launch_math_batch(hipStream_t s, int which, const double* x, const double* y, int64_t n, double* out,
                        double* out2);
-void launch_abs_positions(hipStream_t s, const DevMesh& M, const float* lx, const float* ly, const float* lz,
-                          const int32_t* tet, int64_t n, double* x, double* y, double* z);
+void launch_init_rows(hipStream_t s, int64_t first, int64_t m, const int32_t* species, const RunK* runs,
+                      int32_t n_runs, int32_t* flags, int32_t* hit, uint32_t* pidx, int64_t* n_active, int64_t active,
+                      unsigned long long* step_cnt, unsigned long long step);
+template <typename R>
+void launch_load_order(hipStream_t s, const DevMesh& M, const DevParticles<R>& P, const ReadBack& out);
 size_t sort_temp_bytes(int64_t n, int nbits);
 template <typename R>
 hipError_t sort_particles(hipStream_t s, const DevParticles<R>& P, R* x, R* y, R* z, double* vx, double* vy, double* vz,
@@ -175,6 +178,8 @@ struct start_ctx {
     // runs: one for a single simulation, n_runs for a batch
     std::vector<RunK> runs;
     RunK* d_runs = nullptr;
+    size_t runs_cap = 0;     // entries of d_runs
+    size_t outputs_cap = 0;  // runs that d_node_charge and d_tri_count have room for
     unsigned long long* d_tri_count = nullptr;  // n_runs * n_tris
     double* d_node_charge = nullptr;            // two buffers of n_runs * n_nodes
     int cb = 0;                                 // buffer the next launch scatters into
@@ -183,13 +188,15 @@ struct start_ctx {
     // node charge density tables (built on first use)
     double *d_tet_vol = nullptr, *d_node_vol = nullptr, *d_tet_q = nullptr;
     int32_t *d_adj_start = nullptr, *d_adj_list = nullptr, *d_tet_n = nullptr;
-    // node density output: device buffers and pinned host staging, kept
-    // between calls (the step loop asks for it every step)
-    double* d_rho = nullptr;
-    int32_t* d_written = nullptr;
+    // node density output, page-locked and kept between calls (the step loop
+    // asks for it every step)
     double* h_rho = nullptr;
     int32_t* h_written = nullptr;
     unsigned long long* h_cnt = nullptr;  // page-locked copy of the counters (start_read_stats)
+    // staging of small transfers: one page-locked buffer and its device
+    // counterpart, kStageBytes each (allocated on first use)
+    unsigned char* h_stage = nullptr;
+    unsigned char* d_stage = nullptr;
     uint32_t* h_settle = nullptr;         // page-locked staging of settled load indices
     int64_t h_settle_cap = 0;
     // particles: n live rows in buffers of cap rows (appends grow cap geometrically)
@@ -576,22 +583,106 @@ int ensure_density_tables(start_ctx* c)
     return START_OK;
 }
 
+int ensure_counters(start_ctx* c)
+{
+    if (c->h_cnt) return START_OK;
+    // page-locked, so that the copy is one DMA behind the step
+    hipError_t e = host_pinned_malloc((void**)&c->h_cnt, sizeof(unsigned long long) * kCntTotal);
+    if (e != hipSuccess)
+        return fail(c, e == hipErrorOutOfMemory ? START_ERR_NOMEM : START_ERR_HIP,
+                    std::string("statistics buffer: ") + hipGetErrorString(e));
+    return START_OK;
+}
+
+// Waits for the stream and reports the kernels' error flag.
 int check_kernel_errors(start_ctx* c)
 {
-    unsigned long long h[kCntTotal];
-    HIPCHECK(c, hipMemcpyAsync(h, c->d_cnt, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+    int rc = ensure_counters(c);
+    if (rc != START_OK) return rc;
+    HIPCHECK(c, hipMemcpyAsync(c->h_cnt + kCntError, c->d_cnt + kCntError, sizeof(unsigned long long),
+                               hipMemcpyDeviceToHost, c->stream));
     HIPCHECK(c, hipStreamSynchronize(c->stream));
-    if (h[kCntError] & 1ull) return fail(c, START_ERR_KERNEL, "exact predicate expansion capacity exceeded");
+    if (c->h_cnt[kCntError] & 1ull) return fail(c, START_ERR_KERNEL, "exact predicate expansion capacity exceeded");
     return START_OK;
+}
+
+// The staging buffers, or false: the caller then copies from and to the user's
+// memory directly.  Up to this size one page-locked copy is the faster way
+// (a pageable copy waits 20 us or more, one for each array); beyond it the
+// extra pass over the data costs more than it saves.
+constexpr size_t kStageBytes = 1u << 20;
+bool have_stage(start_ctx* c)
+{
+    if (!c->h_stage) {
+        if (host_pinned_malloc((void**)&c->h_stage, kStageBytes) != hipSuccess) return false;
+    }
+    if (!c->d_stage && dev_malloc((void**)&c->d_stage, kStageBytes) != hipSuccess) return false;
+    return true;
+}
+
+// `bytes` from the device into the user's memory behind the stream's work, with
+// the kernels' error flag: one wait for both where they fit the staging buffer.
+int read_back(start_ctx* c, void* dst, const void* src, size_t bytes)
+{
+    const bool staged = bytes <= kStageBytes && have_stage(c);
+    HIPCHECK(c, hipMemcpyAsync(staged ? c->h_stage : dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    const int rc = check_kernel_errors(c);
+    if (rc == START_OK && staged) memcpy(dst, c->h_stage, bytes);
+    return rc;
+}
+
+// Device scratch of one call for n rows: the sort target and the work list,
+// whose contents never outlive a launch or a sort; memory of its own while a
+// failed growth has left the context without them.
+struct RowScratch {
+    double* rows = nullptr;                       // 5 n
+    double* col[3] = {nullptr, nullptr, nullptr};  // n each
+    int32_t* word[3] = {nullptr, nullptr, nullptr};  // n each
+    void* own = nullptr;
+    ~RowScratch()
+    {
+        if (own) (void)hipFree(own);
+    }
+    hipError_t get(start_ctx* c, int64_t n)
+    {
+        static_assert(sizeof(WorkItem) >= 5 * sizeof(double), "rows of five doubles");
+        if (c->d_sort_temp && n <= c->cap) {
+            rows = (double*)c->d_wl;
+            double* v[3] = {(double*)c->B.vx, (double*)c->B.vy, (double*)c->B.vz};
+            int32_t* w[3] = {c->B.tet, c->B.flags, c->B.hit};
+            for (int k = 0; k < 3; ++k) {
+                col[k] = v[k];
+                word[k] = w[k];
+            }
+            return hipSuccess;
+        }
+        hipError_t e = dev_malloc(&own, (size_t)std::max<int64_t>(n, 1) * (8 * sizeof(double) + 3 * sizeof(int32_t)));
+        if (e != hipSuccess) return e;
+        rows = (double*)own;
+        for (int k = 0; k < 3; ++k) {
+            col[k] = rows + (5 + k) * n;
+            word[k] = (int32_t*)(rows + 8 * n) + k * n;
+        }
+        return hipSuccess;
+    }
+};
+
+void load_order(start_ctx* c, const ReadBack& out)
+{
+    if (c->mixed) launch_load_order<float>(c->stream, c->mesh_view(), c->view<float>(), out);
+    else launch_load_order<double>(c->stream, c->mesh_view(), c->view<double>(), out);
 }
 
 int upload_runs(start_ctx* c)
 {
     for (RunK& r : c->runs) r.log2_conc = (float)log2_factor(r.conc);
     HIPCHECK(c, hipStreamSynchronize(c->stream));
-    if (c->d_runs) (void)hipFree(c->d_runs);
-    c->d_runs = nullptr;
-    HIPCHECK(c, dalloc(&c->d_runs, c->runs.size()));
+    if (c->runs.size() != c->runs_cap || !c->d_runs) {
+        if (c->d_runs) (void)hipFree(c->d_runs);
+        c->d_runs = nullptr;
+        HIPCHECK(c, dalloc(&c->d_runs, c->runs.size()));
+        c->runs_cap = c->runs.size();
+    }
     HIPCHECK(c, hipMemcpy(c->d_runs, c->runs.data(), sizeof(RunK) * c->runs.size(), hipMemcpyHostToDevice));
     drop_graphs(c);  // captured launches hold the old table pointer
     return START_OK;
@@ -667,6 +758,7 @@ int refresh_push_tables(start_ctx* c)
 // Per-run output buffers: node charge (two sets) and triangle counters.
 int alloc_run_outputs(start_ctx* c)
 {
+    if (c->outputs_cap == c->runs.size() && c->d_node_charge && c->d_tri_count) return START_OK;
     if (c->d_node_charge) (void)hipFree(c->d_node_charge);
     if (c->d_tri_count) (void)hipFree(c->d_tri_count);
     c->d_node_charge = nullptr;
@@ -677,6 +769,7 @@ int alloc_run_outputs(start_ctx* c)
     if (e != hipSuccess)
         return fail(c, e == hipErrorOutOfMemory ? START_ERR_NOMEM : START_ERR_HIP,
                     std::string("run buffers: ") + hipGetErrorString(e));
+    c->outputs_cap = c->runs.size();
     return START_OK;
 }
 
@@ -902,22 +995,37 @@ int check_cfg(start_ctx* c, const start_launch_cfg& g)
 int begin_population(start_ctx* c, const std::vector<RunK>& rk, int64_t n, const uint64_t* ids)
 {
     HIPCHECK(c, hipStreamSynchronize(c->stream));
-    free_particles(c);
+    // buffers that fit are kept (some 30 allocations and releases took 6 ms of
+    // a load of 1M particles); far larger ones are given back
+    const bool keep = c->d_sort_temp && c->A.x && n <= c->cap && c->cap <= std::max<int64_t>(4 * n, 65536);
+    if (keep) {
+        drop_graphs(c);
+        free_tracking(c);
+        if (c->d_settle && !c->record) {
+            (void)hipFree(c->d_settle);
+            c->d_settle = nullptr;
+        }
+        c->n = 0;
+    } else {
+        free_particles(c);
+    }
     c->runs = rk;
     int rc = upload_runs(c);
     if (rc != START_OK) return rc;
     rc = alloc_run_outputs(c);
     if (rc != START_OK) return rc;
-    hipError_t he = alloc_pbuf(c->A, n, c->es);
-    if (he == hipSuccess) he = alloc_work_buffers(c, n);
-    if (he == hipSuccess) he = dalloc(&c->d_settle_log, n);
-    if (he != hipSuccess) {
-        free_particles(c);
-        return fail(c, he == hipErrorOutOfMemory ? START_ERR_NOMEM : START_ERR_HIP,
-                    std::string("particle allocation failed: ") + hipGetErrorString(he));
+    if (!keep) {
+        hipError_t he = alloc_pbuf(c->A, n, c->es);
+        if (he == hipSuccess) he = alloc_work_buffers(c, n);
+        if (he == hipSuccess) he = dalloc(&c->d_settle_log, n);
+        if (he != hipSuccess) {
+            free_particles(c);
+            return fail(c, he == hipErrorOutOfMemory ? START_ERR_NOMEM : START_ERR_HIP,
+                        std::string("particle allocation failed: ") + hipGetErrorString(he));
+        }
+        c->cap = n;
     }
     c->n = n;
-    c->cap = n;
     c->ids.assign(ids ? ids : (const uint64_t*)nullptr, ids ? ids + n : (const uint64_t*)nullptr);
     if (!ids) {
         c->ids.resize((size_t)n);
@@ -930,10 +1038,9 @@ int begin_population(start_ctx* c, const std::vector<RunK>& rk, int64_t n, const
                                c->stream));
     HIPCHECK(c, hipMemsetAsync(c->d_node_charge, 0, sizeof(double) * 2 * CL, c->stream));
     if (c->record) {  // no particle has settled yet: step = -1 in every record
-        HIPCHECK(c, dalloc(&c->d_settle, n));
-        HIPCHECK(c, hipMemsetAsync(c->d_settle, 0xff, sizeof(SettleRec) * std::max<int64_t>(n, 1), c->stream));
+        if (!c->d_settle) HIPCHECK(c, dalloc(&c->d_settle, c->cap));
+        HIPCHECK(c, hipMemsetAsync(c->d_settle, 0xff, sizeof(SettleRec) * std::max<int64_t>(c->cap, 1), c->stream));
     }
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
     c->cb = 0;
     c->latest = 0;
     c->wslot = 0;
@@ -1010,52 +1117,49 @@ int grow_particles(start_ctx* c, int64_t need)
 }
 
 // Rows [first, first + m) of the live buffers from host arrays: the state
-// (positions in the frame of their owner in mixed mode, velocities FP64),
-// the flags given, hit = -1, load indices first.., and owners by the locate
-// kernel (min-id closed containment).
+// (positions in the frame of their owner in mixed mode, velocities FP64), the
+// flags of their species and run, hit = -1, load indices first.., and owners by
+// the locate kernel (min-id closed containment); the live row count becomes
+// first + m.  Queued on the stream: the caller waits.
 int upload_rows(start_ctx* c, int64_t first, int64_t m, const double* x, const double* y, const double* z,
-                const double* vx, const double* vy, const double* vz, const int32_t* flags)
+                const double* vx, const double* vy, const double* vz, const int32_t* species)
 {
     if (m == 0) return START_OK;
-    std::vector<uint32_t> pidx((size_t)m);
-    for (int64_t i = 0; i < m; ++i) pidx[(size_t)i] = (uint32_t)(first + i);
-    std::vector<int32_t> hit((size_t)m, -1);
-    HIPCHECK(c, hipMemcpy(c->A.hit + first, hit.data(), sizeof(int32_t) * m, hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->A.pidx + first, pidx.data(), sizeof(uint32_t) * m, hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->A.flags + first, flags, sizeof(int32_t) * m, hipMemcpyHostToDevice));
+    const double* src[6] = {x, y, z, vx, vy, vz};
+    double* dst[6] = {(double*)c->A.x, (double*)c->A.y, (double*)c->A.z,
+                      (double*)c->A.vx, (double*)c->A.vy, (double*)c->A.vz};
     const size_t b8 = sizeof(double) * (size_t)m;
-    DevMesh M = c->mesh_view();
-    if (!c->mixed) {
-        const double* src[6] = {x, y, z, vx, vy, vz};
-        void* dst[6] = {c->A.x, c->A.y, c->A.z, c->A.vx, c->A.vy, c->A.vz};
-        for (int k = 0; k < 6; ++k) HIPCHECK(c, hipMemcpy((double*)dst[k] + first, src[k], b8, hipMemcpyHostToDevice));
-        launch_locate(c->stream, M, (double*)c->A.x + first, (double*)c->A.y + first, (double*)c->A.z + first, m,
-                      c->A.tet + first, c->A.flags + first, nullptr, nullptr, nullptr, c->d_cnt);
-    } else {
-        // positions go to the frame of their owner
-        double *dx = nullptr, *dy = nullptr, *dz = nullptr;
-        hipError_t e = dalloc(&dx, m);
-        if (e == hipSuccess) e = dalloc(&dy, m);
-        if (e == hipSuccess) e = dalloc(&dz, m);
-        if (e == hipSuccess) e = hipMemcpy(dx, x, b8, hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(dy, y, b8, hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(dz, z, b8, hipMemcpyHostToDevice);
-        if (e == hipSuccess) {
-            launch_locate(c->stream, M, dx, dy, dz, m, c->A.tet + first, c->A.flags + first, (float*)c->A.x + first,
-                          (float*)c->A.y + first, (float*)c->A.z + first, c->d_cnt);
-            e = hipStreamSynchronize(c->stream);
-        }
-        if (dx) (void)hipFree(dx);
-        if (dy) (void)hipFree(dy);
-        if (dz) (void)hipFree(dz);
+    RowScratch tmp;
+    if (c->mixed) {  // positions go to the frame of their owner
+        hipError_t e = tmp.get(c, m);
         if (e != hipSuccess) return fail(c, START_ERR_HIP, std::string("particle upload: ") + hipGetErrorString(e));
-        const double* vs[3] = {vx, vy, vz};
-        void* vd[3] = {c->A.vx, c->A.vy, c->A.vz};
-        for (int k = 0; k < 3; ++k)
-            HIPCHECK(c, hipMemcpy((double*)vd[k] + first, vs[k], b8, hipMemcpyHostToDevice));
     }
+    double* pos[3];
+    for (int k = 0; k < 3; ++k) pos[k] = c->mixed ? tmp.col[k] : dst[k] + first;
+    const int32_t* d_species;
+    const size_t total = 6 * b8 + sizeof(int32_t) * (size_t)m;
+    if (total <= kStageBytes && have_stage(c)) {
+        for (int k = 0; k < 6; ++k) memcpy(c->h_stage + k * b8, src[k], b8);
+        memcpy(c->h_stage + 6 * b8, species, sizeof(int32_t) * (size_t)m);
+        HIPCHECK(c, hipMemcpyAsync(c->d_stage, c->h_stage, total, hipMemcpyHostToDevice, c->stream));
+        for (int k = 0; k < 6; ++k)
+            HIPCHECK(c, hipMemcpyAsync(k < 3 ? (void*)pos[k] : (void*)(dst[k] + first), c->d_stage + k * b8, b8,
+                                       hipMemcpyDeviceToDevice, c->stream));
+        d_species = (const int32_t*)(c->d_stage + 6 * b8);
+    } else {
+        for (int k = 0; k < 6; ++k)
+            HIPCHECK(c, hipMemcpyAsync(k < 3 ? (void*)pos[k] : (void*)(dst[k] + first), src[k], b8,
+                                       hipMemcpyHostToDevice, c->stream));
+        HIPCHECK(c, hipMemcpyAsync(c->A.flags + first, species, sizeof(int32_t) * (size_t)m, hipMemcpyHostToDevice,
+                                   c->stream));
+        d_species = c->A.flags + first;
+    }
+    launch_init_rows(c->stream, first, m, d_species, c->d_runs, (int32_t)c->runs.size(), c->A.flags, c->A.hit,
+                     c->A.pidx, c->d_nactive, first + m, c->d_cnt + kCntStep + c->wslot, (unsigned long long)c->step);
+    launch_locate(c->stream, c->mesh_view(), pos[0], pos[1], pos[2], m, c->A.tet + first, c->A.flags + first,
+                  c->mixed ? (float*)c->A.x + first : nullptr, c->mixed ? (float*)c->A.y + first : nullptr,
+                  c->mixed ? (float*)c->A.z + first : nullptr, c->d_cnt);
     HIPCHECK(c, hipGetLastError());
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
     return START_OK;
 }
 
@@ -1139,19 +1243,6 @@ int assign_track_slots(start_ctx* c, int64_t first)
     return START_OK;
 }
 
-// hit = -1, load indices 0..n-1 and the live count of a new population.
-int init_population_tail(start_ctx* c, int64_t n)
-{
-    std::vector<uint32_t> pidx((size_t)n);
-    for (int64_t i = 0; i < n; ++i) pidx[(size_t)i] = (uint32_t)i;
-    std::vector<int32_t> hit((size_t)n, -1);
-    HIPCHECK(c, hipMemcpy(c->A.hit, hit.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->A.pidx, pidx.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
-    int64_t nact = n;
-    HIPCHECK(c, hipMemcpy(c->d_nactive, &nact, sizeof(int64_t), hipMemcpyHostToDevice));
-    return START_OK;
-}
-
 }  // namespace
 
 extern "C" {
@@ -1217,6 +1308,7 @@ int start_create(start_ctx** out, const start_mesh_desc* mesh, const start_param
     r0.key = params->run;
     r0.log2_conc = (float)log2_factor(r0.conc);
     c->runs.assign(1, r0);
+    c->runs_cap = c->outputs_cap = 1;
     std::vector<float> g32;
     if (c->mixed) {
         c->tau32 = build_geo32(c->hm, g32);
@@ -1304,7 +1396,7 @@ void start_destroy(start_ctx* c)
                     c->d_tgl,       c->d_sgs,       c->d_sgl,         c->d_tri_count, c->d_node_charge,
                     c->d_species,   c->d_cnt,       c->d_nactive,     c->d_runs,      c->d_tet_vol,  c->d_node_vol,
                     c->d_tet_q,     c->d_adj_start, c->d_adj_list,    c->d_tet_n,     c->d_phi,
-                    c->d_rho,       c->d_written,   c->d_H,           c->d_H32};
+                    c->d_H,         c->d_H32,       c->d_stage};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (c->h_phi) (void)hipHostFree(c->h_phi);
@@ -1312,6 +1404,7 @@ void start_destroy(start_ctx* c)
     if (c->h_written) (void)hipHostFree(c->h_written);
     if (c->h_cnt) (void)hipHostFree(c->h_cnt);
     if (c->h_settle) (void)hipHostFree(c->h_settle);
+    if (c->h_stage) (void)hipHostFree(c->h_stage);
     if (c->phi_copied) (void)hipEventDestroy(c->phi_copied);
     for (auto& e : c->events) {
         (void)hipEventDestroy(e.a0);
@@ -1338,7 +1431,6 @@ int start_load_batch(start_ctx* c, int32_t n_runs, const start_run_desc* runs, c
     if ((int64_t)n_runs * c->hm.n_nodes > (int64_t)0x7fffffff)
         return fail(c, START_ERR_ARG, "n_runs * n_nodes exceeds the node-charge index range");
     if (n > 0 && (!x || !y || !z || !vx || !vy || !vz || !species)) return fail(c, START_ERR_ARG, "null particle array");
-    std::vector<int32_t> flags((size_t)n);
     std::vector<RunK> rk((size_t)n_runs);
     {
         int64_t i = 0;
@@ -1350,23 +1442,22 @@ int start_load_batch(start_ctx* c, int32_t n_runs, const start_run_desc* runs, c
             rk[(size_t)r].first = (uint32_t)i;
             rk[(size_t)r].node_base = (int64_t)r * c->hm.n_nodes;
             rk[(size_t)r].tri_base = (int64_t)r * c->hm.n_tris;
-            for (int64_t j = 0; j < runs[r].n_particles; ++j, ++i) {
+            for (int64_t j = 0; j < runs[r].n_particles; ++j, ++i)
                 if (species[i] < 0 || species[i] >= (int32_t)c->species.size())
                     return fail(c, START_ERR_ARG, "species index out of range at particle " + std::to_string(i));
-                flags[(size_t)i] = (species[i] << kSpeciesShift) | (r << kRunShift);
-            }
         }
     }
     int rc = begin_population(c, rk, n, ids);
     if (rc != START_OK) return rc;
     c->present.assign(c->species.size(), 0);
     rc = mark_present(c, species, n);
-    if (rc != START_OK || n == 0) return rc;
-    int64_t nact = n;
-    HIPCHECK(c, hipMemcpy(c->d_nactive, &nact, sizeof(int64_t), hipMemcpyHostToDevice));
-    rc = upload_rows(c, 0, n, x, y, z, vx, vy, vz, flags.data());
     if (rc != START_OK) return rc;
-    HIPCHECK(c, hipGetLastError());
+    if (n == 0) {
+        HIPCHECK(c, hipStreamSynchronize(c->stream));
+        return START_OK;
+    }
+    rc = upload_rows(c, 0, n, x, y, z, vx, vy, vz, species);
+    if (rc != START_OK) return rc;
     if (c->cfg.sort_interval > 0) {
         int rc2 = sort_now(c);
         if (rc2 != START_OK) return rc2;
@@ -1474,26 +1565,30 @@ int start_generate(start_ctx* c, int32_t n_sources, const start_source_desc* src
         rc = mark_present(c, sps.data(), n_sources);
         if (rc != START_OK) return rc;
     }
-    rc = init_population_tail(c, n);
-    if (rc != START_OK) return rc;
-    double *d_cen = nullptr, *d_nor = nullptr, *t[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    hipError_t e = dalloc(&d_cen, cen.size());
-    if (e == hipSuccess) e = dalloc(&d_nor, nor.size());
-    if (e == hipSuccess) e = hipMemcpy(d_cen, cen.data(), sizeof(double) * cen.size(), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(d_nor, nor.data(), sizeof(double) * nor.size(), hipMemcpyHostToDevice);
-    // FP64 state: drawn in place; mixed: positions drawn into FP64 scratch,
-    // then to the owner's frame (by the locate); velocities in place
+    // the cell tables in the work list where they fit; mixed: positions drawn
+    // into FP64 scratch, then to the owner's frame (by the locate)
+    RowScratch tmp;
+    hipError_t e = c->mixed ? tmp.get(c, n) : hipSuccess;
+    double *d_own = nullptr, *d_cen = (double*)c->d_wl;
+    if (e == hipSuccess && sizeof(double) * (cen.size() + nor.size()) > sizeof(WorkItem) * (size_t)c->cap) {
+        e = dalloc(&d_own, cen.size() + nor.size());
+        d_cen = d_own;
+    }
+    double* d_nor = d_cen + cen.size();
+    if (e == hipSuccess && !cen.empty())
+        e = hipMemcpyAsync(d_cen, cen.data(), sizeof(double) * cen.size(), hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess && !nor.empty())
+        e = hipMemcpyAsync(d_nor, nor.data(), sizeof(double) * nor.size(), hipMemcpyHostToDevice, c->stream);
     double* dst[6] = {(double*)c->A.x, (double*)c->A.y, (double*)c->A.z,
                       (double*)c->A.vx, (double*)c->A.vy, (double*)c->A.vz};
     if (c->mixed)
-        for (int q = 0; q < 3 && e == hipSuccess; ++q) {
-            e = dalloc(&t[q], n);
-            dst[q] = t[q];
-        }
+        for (int q = 0; q < 3; ++q) dst[q] = tmp.col[q];
     if (e == hipSuccess) {
         for (int32_t s = 0; s < n_sources; ++s)
             launch_generate(c->stream, sk[(size_t)s], (uint32_t)s, seed, d_cen, d_nor, dst[0], dst[1], dst[2],
                             dst[3], dst[4], dst[5], c->A.flags);
+        launch_init_rows(c->stream, 0, n, nullptr, c->d_runs, 1, c->A.flags, c->A.hit, c->A.pidx, c->d_nactive, n,
+                         c->d_cnt + kCntStep + c->wslot, (unsigned long long)c->step);
         DevMesh M = c->mesh_view();
         if (!c->mixed) {
             launch_locate(c->stream, M, dst[0], dst[1], dst[2], n, c->A.tet, c->A.flags, nullptr, nullptr, nullptr,
@@ -1505,10 +1600,7 @@ int start_generate(start_ctx* c, int32_t n_sources, const start_source_desc* src
         e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     }
-    (void)hipFree(d_cen);
-    (void)hipFree(d_nor);
-    for (double* p : t)
-        if (p) (void)hipFree(p);
+    if (d_own) (void)hipFree(d_own);
     if (e != hipSuccess) return fail(c, START_ERR_HIP, std::string("particle sources: ") + hipGetErrorString(e));
     if (c->cfg.sort_interval > 0) {
         rc = sort_now(c);
@@ -1526,31 +1618,26 @@ int start_append_particles(start_ctx* c, int64_t m, const double* x, const doubl
     if (m == 0) return START_OK;
     if (c->n_runs() != 1) return fail(c, START_ERR_STATE, "particles can be appended to a single simulation only");
     if (!x || !y || !z || !vx || !vy || !vz || !species) return fail(c, START_ERR_ARG, "null particle array");
-    std::vector<int32_t> flags((size_t)m);
-    for (int64_t i = 0; i < m; ++i) {
+    for (int64_t i = 0; i < m; ++i)
         if (species[i] < 0 || species[i] >= (int32_t)c->species.size())
             return fail(c, START_ERR_ARG, "species index out of range at particle " + std::to_string(i));
-        flags[(size_t)i] = species[i] << kSpeciesShift;  // run 0
-    }
     const int64_t n0 = c->n;
     int rc = grow_particles(c, n0 + m);
     if (rc != START_OK) return rc;
     rc = mark_present(c, species, m);
     if (rc != START_OK) return rc;
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    // launches read their first step from the device counter, which steps
-    // taken while the context held no particles did not advance
-    const unsigned long long step_now = (unsigned long long)c->step;
-    HIPCHECK(c, hipMemcpy(c->d_cnt + kCntStep + c->wslot, &step_now, sizeof(step_now), hipMemcpyHostToDevice));
-    rc = upload_rows(c, n0, m, x, y, z, vx, vy, vz, flags.data());
+    if (!c->graphs.empty()) {  // captured launches hold the old particle count
+        HIPCHECK(c, hipStreamSynchronize(c->stream));
+        drop_graphs(c);
+    }
+    // (launches read their first step from the device counter, which steps
+    // taken while the context held no particles did not advance; after a sort
+    // the settled particles close the live prefix, and the kernels cover every
+    // row until the next sort compacts them again)
+    rc = upload_rows(c, n0, m, x, y, z, vx, vy, vz, species);
     if (rc != START_OK) return rc;
     c->n = n0 + m;
     for (int64_t i = 0; i < m; ++i) c->ids.push_back(ids ? ids[i] : (uint64_t)(n0 + i));
-    // after a sort the settled particles close the live prefix; the kernels
-    // cover every row until the next sort compacts them again
-    int64_t nact = c->n;
-    HIPCHECK(c, hipMemcpy(c->d_nactive, &nact, sizeof(int64_t), hipMemcpyHostToDevice));
-    drop_graphs(c);  // captured launches hold the old particle count
     rc = assign_track_slots(c, n0);
     if (rc != START_OK) return rc;
     return check_kernel_errors(c);
@@ -1980,11 +2067,10 @@ int start_read_hits(start_ctx* c, double* hit_xyz, int32_t* hit_tri, int32_t* se
     if (c->n == 0) return START_OK;
     if (!c->d_settle) return fail(c, START_ERR_STATE, "settle records are off (start_record_settle)");
     const int64_t n = c->n;
-    double* dx = nullptr;
-    int32_t *dt = nullptr, *ds = nullptr;
-    hipError_t e = dalloc(&dx, 3 * n);
-    if (e == hipSuccess) e = dalloc(&dt, n);
-    if (e == hipSuccess) e = dalloc(&ds, n);
+    RowScratch tmp;
+    hipError_t e = tmp.get(c, n);
+    double* dx = tmp.rows;
+    int32_t *dt = tmp.word[0], *ds = tmp.word[1];
     if (e == hipSuccess) {
         if (c->mixed) launch_hit_points<float>(c->stream, c->mesh_view(), c->view<float>(), c->d_settle, dx, dt, ds);
         else launch_hit_points<double>(c->stream, c->mesh_view(), c->view<double>(), c->d_settle, dx, dt, ds);
@@ -1994,9 +2080,6 @@ int start_read_hits(start_ctx* c, double* hit_xyz, int32_t* hit_tri, int32_t* se
     if (e == hipSuccess) e = hipMemcpyAsync(hit_tri, dt, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(settle_step, ds, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (dx) (void)hipFree(dx);
-    if (dt) (void)hipFree(dt);
-    if (ds) (void)hipFree(ds);
     if (e != hipSuccess) return fail(c, START_ERR_HIP, std::string("hit points: ") + hipGetErrorString(e));
     return START_OK;
 }
@@ -2012,9 +2095,9 @@ int start_adjoint_push(start_ctx* c, const double* lambda, int32_t first_step, d
     if (c->prm.gas.model != START_MODEL_NONE)
         return fail(c, START_ERR_STATE, "the adjoint covers the collisionless push (gas model NONE)");
     const int64_t n = c->n;
-    double *dl = nullptr, *dg = nullptr;
-    hipError_t e = dalloc(&dl, 3 * n);
-    if (e == hipSuccess) e = dalloc(&dg, 2);
+    RowScratch tmp;
+    hipError_t e = tmp.get(c, n);
+    double *dl = tmp.rows, *dg = dl + 3 * n;  // (a row has room for five)
     if (e == hipSuccess) e = hipMemcpyAsync(dl, lambda, sizeof(double) * 3 * n, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(dg, 0, sizeof(double) * 2, c->stream);
     if (e == hipSuccess) {
@@ -2028,8 +2111,6 @@ int start_adjoint_push(start_ctx* c, const double* lambda, int32_t first_step, d
     }
     if (e == hipSuccess) e = hipMemcpyAsync(grad, dg, sizeof(double) * 2, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (dl) (void)hipFree(dl);
-    if (dg) (void)hipFree(dg);
     if (e != hipSuccess) return fail(c, START_ERR_HIP, std::string("adjoint: ") + hipGetErrorString(e));
     return check_kernel_errors(c);
 }
@@ -2052,19 +2133,13 @@ int start_gather_charge(start_ctx* c)
 int start_read_node_charge_runs(start_ctx* c, double* out)
 {
     if (!c || !out) return fail(c, START_ERR_ARG, "null argument");
-    HIPCHECK(c, hipMemcpyAsync(out, c->d_node_charge + (size_t)c->latest * c->charge_len(),
-                               sizeof(double) * c->charge_len(), hipMemcpyDeviceToHost, c->stream));
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    return check_kernel_errors(c);
+    return read_back(c, out, c->d_node_charge + (size_t)c->latest * c->charge_len(), sizeof(double) * c->charge_len());
 }
 
 int start_read_node_charge(start_ctx* c, double* out)
 {
     if (!c || !out) return fail(c, START_ERR_ARG, "null argument");
-    HIPCHECK(c, hipMemcpyAsync(out, c->d_node_charge + (size_t)c->latest * c->charge_len(),
-                               sizeof(double) * c->hm.n_nodes, hipMemcpyDeviceToHost, c->stream));
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    return check_kernel_errors(c);
+    return read_back(c, out, c->d_node_charge + (size_t)c->latest * c->charge_len(), sizeof(double) * c->hm.n_nodes);
 }
 
 }  // extern "C"
@@ -2081,10 +2156,8 @@ int node_density_to_host(start_ctx* c, int32_t mode, bool want_written)
     int rc = ensure_density_tables(c);
     if (rc != START_OK) return rc;
     const int64_t M = c->hm.n_nodes, T = c->hm.n_tets;
-    if (!c->d_rho) {
-        hipError_t e = dalloc(&c->d_rho, M);
-        if (e == hipSuccess) e = dalloc(&c->d_written, M);
-        if (e == hipSuccess) e = host_pinned_malloc((void**)&c->h_rho, sizeof(double) * (size_t)M);
+    if (!c->h_written) {
+        hipError_t e = c->h_rho ? hipSuccess : host_pinned_malloc((void**)&c->h_rho, sizeof(double) * (size_t)M);
         if (e == hipSuccess)
             e = host_pinned_malloc((void**)&c->h_written, sizeof(int32_t) * (size_t)M);
         if (e != hipSuccess)
@@ -2096,18 +2169,21 @@ int node_density_to_host(start_ctx* c, int32_t mode, bool want_written)
         HIPCHECK(c, hipMemsetAsync(c->d_tet_n, 0, sizeof(int32_t) * T, c->stream));
     }
     const double* q = c->d_node_charge + (size_t)c->latest * M;
+    // the kernel writes the page-locked buffers themselves: 1 MB crosses the
+    // bus with the kernel's stores instead of in a copy behind it
+    double* const rho = c->h_rho;
+    int32_t* const written = want_written && mode == START_DENSITY_TET_AVERAGE ? c->h_written : nullptr;
     if (c->mixed)
         launch_node_density<float>(c->stream, c->view<float>(), c->d_species, mode, q, c->d_node_vol,
-                                   c->d_adj_start, c->d_adj_list, c->d_tet_vol, c->d_tet_q, c->d_tet_n, M, c->d_rho,
-                                   c->d_written);
+                                   c->d_adj_start, c->d_adj_list, c->d_tet_vol, c->d_tet_q, c->d_tet_n, M, rho,
+                                   written);
     else
         launch_node_density<double>(c->stream, c->view<double>(), c->d_species, mode, q, c->d_node_vol,
-                                    c->d_adj_start, c->d_adj_list, c->d_tet_vol, c->d_tet_q, c->d_tet_n, M, c->d_rho,
-                                    c->d_written);
+                                    c->d_adj_start, c->d_adj_list, c->d_tet_vol, c->d_tet_q, c->d_tet_n, M, rho,
+                                    written);
     HIPCHECK(c, hipGetLastError());
-    HIPCHECK(c, hipMemcpyAsync(c->h_rho, c->d_rho, sizeof(double) * M, hipMemcpyDeviceToHost, c->stream));
-    if (want_written)
-        HIPCHECK(c, hipMemcpyAsync(c->h_written, c->d_written, sizeof(int32_t) * M, hipMemcpyDeviceToHost, c->stream));
+    // (every node has a barycentric value: its mask needs no device)
+    if (want_written && !written) std::fill(c->h_written, c->h_written + M, 1);
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     return START_OK;
 }
@@ -2141,64 +2217,79 @@ int start_read_particles(start_ctx* c, double* x, double* y, double* z, double* 
                          int32_t* tet, int32_t* status, int32_t* hit_tri)
 {
     if (!c) return fail(nullptr, START_ERR_ARG, "null context");
-    int64_t n = c->n;
+    const int64_t n = c->n;
     if (n == 0) return START_OK;
     hipStream_t s = c->stream;
-    // device order differs from load order after a sort: bring back by load index
-    std::vector<uint32_t> pidx((size_t)n);
-    HIPCHECK(c, hipMemcpyAsync(pidx.data(), c->A.pidx, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, s));
-    std::vector<double> tmp((size_t)n);
-    std::vector<int32_t> itmp((size_t)n);
-    double* pos_src[3] = {nullptr, nullptr, nullptr};
-    double* abs_buf = nullptr;
-    if (c->mixed && (x || y || z)) {
-        HIPCHECK(c, dalloc(&abs_buf, 3 * n));
-        launch_abs_positions(s, c->mesh_view(), (float*)c->A.x, (float*)c->A.y, (float*)c->A.z, c->A.tet, n, abs_buf,
-                             abs_buf + n, abs_buf + 2 * n);
-        pos_src[0] = abs_buf;
-        pos_src[1] = abs_buf + n;
-        pos_src[2] = abs_buf + 2 * n;
-    } else if (!c->mixed) {
-        pos_src[0] = (double*)c->A.x;
-        pos_src[1] = (double*)c->A.y;
-        pos_src[2] = (double*)c->A.z;
-    }
-    double* ddst[6] = {x, y, z, vx, vy, vz};
-    void* vsrc[3] = {c->A.vx, c->A.vy, c->A.vz};
-    hipError_t e = hipSuccess;
-    for (int k = 0; k < 6 && e == hipSuccess; ++k) {
-        if (!ddst[k]) continue;
-        const void* src = k < 3 ? (const void*)pos_src[k] : vsrc[k - 3];
-        e = hipMemcpyAsync(tmp.data(), src, sizeof(double) * n, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e == hipSuccess)
-            for (int64_t j = 0; j < n; ++j) ddst[k][pidx[(size_t)j]] = tmp[(size_t)j];
-    }
-    if (abs_buf) (void)hipFree(abs_buf);
-    if (e != hipSuccess) return fail(c, START_ERR_HIP, std::string("read particles: ") + hipGetErrorString(e));
-    int32_t* isrc[3] = {c->A.tet, c->A.flags, c->A.hit};
+    double* fdst[6] = {x, y, z, vx, vy, vz};
     int32_t* idst[3] = {tet, status, hit_tri};
-    for (int k = 0; k < 3; ++k) {
-        if (!idst[k]) continue;
-        HIPCHECK(c, hipMemcpyAsync(itmp.data(), isrc[k], sizeof(int32_t) * n, hipMemcpyDeviceToHost, s));
-        HIPCHECK(c, hipStreamSynchronize(s));
-        for (int64_t j = 0; j < n; ++j) {
-            int32_t v = itmp[(size_t)j];
-            if (k == 1) v = (v & kSettled) ? START_SETTLED : START_ACTIVE;
-            idst[k][pidx[(size_t)j]] = v;
-        }
+    const size_t b8 = sizeof(double) * (size_t)n, b4 = sizeof(int32_t) * (size_t)n;
+    // device order differs from load order after a sort: the rows are written
+    // by load index on the device and then copied
+    ReadBack out{};
+    int32_t** iout[3] = {&out.tet, &out.settled, &out.hit};
+    size_t total = 0;
+    for (double* p : fdst) total += p ? b8 : 0;
+    for (int32_t* p : idst) total += p ? b4 : 0;
+    const bool staged = total <= kStageBytes && have_stage(c);
+    RowScratch tmp;
+    if (staged) {
+        size_t at = 0;
+        for (int k = 0; k < 6; ++k)
+            if (fdst[k]) {
+                out.f[k] = (double*)(c->d_stage + at);
+                at += b8;
+            }
+        for (int k = 0; k < 3; ++k)
+            if (idst[k]) {
+                *iout[k] = (int32_t*)(c->d_stage + at);
+                at += b4;
+            }
+    } else {
+        hipError_t e = tmp.get(c, n);
+        if (e != hipSuccess)
+            return fail(c, e == hipErrorOutOfMemory ? START_ERR_NOMEM : START_ERR_HIP,
+                        std::string("read particles: ") + hipGetErrorString(e));
+        for (int k = 0; k < 6; ++k)
+            if (fdst[k]) out.f[k] = k < 3 ? tmp.rows + k * n : tmp.col[k - 3];
+        for (int k = 0; k < 3; ++k)
+            if (idst[k]) *iout[k] = tmp.word[k];
     }
-    HIPCHECK(c, hipStreamSynchronize(s));
-    return check_kernel_errors(c);
+    load_order(c, out);
+    HIPCHECK(c, hipGetLastError());
+    if (staged) {
+        HIPCHECK(c, hipMemcpyAsync(c->h_stage, c->d_stage, total, hipMemcpyDeviceToHost, s));
+    } else {
+        for (int k = 0; k < 6; ++k)
+            if (fdst[k]) HIPCHECK(c, hipMemcpyAsync(fdst[k], out.f[k], b8, hipMemcpyDeviceToHost, s));
+        for (int k = 0; k < 3; ++k)
+            if (idst[k]) HIPCHECK(c, hipMemcpyAsync(idst[k], *iout[k], b4, hipMemcpyDeviceToHost, s));
+    }
+    const int rc = check_kernel_errors(c);
+    if (rc != START_OK || !staged) return rc;
+    size_t at = 0;
+    for (double* p : fdst)
+        if (p) {
+            memcpy(p, c->h_stage + at, b8);
+            at += b8;
+        }
+    for (int32_t* p : idst)
+        if (p) {
+            memcpy(p, c->h_stage + at, b4);
+            at += b4;
+        }
+    return START_OK;
 }
 
 int start_read_tri_counts(start_ctx* c, uint64_t* counts)
 {
     if (!c || !counts) return fail(c, START_ERR_ARG, "null argument");
     if (c->hm.n_tris == 0) return START_OK;
-    HIPCHECK(c, hipMemcpyAsync(counts, c->d_tri_count, sizeof(uint64_t) * c->hm.n_tris, hipMemcpyDeviceToHost,
-                               c->stream));
+    const size_t bytes = sizeof(uint64_t) * c->hm.n_tris;
+    const bool staged = bytes <= kStageBytes && have_stage(c);
+    HIPCHECK(c, hipMemcpyAsync(staged ? (void*)c->h_stage : (void*)counts, c->d_tri_count, bytes,
+                               hipMemcpyDeviceToHost, c->stream));
     HIPCHECK(c, hipStreamSynchronize(c->stream));
+    if (staged) memcpy(counts, c->h_stage, bytes);
     return START_OK;
 }
 
@@ -2206,25 +2297,33 @@ int start_read_tri_counts_runs(start_ctx* c, uint64_t* counts)
 {
     if (!c || !counts) return fail(c, START_ERR_ARG, "null argument");
     if (c->hm.n_tris == 0) return START_OK;
-    HIPCHECK(c, hipMemcpyAsync(counts, c->d_tri_count, sizeof(uint64_t) * c->n_runs() * c->hm.n_tris,
+    const size_t bytes = sizeof(uint64_t) * c->n_runs() * c->hm.n_tris;
+    const bool staged = bytes <= kStageBytes && have_stage(c);
+    HIPCHECK(c, hipMemcpyAsync(staged ? (void*)c->h_stage : (void*)counts, c->d_tri_count, bytes,
                                hipMemcpyDeviceToHost, c->stream));
     HIPCHECK(c, hipStreamSynchronize(c->stream));
+    if (staged) memcpy(counts, c->h_stage, bytes);
     return START_OK;
 }
 
 int start_read_settled(start_ctx* c, uint64_t* ids, int64_t* n)
 {
     if (!c || !n) return fail(c, START_ERR_ARG, "null argument");
-    std::vector<int32_t> flags((size_t)c->n);
-    std::vector<uint32_t> pidx((size_t)c->n);
+    std::vector<int32_t> settled((size_t)c->n);
     if (c->n) {
-        HIPCHECK(c, hipMemcpyAsync(flags.data(), c->A.flags, sizeof(int32_t) * c->n, hipMemcpyDeviceToHost, c->stream));
-        HIPCHECK(c, hipMemcpyAsync(pidx.data(), c->A.pidx, sizeof(uint32_t) * c->n, hipMemcpyDeviceToHost, c->stream));
+        RowScratch tmp;
+        hipError_t e = tmp.get(c, c->n);
+        if (e != hipSuccess)
+            return fail(c, e == hipErrorOutOfMemory ? START_ERR_NOMEM : START_ERR_HIP,
+                        std::string("settled ids: ") + hipGetErrorString(e));
+        ReadBack out{};
+        out.settled = tmp.word[0];
+        load_order(c, out);
+        HIPCHECK(c, hipGetLastError());
+        HIPCHECK(c, hipMemcpyAsync(settled.data(), out.settled, sizeof(int32_t) * (size_t)c->n, hipMemcpyDeviceToHost,
+                                   c->stream));
     }
     HIPCHECK(c, hipStreamSynchronize(c->stream));
-    std::vector<uint8_t> settled((size_t)c->n, 0);
-    for (int64_t j = 0; j < c->n; ++j)
-        if (flags[(size_t)j] & kSettled) settled[pidx[(size_t)j]] = 1;
     int64_t cap = *n, k = 0;
     for (int64_t i = 0; i < c->n; ++i)
         if (settled[(size_t)i]) {
@@ -2238,11 +2337,9 @@ int start_read_settled(start_ctx* c, uint64_t* ids, int64_t* n)
 int start_read_settled_since(start_ctx* c, int64_t first, uint64_t* ids, int64_t* n)
 {
     if (!c || !n || first < 0) return fail(c, START_ERR_ARG, "bad argument");
-    if (!c->h_cnt) {
-        hipError_t e = host_pinned_malloc((void**)&c->h_cnt, sizeof(unsigned long long) * kCntTotal);
-        if (e != hipSuccess)
-            return fail(c, e == hipErrorOutOfMemory ? START_ERR_NOMEM : START_ERR_HIP,
-                        std::string("statistics buffer: ") + hipGetErrorString(e));
+    {
+        const int rc = ensure_counters(c);
+        if (rc != START_OK) return rc;
     }
     HIPCHECK(c, hipMemcpyAsync(c->h_cnt + kCntSettled, c->d_cnt + kCntSettled, sizeof(unsigned long long),
                                hipMemcpyDeviceToHost, c->stream));
@@ -2276,11 +2373,9 @@ int start_read_settled_since(start_ctx* c, int64_t first, uint64_t* ids, int64_t
 int start_read_stats(start_ctx* c, start_stats* out)
 {
     if (!c || !out) return fail(c, START_ERR_ARG, "null argument");
-    if (!c->h_cnt) {  // page-locked, so that the copy is one DMA behind the step
-        hipError_t e = host_pinned_malloc((void**)&c->h_cnt, sizeof(unsigned long long) * kCntTotal);
-        if (e != hipSuccess)
-            return fail(c, e == hipErrorOutOfMemory ? START_ERR_NOMEM : START_ERR_HIP,
-                        std::string("statistics buffer: ") + hipGetErrorString(e));
+    {
+        const int rc = ensure_counters(c);
+        if (rc != START_OK) return rc;
     }
     const unsigned long long* h = c->h_cnt;
     HIPCHECK(c, hipMemcpyAsync(c->h_cnt, c->d_cnt, sizeof(unsigned long long) * kCntTotal, hipMemcpyDeviceToHost,
@@ -2305,11 +2400,9 @@ int start_read_stats_settled(start_ctx* c, start_stats* out, int64_t first, uint
     // the counters and a window of the settle log after `first`, in one sync
     const int64_t log_len = c->n;
     const int64_t W = std::max<int64_t>(0, std::min<int64_t>({*n, (int64_t)1024, log_len - first}));
-    if (!c->h_cnt) {
-        hipError_t e = host_pinned_malloc((void**)&c->h_cnt, sizeof(unsigned long long) * kCntTotal);
-        if (e != hipSuccess)
-            return fail(c, e == hipErrorOutOfMemory ? START_ERR_NOMEM : START_ERR_HIP,
-                        std::string("statistics buffer: ") + hipGetErrorString(e));
+    {
+        const int rc = ensure_counters(c);
+        if (rc != START_OK) return rc;
     }
     if (std::max<int64_t>(W, 1) > c->h_settle_cap) {
         const int64_t cap = std::max<int64_t>(W, 4096);
@@ -2374,27 +2467,34 @@ int start_locate(start_ctx* c, int64_t n, const double* x, const double* y, cons
 {
     if (!c || n < 0 || (n > 0 && (!x || !y || !z || !out_tet))) return fail(c, START_ERR_ARG, "bad argument");
     if (n == 0) return START_OK;
-    double *dx = nullptr, *dy = nullptr, *dz = nullptr;
-    int32_t* dt = nullptr;
-    hipError_t e = dalloc(&dx, n);
-    if (e == hipSuccess) e = dalloc(&dy, n);
-    if (e == hipSuccess) e = dalloc(&dz, n);
-    if (e == hipSuccess) e = dalloc(&dt, n);
-    if (e == hipSuccess) e = hipMemcpyAsync(dx, x, sizeof(double) * n, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(dy, y, sizeof(double) * n, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(dz, z, sizeof(double) * n, hipMemcpyHostToDevice, c->stream);
+    const size_t b8 = sizeof(double) * (size_t)n, b4 = sizeof(int32_t) * (size_t)n;
+    const bool staged = 3 * b8 + b4 <= kStageBytes && have_stage(c);
+    void* own = nullptr;
+    hipError_t e = staged ? hipSuccess : dev_malloc(&own, 3 * b8 + b4);
+    double* d = staged ? (double*)c->d_stage : (double*)own;
+    int32_t* dt = (int32_t*)(d + 3 * n);
+    const double* src[3] = {x, y, z};
+    if (staged) {
+        for (int k = 0; k < 3; ++k) memcpy(c->h_stage + k * b8, src[k], b8);
+        e = hipMemcpyAsync(d, c->h_stage, 3 * b8, hipMemcpyHostToDevice, c->stream);
+    } else {
+        for (int k = 0; k < 3 && e == hipSuccess; ++k)
+            e = hipMemcpyAsync(d + k * n, src[k], b8, hipMemcpyHostToDevice, c->stream);
+    }
     if (e == hipSuccess) {
-        launch_locate(c->stream, c->mesh_view(), dx, dy, dz, n, dt, nullptr, nullptr, nullptr, nullptr, c->d_cnt);
+        launch_locate(c->stream, c->mesh_view(), d, d + n, d + 2 * n, n, dt, nullptr, nullptr, nullptr, nullptr,
+                      c->d_cnt);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(out_tet, dt, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(dx);
-    (void)hipFree(dy);
-    (void)hipFree(dz);
-    (void)hipFree(dt);
+    // (staged: behind the points in the buffer, which may still be on their way)
+    void* const out = staged ? (void*)(c->h_stage + 3 * b8) : (void*)out_tet;
+    if (e == hipSuccess) e = hipMemcpyAsync(out, dt, b4, hipMemcpyDeviceToHost, c->stream);
+    int rc = START_OK;
+    if (e == hipSuccess) rc = check_kernel_errors(c);
+    if (own) (void)hipFree(own);
     if (e != hipSuccess) return fail(c, START_ERR_HIP, std::string("locate: ") + hipGetErrorString(e));
-    return check_kernel_errors(c);
+    if (rc == START_OK && staged) memcpy(out_tet, out, b4);
+    return rc;
 }
 
 // start_locate with the points and owners staged in the file-scope `scratch`

@@ -2506,19 +2506,71 @@ __global__ void math_batch_kernel(int which, const double* __restrict__ x, const
     out2[i] = r2;
 }
 
-// absolute FP64 positions of the mixed layout, for read-back
-__global__ void abs_positions_kernel(DevMesh M, const float* __restrict__ lx, const float* __restrict__ ly,
-                                     const float* __restrict__ lz, const int32_t* __restrict__ tet, int64_t n,
-                                     double* __restrict__ x, double* __restrict__ y, double* __restrict__ z)
+// The rows of a new population besides its state: load indices, hit triangle
+// -1, and the flags of its species and run (species null: the flags are there);
+// with them the live row count and the next launch's step.
+__global__ void init_rows_kernel(int64_t first, int64_t m, const int32_t* __restrict__ species,
+                                 const RunK* __restrict__ runs, int32_t n_runs, int32_t* __restrict__ flags,
+                                 int32_t* __restrict__ hit, uint32_t* __restrict__ pidx, int64_t* __restrict__ n_active,
+                                 int64_t active, unsigned long long* __restrict__ step_cnt, unsigned long long step)
 {
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double p[3];
-    abs_pos(M, tet[i], lx[i], ly[i], lz[i], p);
-    x[i] = p[0];
-    y[i] = p[1];
-    z[i] = p[2];
+    const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (j == 0) {
+        *n_active = active;
+        *step_cnt = step;
+    }
+    if (j >= m) return;
+    const int64_t i = first + j;
+    hit[i] = -1;
+    pidx[i] = (uint32_t)i;
+    if (species) {
+        int32_t lo = 0, hi = n_runs - 1;  // the last run whose first row is not after i
+        while (lo < hi) {
+            const int32_t mid = (lo + hi + 1) / 2;
+            if ((int64_t)runs[mid].first <= i) lo = mid;
+            else hi = mid - 1;
+        }
+        flags[i] = (species[j] << kSpeciesShift) | (lo << kRunShift);
+    }
 }
+
+void launch_init_rows(hipStream_t s, int64_t first, int64_t m, const int32_t* species, const RunK* runs,
+                      int32_t n_runs, int32_t* flags, int32_t* hit, uint32_t* pidx, int64_t* n_active, int64_t active,
+                      unsigned long long* step_cnt, unsigned long long step)
+{
+    init_rows_kernel<<<(unsigned)std::max<int64_t>(1, (m + 255) / 256), 256, 0, s>>>(
+        first, m, species, runs, n_runs, flags, hit, pidx, n_active, active, step_cnt, step);
+}
+
+// The state by load index, positions absolute in FP64: the rows written
+// where they belong, so that the host only copies.  Null outputs are skipped.
+template <typename R>
+__global__ void load_order_kernel(DevMesh M, DevParticles<R> P, ReadBack out)
+{
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i >= P.n) return;
+    const uint32_t j = P.pidx[i];
+    if (out.f[0] || out.f[1] || out.f[2]) {
+        double p[3];
+        abs_pos(M, P.tet[i], P.x[i], P.y[i], P.z[i], p);
+        for (int k = 0; k < 3; ++k)
+            if (out.f[k]) out.f[k][j] = p[k];
+    }
+    if (out.f[3]) out.f[3][j] = P.vx[i];
+    if (out.f[4]) out.f[4][j] = P.vy[i];
+    if (out.f[5]) out.f[5][j] = P.vz[i];
+    if (out.tet) out.tet[j] = P.tet[i];
+    if (out.settled) out.settled[j] = (P.flags[i] & kSettled) ? 1 : 0;
+    if (out.hit) out.hit[j] = P.hit[i];
+}
+
+template <typename R>
+void launch_load_order(hipStream_t s, const DevMesh& M, const DevParticles<R>& P, const ReadBack& out)
+{
+    if (P.n > 0) load_order_kernel<R><<<(unsigned)((P.n + 255) / 256), 256, 0, s>>>(M, P, out);
+}
+template void launch_load_order<double>(hipStream_t, const DevMesh&, const DevParticles<double>&, const ReadBack&);
+template void launch_load_order<float>(hipStream_t, const DevMesh&, const DevParticles<float>&, const ReadBack&);
 
 // ---------------------------------------------------------------------------
 // Adjoint of the collisionless push and the surface-hit map.
@@ -2853,12 +2905,6 @@ void launch_math_batch(hipStream_t s, int which, const double* x, const double* 
                        double* out2)
 {
     if (n > 0) math_batch_kernel<<<blocks_for(n, 256), 256, 0, s>>>(which, x, y, n, out, out2);
-}
-
-void launch_abs_positions(hipStream_t s, const DevMesh& M, const float* lx, const float* ly, const float* lz,
-                          const int32_t* tet, int64_t n, double* x, double* y, double* z)
-{
-    if (n > 0) abs_positions_kernel<<<blocks_for(n, 256), 256, 0, s>>>(M, lx, ly, lz, tet, n, x, y, z);
 }
 
 template void launch_step<double>(hipStream_t, const DevMesh&, const DevParticles<double>&, const StepParams&,
