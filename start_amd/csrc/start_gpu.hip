@@ -56,12 +56,12 @@ void launch_init_rows(hipStream_t s, int64_t first, int64_t m, const int32_t* sp
                       unsigned long long* step_cnt, unsigned long long step);
 template <typename R>
 void launch_load_order(hipStream_t s, const DevMesh& M, const DevParticles<R>& P, const ReadBack& out);
-size_t sort_temp_bytes(int64_t n, int nbits);
+size_t sort_scratch_len(int64_t n_tets);
+size_t sort_zeroed_len(int64_t n_tets);
 template <typename R>
 hipError_t sort_particles(hipStream_t s, const DevParticles<R>& P, R* x, R* y, R* z, double* vx, double* vy, double* vz,
-                          int32_t* tet, int32_t* flags, int32_t* hit, uint32_t* pidx, int32_t* keys,
-                          int32_t* keys_out, int32_t* idx, int32_t* perm, void* temp, size_t temp_bytes,
-                          int32_t n_tets, int nbits, int64_t* n_active);
+                          int32_t* tet, int32_t* flags, int32_t* hit, uint32_t* pidx, int32_t* rank, int32_t* scratch,
+                          int32_t n_tets, int64_t* n_active);
 }  // namespace sg
 
 using namespace sg;
@@ -205,10 +205,7 @@ struct start_ctx {
     PBuf A, B;  // live arrays and the sort target
     std::vector<uint64_t> ids;
     WorkItem* d_wl = nullptr;
-    int32_t *d_keys = nullptr, *d_keys_out = nullptr, *d_idx = nullptr, *d_perm = nullptr;
-    void* d_sort_temp = nullptr;
-    size_t sort_temp = 0;
-    int sort_bits = 1;
+    int32_t *d_rank = nullptr, *d_sort = nullptr;  // sort: places among equal keys, key tables
     int64_t* d_nactive = nullptr;
     unsigned long long* d_cnt = nullptr;
     uint64_t step = 0;
@@ -380,30 +377,21 @@ void free_tracking(start_ctx* c)
 void free_work_buffers(start_ctx* c)
 {
     free_pbuf(c->B);
-    void* ptrs[] = {c->d_wl, c->d_keys, c->d_keys_out, c->d_idx, c->d_perm, c->d_sort_temp};
+    void* ptrs[] = {c->d_wl, c->d_rank, c->d_sort};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     c->d_wl = nullptr;
-    c->d_keys = c->d_keys_out = c->d_idx = c->d_perm = nullptr;
-    c->d_sort_temp = nullptr;
-    c->sort_temp = 0;
+    c->d_rank = c->d_sort = nullptr;
 }
 
 hipError_t alloc_work_buffers(start_ctx* c, int64_t cap)
 {
     hipError_t he = dalloc(&c->d_wl, cap);
     if (he == hipSuccess) he = alloc_pbuf(c->B, cap, c->es);
-    if (he == hipSuccess) he = dalloc(&c->d_keys, cap);
-    if (he == hipSuccess) he = dalloc(&c->d_keys_out, cap);
-    if (he == hipSuccess) he = dalloc(&c->d_idx, cap);
-    if (he == hipSuccess) he = dalloc(&c->d_perm, cap);
-    if (he == hipSuccess) {
-        int bits = 1;
-        while (bits < 31 && ((int64_t)1 << bits) <= c->hm.n_tets + 1) ++bits;
-        c->sort_bits = bits;
-        c->sort_temp = sort_temp_bytes(cap, bits);
-        he = dev_malloc(&c->d_sort_temp, std::max<size_t>(c->sort_temp, 16));
-    }
+    if (he == hipSuccess) he = dalloc(&c->d_rank, cap);
+    if (he == hipSuccess) he = dalloc(&c->d_sort, sort_scratch_len(c->hm.n_tets));
+    if (he == hipSuccess)
+        he = hipMemsetAsync(c->d_sort, 0, sizeof(int32_t) * sort_zeroed_len(c->hm.n_tets), c->stream);
     return he;
 }
 
@@ -421,14 +409,13 @@ void free_particles(start_ctx* c)
     c->cap = 0;
 }
 
-// radix sort by owning tet, settled particles last, then swap the buffer sets
+// sort by owning tet, settled particles last, then swap the buffer sets
 template <typename R>
 hipError_t sort_typed(start_ctx* c)
 {
     PBuf& B = c->B;
     return sort_particles<R>(c->stream, c->view<R>(), (R*)B.x, (R*)B.y, (R*)B.z, (double*)B.vx, (double*)B.vy, (double*)B.vz, B.tet,
-                             B.flags, B.hit, B.pidx, c->d_keys, c->d_keys_out, c->d_idx, c->d_perm, c->d_sort_temp,
-                             c->sort_temp, (int32_t)c->hm.n_tets, c->sort_bits, c->d_nactive);
+                             B.flags, B.hit, B.pidx, c->d_rank, c->d_sort, (int32_t)c->hm.n_tets, c->d_nactive);
 }
 
 int sort_now(start_ctx* c)
@@ -646,7 +633,7 @@ struct RowScratch {
     hipError_t get(start_ctx* c, int64_t n)
     {
         static_assert(sizeof(WorkItem) >= 5 * sizeof(double), "rows of five doubles");
-        if (c->d_sort_temp && n <= c->cap) {
+        if (c->d_sort && n <= c->cap) {
             rows = (double*)c->d_wl;
             double* v[3] = {(double*)c->B.vx, (double*)c->B.vy, (double*)c->B.vz};
             int32_t* w[3] = {c->B.tet, c->B.flags, c->B.hit};
@@ -997,7 +984,7 @@ int begin_population(start_ctx* c, const std::vector<RunK>& rk, int64_t n, const
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     // buffers that fit are kept (some 30 allocations and releases took 6 ms of
     // a load of 1M particles); far larger ones are given back
-    const bool keep = c->d_sort_temp && c->A.x && n <= c->cap && c->cap <= std::max<int64_t>(4 * n, 65536);
+    const bool keep = c->d_sort && c->A.x && n <= c->cap && c->cap <= std::max<int64_t>(4 * n, 65536);
     if (keep) {
         drop_graphs(c);
         free_tracking(c);
