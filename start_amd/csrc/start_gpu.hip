@@ -43,7 +43,8 @@ void launch_adjoint_push(hipStream_t s, const DevMesh& M, const DevParticles<R>&
 template <typename R>
 void launch_track_eligible(hipStream_t s, const DevMesh& M, const DevParticles<R>& P, const StepParams& S,
                            uint8_t* out);
-void launch_field(hipStream_t s, const DevMesh& M, const double* phi, double* E, float* E32);
+void launch_field(hipStream_t s, const DevMesh& M, const double* phi, double* E, float* E32, const double* q,
+                  const double* m, int32_t n_slots, double dt, double* H, float* H32);
 void launch_e32(hipStream_t s, const double* E, float* E32, int64_t nt);
 void launch_tet_boxes(hipStream_t s, const DevMesh& M, TetBox* box);
 void launch_push_table(hipStream_t s, const double* E, const float* E32, int64_t nt, const double* q,
@@ -720,6 +721,18 @@ int mark_present(start_ctx* c, const int32_t* species, int64_t n)
     return assign_push_slots(c);
 }
 
+// Charge and mass of the species of each push table slot.
+void push_species(const start_ctx* c, std::vector<double>& q, std::vector<double>& m)
+{
+    q.assign((size_t)c->n_push, 0.0);
+    m.assign((size_t)c->n_push, 0.0);
+    for (const auto& k : c->species)
+        if (k.push_slot >= 0) {
+            q[(size_t)k.push_slot] = k.charge;
+            m[(size_t)k.push_slot] = k.mass;
+        }
+}
+
 // The tables of the current field and time step, queued on the library's
 // stream before the next step.
 int refresh_push_tables(start_ctx* c)
@@ -727,13 +740,7 @@ int refresh_push_tables(start_ctx* c)
     if (!c->push_dirty) return START_OK;
     if (c->n_push > 0) {
         std::vector<double> q, m;
-        for (const auto& k : c->species)
-            if (k.push_slot >= 0) {
-                q.resize((size_t)std::max<int32_t>((int32_t)q.size(), k.push_slot + 1));
-                m.resize(q.size());
-                q[(size_t)k.push_slot] = k.charge;
-                m[(size_t)k.push_slot] = k.mass;
-            }
+        push_species(c, q, m);
         launch_push_table(c->stream, c->d_E, c->d_E32, c->hm.n_tets, q.data(), m.data(), c->n_push, c->prm.dt, c->d_H,
                           c->d_H32);
         HIPCHECK(c, hipGetLastError());
@@ -1750,8 +1757,11 @@ int start_set_node_potential_basis(start_ctx* c, int32_t which, const double* ph
     HIPCHECK(c, hipMemcpyAsync(c->d_phi, c->h_phi, bytes, hipMemcpyHostToDevice, c->stream));
     HIPCHECK(c, hipEventRecord(c->phi_copied, c->stream));
     c->phi_pending = true;
-    launch_field(c->stream, c->mesh_view(), c->d_phi, which ? c->d_E1 : c->d_E, which ? c->d_E1_32 : c->d_E32);
-    if (which == 0) c->push_dirty = true;
+    std::vector<double> q, m;
+    if (which == 0) push_species(c, q, m);  // with the push tables of the new field
+    launch_field(c->stream, c->mesh_view(), c->d_phi, which ? c->d_E1 : c->d_E, which ? c->d_E1_32 : c->d_E32, q.data(),
+                 m.data(), (int32_t)q.size(), c->prm.dt, c->d_H, c->d_H32);
+    if (which == 0) c->push_dirty = c->n_push == 0;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(c, START_ERR_HIP, std::string("field from potential: ") + hipGetErrorString(e));
     return START_OK;

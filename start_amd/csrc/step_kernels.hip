@@ -2370,28 +2370,6 @@ __global__ void node_density_bary_kernel(const double* __restrict__ q, const dou
     if (written) written[n] = 1;
 }
 
-// E = -grad(phi) = -sum_j (phi_j - phi_0) A_j  (A_j: gradient of lambda_j)
-__global__ void field_kernel(DevMesh M, const double* __restrict__ phi, double* __restrict__ E, float* __restrict__ E32)
-{
-    int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= M.n_tets) return;
-    int4 nv = M.tnode[t];
-    const double* g = M.geo + 12 * t;
-    double p0 = phi[nv.x], d1 = phi[nv.y] - p0, d2 = phi[nv.z] - p0, d3 = phi[nv.w] - p0;
-    double ex = -((d1 * g[3] + d2 * g[6]) + d3 * g[9]);
-    double ey = -((d1 * g[4] + d2 * g[7]) + d3 * g[10]);
-    double ez = -((d1 * g[5] + d2 * g[8]) + d3 * g[11]);
-    E[3 * t] = ex;
-    E[3 * t + 1] = ey;
-    E[3 * t + 2] = ez;
-    if (E32) {
-        E32[4 * t] = (float)ex;
-        E32[4 * t + 1] = (float)ey;
-        E32[4 * t + 2] = (float)ez;
-        E32[4 * t + 3] = 0.0f;
-    }
-}
-
 // Push increments h = (((E*q)/m)*dt)/2 of field basis 0 for each charged
 // species slot (push<R>'s arithmetic, FP64 from E and FP32 from the FP32 field),
 // -0 where push<R> returns early (dt == 0 or E == 0 exactly).
@@ -2404,36 +2382,68 @@ __device__ inline R push_increment(R e, R q, R m, R dt)
 {
     return (((e * q) / m) * dt) / R(2);
 }
-__global__ void push_table_kernel(const double* __restrict__ E, const float* __restrict__ E32, int64_t nt,
-                                  PushSlots ps, double dt, double* __restrict__ H, float* __restrict__ H32)
+__device__ inline void push_rows(const double* e, const float* e32, int64_t t, int64_t nt, const PushSlots& ps,
+                                 double dt, double* __restrict__ H, float* __restrict__ H32)
 {
-    int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= nt) return;
     for (int k = 0; k < ps.n; ++k) {
         if (H) {
-            const double ex = E[3 * t], ey = E[3 * t + 1], ez = E[3 * t + 2];
-            const bool skip = dt == 0.0 || (ex == 0.0 && ey == 0.0 && ez == 0.0);
+            const bool skip = dt == 0.0 || (e[0] == 0.0 && e[1] == 0.0 && e[2] == 0.0);
             double* h = H + 3 * ((int64_t)k * nt + t);
-            h[0] = skip ? -0.0 : push_increment<double>(ex, ps.q[k], ps.m[k], dt);
-            h[1] = skip ? -0.0 : push_increment<double>(ey, ps.q[k], ps.m[k], dt);
-            h[2] = skip ? -0.0 : push_increment<double>(ez, ps.q[k], ps.m[k], dt);
+            for (int c = 0; c < 3; ++c) h[c] = skip ? -0.0 : push_increment<double>(e[c], ps.q[k], ps.m[k], dt);
         }
         if (H32) {
-            const float ex = E32[4 * t], ey = E32[4 * t + 1], ez = E32[4 * t + 2];
             const float q = (float)ps.q[k], m = (float)ps.m[k], d = (float)dt;
-            const bool skip = d == 0.0f || (ex == 0.0f && ey == 0.0f && ez == 0.0f);
+            const bool skip = d == 0.0f || (e32[0] == 0.0f && e32[1] == 0.0f && e32[2] == 0.0f);
             float4 h;
-            h.x = skip ? -0.0f : push_increment<float>(ex, q, m, d);
-            h.y = skip ? -0.0f : push_increment<float>(ey, q, m, d);
-            h.z = skip ? -0.0f : push_increment<float>(ez, q, m, d);
+            h.x = skip ? -0.0f : push_increment<float>(e32[0], q, m, d);
+            h.y = skip ? -0.0f : push_increment<float>(e32[1], q, m, d);
+            h.z = skip ? -0.0f : push_increment<float>(e32[2], q, m, d);
             h.w = 0.0f;
             reinterpret_cast<float4*>(H32)[(int64_t)k * nt + t] = h;
         }
     }
 }
 
-void launch_push_table(hipStream_t s, const double* E, const float* E32, int64_t nt, const double* q,
-                       const double* m, int32_t n_slots, double dt, double* H, float* H32)
+// E = -grad(phi) = -sum_j (phi_j - phi_0) A_j  (A_j: gradient of lambda_j), and
+// the push increments with it (ps.n slots, 0: none) while the field is in
+// registers: FP64 bound by memory, 160 B per tet in one launch instead of 184 in
+// two.  750k tets: 17.5 + 8.0 -> 20.9 us.
+__global__ void field_kernel(DevMesh M, const double* __restrict__ phi, double* __restrict__ E, float* __restrict__ E32,
+                             PushSlots ps, double dt, double* __restrict__ H, float* __restrict__ H32)
+{
+    int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (t >= M.n_tets) return;
+    int4 nv = M.tnode[t];
+    TetMap m;
+    m.load(M, (int32_t)t);
+    const double* g = m.g;
+    double p0 = phi[nv.x], d1 = phi[nv.y] - p0, d2 = phi[nv.z] - p0, d3 = phi[nv.w] - p0;
+    double e[3];
+    float e32[3];
+    for (int c = 0; c < 3; ++c) {
+        e[c] = -((d1 * g[3 + c] + d2 * g[6 + c]) + d3 * g[9 + c]);
+        e32[c] = (float)e[c];
+        E[3 * t + c] = e[c];
+    }
+    if (E32) reinterpret_cast<float4*>(E32)[t] = make_float4(e32[0], e32[1], e32[2], 0.0f);
+    push_rows(e, e32, t, M.n_tets, ps, dt, H, H32);
+}
+
+__global__ void push_table_kernel(const double* __restrict__ E, const float* __restrict__ E32, int64_t nt,
+                                  PushSlots ps, double dt, double* __restrict__ H, float* __restrict__ H32)
+{
+    int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (t >= nt) return;
+    double e[3];
+    float e32[3];
+    for (int c = 0; c < 3; ++c) {
+        e[c] = E[3 * t + c];
+        e32[c] = E32 ? E32[4 * t + c] : 0.0f;
+    }
+    push_rows(e, e32, t, nt, ps, dt, H, H32);
+}
+
+static PushSlots push_slots(const double* q, const double* m, int32_t n_slots)
 {
     PushSlots ps{};
     ps.n = n_slots;
@@ -2441,8 +2451,15 @@ void launch_push_table(hipStream_t s, const double* E, const float* E32, int64_t
         ps.q[k] = q[k];
         ps.m[k] = m[k];
     }
+    return ps;
+}
+
+void launch_push_table(hipStream_t s, const double* E, const float* E32, int64_t nt, const double* q,
+                       const double* m, int32_t n_slots, double dt, double* H, float* H32)
+{
     if (nt > 0 && n_slots > 0)
-        push_table_kernel<<<(unsigned)((nt + 255) / 256), 256, 0, s>>>(E, E32, nt, ps, dt, H, H32);
+        push_table_kernel<<<(unsigned)((nt + 255) / 256), 256, 0, s>>>(E, E32, nt, push_slots(q, m, n_slots), dt, H,
+                                                                       H32);
 }
 
 __device__ inline float round_down(double x)
@@ -2886,9 +2903,10 @@ template void launch_node_density<float>(hipStream_t, const DevParticles<float>&
                                          const double*, const double*, const int32_t*, const int32_t*,
                                          const double*, double*, int32_t*, int64_t, double*, int32_t*);
 
-void launch_field(hipStream_t s, const DevMesh& M, const double* phi, double* E, float* E32)
+void launch_field(hipStream_t s, const DevMesh& M, const double* phi, double* E, float* E32, const double* q,
+                  const double* m, int32_t n_slots, double dt, double* H, float* H32)
 {
-    field_kernel<<<blocks_for(M.n_tets, 256), 256, 0, s>>>(M, phi, E, E32);
+    field_kernel<<<blocks_for(M.n_tets, 256), 256, 0, s>>>(M, phi, E, E32, push_slots(q, m, n_slots), dt, H, H32);
 }
 
 void launch_e32(hipStream_t s, const double* E, float* E32, int64_t nt)
