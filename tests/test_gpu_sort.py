@@ -15,7 +15,7 @@ from ._parity import Pair
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 3000])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 1024, 3000])
 @pytest.mark.parametrize("cells", [1, 8, 9])  # 6, 3,072 and 4,374 tets: one workgroup of keys and two
 @pytest.mark.parametrize("spread", ["box", "point"])
 def test_sorted_population_matches_the_oracle(n, cells, spread):
