@@ -108,6 +108,13 @@ struct DevParticles {
     int64_t n;
 };
 
+// State columns x, y, z, vx, vy, vz of rows to load: where they are and where
+// they go (source null: in place).
+struct RowColumns {
+    const double* src[6];
+    double* dst[6];
+};
+
 // Device columns of a read-back in load order (null: not wanted): x, y, z,
 // vx, vy, vz, owner, settled or not, hit triangle.
 struct ReadBack {

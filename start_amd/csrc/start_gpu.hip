@@ -52,7 +52,7 @@ void launch_push_table(hipStream_t s, const double* E, const float* E32, int64_t
 void launch_orient_batch(hipStream_t s, const double* pts, int64_t n, int32_t* out);
 void launch_math_batch(hipStream_t s, int which, const double* x, const double* y, int64_t n, double* out,
                        double* out2);
-void launch_init_rows(hipStream_t s, int64_t first, int64_t m, const int32_t* species, const RunK* runs,
+void launch_init_rows(hipStream_t s, int64_t first, int64_t m, const RowColumns& cols, const int32_t* species, const RunK* runs,
                       int32_t n_runs, int32_t* flags, int32_t* hit, uint32_t* pidx, int64_t* n_active, int64_t active,
                       unsigned long long* step_cnt, unsigned long long step);
 template <typename R>
@@ -1131,14 +1131,16 @@ int upload_rows(start_ctx* c, int64_t first, int64_t m, const double* x, const d
     double* pos[3];
     for (int k = 0; k < 3; ++k) pos[k] = c->mixed ? tmp.col[k] : dst[k] + first;
     const int32_t* d_species;
+    RowColumns cols{};
     const size_t total = 6 * b8 + sizeof(int32_t) * (size_t)m;
     if (total <= kStageBytes && have_stage(c)) {
         for (int k = 0; k < 6; ++k) memcpy(c->h_stage + k * b8, src[k], b8);
         memcpy(c->h_stage + 6 * b8, species, sizeof(int32_t) * (size_t)m);
         HIPCHECK(c, hipMemcpyAsync(c->d_stage, c->h_stage, total, hipMemcpyHostToDevice, c->stream));
-        for (int k = 0; k < 6; ++k)
-            HIPCHECK(c, hipMemcpyAsync(k < 3 ? (void*)pos[k] : (void*)(dst[k] + first), c->d_stage + k * b8, b8,
-                                       hipMemcpyDeviceToDevice, c->stream));
+        for (int k = 0; k < 6; ++k) {
+            cols.src[k] = (const double*)(c->d_stage + k * b8);
+            cols.dst[k] = k < 3 ? pos[k] : dst[k] + first;
+        }
         d_species = (const int32_t*)(c->d_stage + 6 * b8);
     } else {
         for (int k = 0; k < 6; ++k)
@@ -1148,7 +1150,7 @@ int upload_rows(start_ctx* c, int64_t first, int64_t m, const double* x, const d
                                    c->stream));
         d_species = c->A.flags + first;
     }
-    launch_init_rows(c->stream, first, m, d_species, c->d_runs, (int32_t)c->runs.size(), c->A.flags, c->A.hit,
+    launch_init_rows(c->stream, first, m, cols, d_species, c->d_runs, (int32_t)c->runs.size(), c->A.flags, c->A.hit,
                      c->A.pidx, c->d_nactive, first + m, c->d_cnt + kCntStep + c->wslot, (unsigned long long)c->step);
     launch_locate(c->stream, c->mesh_view(), pos[0], pos[1], pos[2], m, c->A.tet + first, c->A.flags + first,
                   c->mixed ? (float*)c->A.x + first : nullptr, c->mixed ? (float*)c->A.y + first : nullptr,
@@ -1581,7 +1583,7 @@ int start_generate(start_ctx* c, int32_t n_sources, const start_source_desc* src
         for (int32_t s = 0; s < n_sources; ++s)
             launch_generate(c->stream, sk[(size_t)s], (uint32_t)s, seed, d_cen, d_nor, dst[0], dst[1], dst[2],
                             dst[3], dst[4], dst[5], c->A.flags);
-        launch_init_rows(c->stream, 0, n, nullptr, c->d_runs, 1, c->A.flags, c->A.hit, c->A.pidx, c->d_nactive, n,
+        launch_init_rows(c->stream, 0, n, RowColumns{}, nullptr, c->d_runs, 1, c->A.flags, c->A.hit, c->A.pidx, c->d_nactive, n,
                          c->d_cnt + kCntStep + c->wslot, (unsigned long long)c->step);
         DevMesh M = c->mesh_view();
         if (!c->mixed) {

@@ -2525,8 +2525,9 @@ __global__ void math_batch_kernel(int which, const double* __restrict__ x, const
 
 // The rows of a new population besides its state: load indices, hit triangle
 // -1, and the flags of its species and run (species null: the flags are there);
-// with them the live row count and the next launch's step.
-__global__ void init_rows_kernel(int64_t first, int64_t m, const int32_t* __restrict__ species,
+// with them the live row count and the next launch's step, and the state from
+// the staging buffer (one launch instead of six copies of 3 us each).
+__global__ void init_rows_kernel(int64_t first, int64_t m, RowColumns cols, const int32_t* __restrict__ species,
                                  const RunK* __restrict__ runs, int32_t n_runs, int32_t* __restrict__ flags,
                                  int32_t* __restrict__ hit, uint32_t* __restrict__ pidx, int64_t* __restrict__ n_active,
                                  int64_t active, unsigned long long* __restrict__ step_cnt, unsigned long long step)
@@ -2537,6 +2538,8 @@ __global__ void init_rows_kernel(int64_t first, int64_t m, const int32_t* __rest
         *step_cnt = step;
     }
     if (j >= m) return;
+    for (int k = 0; k < 6; ++k)
+        if (cols.src[k]) cols.dst[k][j] = cols.src[k][j];
     const int64_t i = first + j;
     hit[i] = -1;
     pidx[i] = (uint32_t)i;
@@ -2551,12 +2554,12 @@ __global__ void init_rows_kernel(int64_t first, int64_t m, const int32_t* __rest
     }
 }
 
-void launch_init_rows(hipStream_t s, int64_t first, int64_t m, const int32_t* species, const RunK* runs,
+void launch_init_rows(hipStream_t s, int64_t first, int64_t m, const RowColumns& cols, const int32_t* species, const RunK* runs,
                       int32_t n_runs, int32_t* flags, int32_t* hit, uint32_t* pidx, int64_t* n_active, int64_t active,
                       unsigned long long* step_cnt, unsigned long long step)
 {
     init_rows_kernel<<<(unsigned)std::max<int64_t>(1, (m + 255) / 256), 256, 0, s>>>(
-        first, m, species, runs, n_runs, flags, hit, pidx, n_active, active, step_cnt, step);
+        first, m, cols, species, runs, n_runs, flags, hit, pidx, n_active, active, step_cnt, step);
 }
 
 // The state by load index, positions absolute in FP64: the rows written
