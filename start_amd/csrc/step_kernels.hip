@@ -2126,8 +2126,10 @@ __global__ void __launch_bounds__(64) step_resolve(DevMesh M, DevParticles<R> P,
 {
     const uint64_t nw = cnt[kCntWork + 2 * S.work_slot];
     const uint32_t step0 = (uint32_t)cnt[kCntStep + S.work_slot];
-    for (uint64_t w = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; w < nw;
-         w += (uint64_t)gridDim.x * blockDim.x) {
+    // Items go to the waves in turn: lanes of one wave wait for each other's
+    // exact work (10 us and more an item), waves do not.  16 runs of 1e4 to 4e5
+    // particles, mixed, 200 steps, 123 items: 640-860 -> 390 us.
+    for (uint64_t w = blockIdx.x + (uint64_t)gridDim.x * threadIdx.x; w < nw; w += (uint64_t)gridDim.x * blockDim.x) {
         RegSink<GlobalSink> sink{GlobalSink{node_charge}, 0.0, 0.0, 0.0, 0.0};
         WorkItem it = wl[w];
         int64_t i = it.i;
