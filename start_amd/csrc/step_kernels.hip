@@ -1443,6 +1443,33 @@ __device__ inline int move_to(const DevMesh& M, PState<R>& s, bool strict, R x1,
     return outcome;
 }
 
+// The common step of a particle strictly inside its tet (rec: the tet's
+// record), as step_tile takes it: pushed, moved and still inside, with no
+// collision to look at.  False, and nothing done, in any other case.  For the
+// straggler kernel, where a particle's steps are one serial chain: 390 -> 263
+// us for the rest of 200 steps.
+template <typename R, typename Sink>
+__device__ inline bool plain_step(const DevMesh& M, const StepParams& S, const PConst& c, uint32_t step, PState<R>& s,
+                                  const TetRec<R>& rec, Sink& sink)
+{
+    if (is_frozen(M, S, s)) return false;
+    PState<R> n = s;
+    push_in(n, rec);
+    R x1, y1, z1;
+    end_point(S, c.vid, c.key, step, n, x1, y1, z1);
+    if (S.model != 0 && may_collide<R>(variate_word(S.seed, c.key, c.vid, step), c.ca, c.cb, n.v2)) return false;
+    Lam lam;
+    rec.bary(x1, y1, z1, lam.l);
+    const double tau = tau_of<R>(M);
+    if (!(lam.l[0] > tau && lam.l[1] > tau && lam.l[2] > tau && lam.l[3] > tau)) return false;
+    s = n;
+    s.x = x1;
+    s.y = y1;
+    s.z = z1;
+    sink.add(1.0, lam.l);
+    return true;
+}
+
 // One step of one particle (ParticleDynamicsProcessor.cpp:166-199 stage order,
 // then the relocation and charge of the next gather), as the straggler kernel
 // takes it; step_tile runs the same stages with the common case first.
@@ -2161,6 +2188,14 @@ __global__ void __launch_bounds__(64) step_resolve(DevMesh M, DevParticles<R> P,
             s.set_v2();
             unsigned long long extra = 0;
             for (int ks = it.k + 1; ks < S.nsteps; ++ks) {
+                if (s.t >= 0 && (s.f & kStrict) && !S.trk_slot) {
+                    if (s.t != rec.t) rec.template load<true>(M, S, k, rk, s.t);
+                    while (ks < S.nsteps && plain_step(M, S, pc, step0 + (uint32_t)ks, s, rec, sink)) {
+                        ++ks;
+                        ++extra;
+                    }
+                    if (ks == S.nsteps) break;
+                }
                 const R px = s.x, py = s.y, pz = s.z;
                 const int32_t t_before = s.t;
                 int32_t tri = -1;
