@@ -1656,6 +1656,20 @@ __device__ __forceinline__ RareStep rare_step(const StepArgs<R>& A, uint32_t row
     return r;
 }
 
+// Mixed layout: a stored point that FP32 cannot place inside tet t, by the FP64
+// map (lam: its coordinates then).
+__device__ inline bool inside64(const DevMesh& M, int32_t t, float x, float y, float z, double* lam)
+{
+    double q[3], l[4];
+    abs_pos(M, t, x, y, z, q);
+    bary_at(M, t, q[0], q[1], q[2], l);
+    const bool in = l[0] > M.tau && l[1] > M.tau && l[2] > M.tau && l[3] > M.tau;
+    if (in)
+        for (int k = 0; k < 4; ++k) lam[k] = l[k];
+    return in;
+}
+__device__ inline bool inside64(const DevMesh&, int32_t, double, double, double, double*) { return false; }
+
 // One tile of the streaming kernel: BS consecutive particles, one per thread,
 // S.nsteps steps with the state and the owning tet's record in registers.  A
 // particle whose relocation cannot be certified stops and goes to the work
@@ -1779,12 +1793,12 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                         inside = in_bbox_at(M, S, s.t, s.x, s.y, s.z) && stays_outside(M, s, x1, y1, z1);
                     } else if (strict) {
                         // From tet to tet along the segment.  (Mixed: one hop in
-                        // FP32; further ones go through the FP64 maps of
-                        // rare_step.)
+                        // FP32, further ones through the FP64 maps.)
                         constexpr bool kFar = kWalk && std::is_same<R, double>::value;
                         int fneg = 0;
                         int f = kFar ? exit_face(tau, lam.l, [&](double* l0) { rec.bary(s.x, s.y, s.z, l0); })
                                      : (classify(lam.l, tau, fneg) == kOneFace ? fneg : (int)kNoFace);
+                        if (f < 0) inside = inside64(M, s.t, x1, y1, z1, lam.l);
                         if (f >= 0) {
                             int32_t code = (&rows->nbr.x)[f];
                             if (S.charge && charge != 0.0) sink.flush_nodes(rows->node, base, charge);
@@ -1798,7 +1812,8 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                             for (int hop = 0; code >= 0 && hop < (kFar ? 6 : 1); ++hop) {
                                 rec.template load_in<kBatch>(M, S, k, rk, code, rows);
                                 rec.bary(nx, ny, nz, lam.l);
-                                if (lam.l[0] > tau && lam.l[1] > tau && lam.l[2] > tau && lam.l[3] > tau) {
+                                if ((lam.l[0] > tau && lam.l[1] > tau && lam.l[2] > tau && lam.l[3] > tau) ||
+                                    inside64(M, code, nx, ny, nz, lam.l)) {
                                     inside = true;
                                     break;
                                 }
@@ -1816,6 +1831,40 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                             } else if (f >= 0 && code <= -2) {
                                 settles = true;  // on triangle -2 - code
                                 s.f = code;
+                            }
+                        }
+                        if constexpr (kWalk && !std::is_same<R, double>::value) {
+                            // Where steps are a tenth of a tet, half the waves
+                            // have a lane beyond two faces, and on a curved mesh
+                            // many points FP32 cannot place.  Both left to
+                            // rare_step, 16M particles on 3M tets ran at 1.15e10
+                            // particle-steps/s, so at 1.51e10 (1.67e10 with four
+                            // waves per SIMD and every case in the loop; at four
+                            // waves this loop takes scratch memory, 1.12e10).
+                            if (!inside && !settles) {
+                                if (f < 0 && S.charge && charge != 0.0) sink.flush_nodes(rows->node, base, charge);
+                                double p0[3], p1[3];
+                                abs_pos(M, s.t, s.x, s.y, s.z, p0);
+                                abs_pos(M, s.t, x1, y1, z1, p1);
+                                int32_t where = -1;
+                                const int w = walk64(M, s.t, p0, p1, where);
+                                if (w == kWalkSurface) {
+                                    settles = true;
+                                    s.f = -2 - where;
+                                } else if (w == kWalkInside) {
+                                    R nx, ny, nz;
+                                    to_frame(M, where, p1, nx, ny, nz);
+                                    rec.template load_in<kBatch>(M, S, k, rk, where, rows);
+                                    rec.bary(nx, ny, nz, lam.l);
+                                    if ((lam.l[0] > tau && lam.l[1] > tau && lam.l[2] > tau && lam.l[3] > tau) ||
+                                        inside64(M, where, nx, ny, nz, lam.l)) {
+                                        inside = true;
+                                        s.t = where;
+                                        x1 = nx;
+                                        y1 = ny;
+                                        z1 = nz;
+                                    }
+                                }
                             }
                         }
                     }
