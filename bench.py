@@ -424,13 +424,6 @@ def roofline(r, key: str):
         achieved = valu_ps * ps / dur if dur > 0 else 0.0
         out = {"bound": "valu", "achieved": round(achieved, 1), "peak": VALU_PEAK, "unit": "wave-instructions/s",
                "frac": round(achieved / VALU_PEAK, 4), "valu_per_particle_step": valu_ps, **common}
-        if key.endswith("_sweep"):
-            # the batched kernel's counted issue rate exceeds the one-wave64-
-            # instruction-per-4-cycles model (6.8e11 against 6.1e11 per second,
-            # transcendental instructions excluded), so that model does not bound
-            # it and no fraction is claimed
-            out["frac"] = None
-            out["note"] = "counted VALU issue above the wave64 4-cycle model: no fraction claimed"
         if hbm_ps is not None and dur > 0:
             out["hbm_frac_measured"] = round(hbm_ps * ps / dur / 1e9 / HBM_PEAK_GBS, 4)
     if out["frac"] is not None and out["frac"] > 1.0:

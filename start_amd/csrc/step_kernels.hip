@@ -1684,7 +1684,7 @@ __device__ inline bool inside64(const DevMesh&, int32_t, double, double, double,
 // 162k tets, mixed: 6.37 -> 3.10 ms.  Where one lane of nearly every wave
 // changes tet in every step the latency of the next record bounds it and the
 // gain is small: 4% on a run of 1M particles through a 374k-tet chamber, and
-// the launches of 4,096 waves between two plates are slower, 380 -> 477 us per
+// the launches of 4,096 waves between two plates are slower, 380 -> 450 us per
 // 50 steps, because a quarter of the waves waits for a second round.
 // 3 waves per SIMD (168 registers): 4 waves put values of the loop into
 // scratch memory (1.47 ms), 2 waves hide too little of it (1.36 ms).
@@ -2749,7 +2749,7 @@ __device__ __noinline__ Located locate_slow(const DevMesh& M, int32_t hint, doub
 // A lane per particle; latency of the few waves there are bounds it (4 waves
 // per SIMD for 262,144 particles), so a step reads memory only where the owner
 // changes, and the owner is found from barycentric maps, the exact predicates
-// out of line.  262,144 particles, 1,000 steps, 156k tets: 5.6 -> 1.9 ms
+// out of line.  262,144 particles, 1,000 steps, 203k tets: 5.6 -> 1.9 ms
 // (the predicates in every step, three divisions, fields read in every step).
 template <typename R>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) adjoint_push_kernel(DevMesh M, DevParticles<R> P,
