@@ -661,6 +661,22 @@ void load_order(start_ctx* c, const ReadBack& out)
     else launch_load_order<double>(c->stream, c->mesh_view(), c->view<double>(), out);
 }
 
+// Column `src` (rows in device order) into `dst` by load index, ordered on the
+// host: for a context that a failed growth left without device scratch.
+template <typename T, typename F>
+int host_order(start_ctx* c, T* dst, const void* src, F value)
+{
+    const size_t n = (size_t)c->n;
+    std::vector<uint32_t> pidx(n);
+    std::vector<T> tmp(n);
+    HIPCHECK(c, hipMemcpyAsync(pidx.data(), c->A.pidx, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, c->stream));
+    HIPCHECK(c, hipMemcpyAsync(tmp.data(), src, sizeof(T) * n, hipMemcpyDeviceToHost, c->stream));
+    HIPCHECK(c, hipStreamSynchronize(c->stream));
+    for (size_t j = 0; j < n; ++j) dst[pidx[j]] = value(tmp[j]);
+    return START_OK;
+}
+int32_t status_of(int32_t flags) { return (flags & kSettled) ? START_SETTLED : START_ACTIVE; }
+
 int upload_runs(start_ctx* c)
 {
     for (RunK& r : c->runs) r.log2_conc = (float)log2_factor(r.conc);
@@ -2245,9 +2261,19 @@ int start_read_particles(start_ctx* c, double* x, double* y, double* z, double* 
             }
     } else {
         hipError_t e = tmp.get(c, n);
-        if (e != hipSuccess)
+        if (e != hipSuccess && c->mixed && (x || y || z))  // absolute positions need device memory
             return fail(c, e == hipErrorOutOfMemory ? START_ERR_NOMEM : START_ERR_HIP,
                         std::string("read particles: ") + hipGetErrorString(e));
+        if (e != hipSuccess) {
+            const void* fsrc[6] = {c->A.x, c->A.y, c->A.z, c->A.vx, c->A.vy, c->A.vz};
+            const int32_t* isrc[3] = {c->A.tet, c->A.flags, c->A.hit};
+            int rc = START_OK;
+            for (int k = 0; k < 6 && rc == START_OK; ++k)
+                if (fdst[k]) rc = host_order(c, fdst[k], fsrc[k], [](double v) { return v; });
+            for (int k = 0; k < 3 && rc == START_OK; ++k)
+                if (idst[k]) rc = host_order(c, idst[k], isrc[k], [k](int32_t v) { return k == 1 ? status_of(v) : v; });
+            return rc == START_OK ? check_kernel_errors(c) : rc;
+        }
         for (int k = 0; k < 6; ++k)
             if (fdst[k]) out.f[k] = k < 3 ? tmp.rows + k * n : tmp.col[k - 3];
         for (int k = 0; k < 3; ++k)
@@ -2311,16 +2337,17 @@ int start_read_settled(start_ctx* c, uint64_t* ids, int64_t* n)
     std::vector<int32_t> settled((size_t)c->n);
     if (c->n) {
         RowScratch tmp;
-        hipError_t e = tmp.get(c, c->n);
-        if (e != hipSuccess)
-            return fail(c, e == hipErrorOutOfMemory ? START_ERR_NOMEM : START_ERR_HIP,
-                        std::string("settled ids: ") + hipGetErrorString(e));
-        ReadBack out{};
-        out.settled = tmp.word[0];
-        load_order(c, out);
-        HIPCHECK(c, hipGetLastError());
-        HIPCHECK(c, hipMemcpyAsync(settled.data(), out.settled, sizeof(int32_t) * (size_t)c->n, hipMemcpyDeviceToHost,
-                                   c->stream));
+        if (tmp.get(c, c->n) == hipSuccess) {
+            ReadBack out{};
+            out.settled = tmp.word[0];
+            load_order(c, out);
+            HIPCHECK(c, hipGetLastError());
+            HIPCHECK(c, hipMemcpyAsync(settled.data(), out.settled, sizeof(int32_t) * (size_t)c->n,
+                                       hipMemcpyDeviceToHost, c->stream));
+        } else {
+            const int rc = host_order(c, settled.data(), c->A.flags, status_of);
+            if (rc != START_OK) return rc;
+        }
     }
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     int64_t cap = *n, k = 0;
