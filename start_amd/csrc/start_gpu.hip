@@ -288,10 +288,14 @@ struct start_ctx {
 
 namespace {
 
+// Every error return ends here.  One that may have left work queued waits for
+// it, so that neither the staging buffers nor the caller's arrays are still in
+// use when it returns.
 int fail(start_ctx* c, int code, const std::string& msg)
 {
     if (c) c->err = msg;
     else g_create_error = msg;
+    if (c && c->stream && code != START_ERR_ARG && code != START_ERR_STATE) (void)hipStreamSynchronize(c->stream);
     return code;
 }
 

@@ -2143,7 +2143,8 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kWindow
             cnt[kCntTile + (1 - S.work_slot)] = 0ull;
         }
     }
-    const int64_t n_active = *S.n_active;
+    // (an append that failed half-way can leave the count ahead of the rows)
+    const int64_t n_active = min(*S.n_active, A.P.n);
     if (!kPersistent) {
         if ((int64_t)blockIdx.x * BS < n_active)  // else the whole block is past the live particles
         {
