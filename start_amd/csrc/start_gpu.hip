@@ -769,6 +769,29 @@ int refresh_push_tables(start_ctx* c)
     return START_OK;
 }
 
+// The second field basis (zero until it is set): both tables or neither.
+int ensure_second_basis(start_ctx* c)
+{
+    if (c->d_E1) return START_OK;
+    const int64_t T = c->hm.n_tets;
+    double* E = nullptr;
+    float* E32 = nullptr;
+    HIPCHECK(c, hipStreamSynchronize(c->stream));
+    hipError_t e = dalloc(&E, 3 * T);
+    if (e == hipSuccess) e = hipMemsetAsync(E, 0, sizeof(double) * 3 * (size_t)T, c->stream);
+    if (e == hipSuccess && c->mixed) e = dalloc(&E32, 4 * T);
+    if (e == hipSuccess && c->mixed) e = hipMemsetAsync(E32, 0, sizeof(float) * 4 * (size_t)T, c->stream);
+    if (e != hipSuccess) {
+        if (E) (void)hipFree(E);
+        if (E32) (void)hipFree(E32);
+        return fail(c, START_ERR_HIP, std::string("second field basis: ") + hipGetErrorString(e));
+    }
+    c->d_E1 = E;
+    c->d_E1_32 = E32;
+    drop_graphs(c);
+    return START_OK;
+}
+
 // Per-run output buffers: node charge (two sets) and triangle counters.
 int alloc_run_outputs(start_ctx* c)
 {
@@ -1721,11 +1744,9 @@ int start_set_tet_field_basis(start_ctx* c, int32_t which, const double* E)
     if (!c || !E) return fail(c, START_ERR_ARG, "null argument");
     if (which != 0 && which != 1) return fail(c, START_ERR_ARG, "field basis must be 0 or 1");
     const int64_t T = c->hm.n_tets;
-    if (which == 1 && !c->d_E1) {
-        HIPCHECK(c, hipStreamSynchronize(c->stream));
-        HIPCHECK(c, dalloc(&c->d_E1, 3 * T));
-        if (c->mixed) HIPCHECK(c, dalloc(&c->d_E1_32, 4 * T));
-        drop_graphs(c);
+    if (which == 1) {
+        const int rc = ensure_second_basis(c);
+        if (rc != START_OK) return rc;
     }
     double* dE = which ? c->d_E1 : c->d_E;
     float* dE32 = which ? c->d_E1_32 : c->d_E32;
@@ -1754,23 +1775,18 @@ int start_set_node_potential_basis(start_ctx* c, int32_t which, const double* ph
 {
     if (!c || !phi) return fail(c, START_ERR_ARG, "null argument");
     if (which != 0 && which != 1) return fail(c, START_ERR_ARG, "field basis must be 0 or 1");
-    const int64_t T = c->hm.n_tets;
-    if (which == 1 && !c->d_E1) {
-        HIPCHECK(c, hipStreamSynchronize(c->stream));
-        HIPCHECK(c, dalloc(&c->d_E1, 3 * T));
-        if (c->mixed) HIPCHECK(c, dalloc(&c->d_E1_32, 4 * T));
-        drop_graphs(c);
+    if (which == 1) {
+        const int rc = ensure_second_basis(c);
+        if (rc != START_OK) return rc;
     }
     // Stream-ordered and asynchronous: launches already queued use the field
     // they were queued with, later ones the new one.  The caller's array is
     // copied into pinned staging before the call returns; the only wait is for
     // the previous call's copy out of that staging buffer.
     const size_t bytes = sizeof(double) * (size_t)c->hm.n_nodes;
-    if (!c->d_phi) {
-        HIPCHECK(c, dalloc(&c->d_phi, c->hm.n_nodes));
-        HIPCHECK(c, host_pinned_malloc((void**)&c->h_phi, std::max<size_t>(bytes, 8)));
-        HIPCHECK(c, hipEventCreateWithFlags(&c->phi_copied, hipEventDisableTiming));
-    }
+    if (!c->d_phi) HIPCHECK(c, dalloc(&c->d_phi, c->hm.n_nodes));
+    if (!c->h_phi) HIPCHECK(c, host_pinned_malloc((void**)&c->h_phi, std::max<size_t>(bytes, 8)));
+    if (!c->phi_copied) HIPCHECK(c, hipEventCreateWithFlags(&c->phi_copied, hipEventDisableTiming));
     if (c->phi_pending) {
         HIPCHECK(c, hipEventSynchronize(c->phi_copied));
         c->phi_pending = false;
@@ -1783,8 +1799,8 @@ int start_set_node_potential_basis(start_ctx* c, int32_t which, const double* ph
     if (which == 0) push_species(c, q, m);  // with the push tables of the new field
     launch_field(c->stream, c->mesh_view(), c->d_phi, which ? c->d_E1 : c->d_E, which ? c->d_E1_32 : c->d_E32, q.data(),
                  m.data(), (int32_t)q.size(), c->prm.dt, c->d_H, c->d_H32);
-    if (which == 0) c->push_dirty = c->n_push == 0;
     hipError_t e = hipGetLastError();
+    if (which == 0) c->push_dirty = e != hipSuccess || c->n_push == 0;
     if (e != hipSuccess) return fail(c, START_ERR_HIP, std::string("field from potential: ") + hipGetErrorString(e));
     return START_OK;
 }

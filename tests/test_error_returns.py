@@ -31,6 +31,8 @@ CALLS = {
     "hits": lambda e, w, k: e.hits(),
     "adjoint": lambda e, w, k: e.adjoint_push(np.ones((e.n, 3))),
     "stats": lambda e, w, k: e.stats(),
+    "potential": lambda e, w, k: e.set_node_potential(w.phi + k),
+    "basis": lambda e, w, k: e.set_field_basis(1, phi=w.phi + k),
     "track": lambda e, w, k: e.track_movements(50, 8),
 }
 
