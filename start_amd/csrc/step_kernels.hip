@@ -1776,9 +1776,14 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
         // coordinates of the end point above tau; their sum of magnitudes is
         // then 1) with no collision to look at.  The loop is uniform and the
         // common case touches no memory, so the state and the tet's record
-        // stay in registers.  A lane that crosses into a tet where it is
-        // certified, meets a surface or flies on outside the mesh is handled
+        // stay in registers.  A lane that collides, crosses into a tet where it
+        // is certified, meets a surface or flies on outside the mesh is handled
         // in place; a step with any other case in any lane leaves the loop.
+        // Collisions in place matter in longer steps: at dt 5e-8 and 0.3 Pa a
+        // third of the waves has one in every step, and sent through memory
+        // they took 16M particles on 3M tets to 1.54e10 particle-steps/s
+        // mixed, 2.29e10 FP64, against 1.75e10 and 2.64e10 here (1.71e10 and
+        // 2.00e10 with four waves per SIMD and every case in the loop).
         bool rare;
         for (;;) {
             const uint32_t step = step0 + (uint32_t)ks;
@@ -1794,7 +1799,10 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
             Lam lam;
             rec.bary(x1, y1, z1, lam.l);
             bool inside = strict && lam.l[0] > tau && lam.l[1] > tau && lam.l[2] > tau && lam.l[3] > tau;
-            rare = rare || draw;
+            if (__ballot(alive && draw && !rare) != 0) {
+                // (a degenerate segment ends before the collision, :188-190)
+                if (alive && draw && !rare && !(x1 == s.x && y1 == s.y && z1 == s.z)) collide(S, pc, step, n);
+            }
             bool settles = false;
             if (__ballot(alive && (rare || !inside)) != 0) {
                 if (alive && !rare && !inside) {
@@ -1847,9 +1855,8 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                             // have a lane beyond two faces, and on a curved mesh
                             // many points FP32 cannot place.  Both left to
                             // rare_step, 16M particles on 3M tets ran at 1.15e10
-                            // particle-steps/s, so at 1.51e10 (1.67e10 with four
-                            // waves per SIMD and every case in the loop; at four
-                            // waves this loop takes scratch memory, 1.12e10).
+                            // particle-steps/s, so at 1.54e10 (collisions still
+                            // in rare_step in both).
                             if (!inside && !settles) {
                                 if (f < 0 && S.charge && charge != 0.0) sink.flush_nodes(rows->node, base, charge);
                                 double p0[3], p1[3];
