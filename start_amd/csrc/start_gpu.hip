@@ -47,7 +47,7 @@ void launch_field(hipStream_t s, const DevMesh& M, const double* phi, double* E,
                   const double* m, int32_t n_slots, double dt, double* H, float* H32);
 void launch_e32(hipStream_t s, const double* E, float* E32, int64_t nt);
 void launch_tet_boxes(hipStream_t s, const DevMesh& M, TetBox* box);
-void launch_push_table(hipStream_t s, const double* E, const float* E32, int64_t nt, const double* q,
+void launch_push_table(hipStream_t s, const DevMesh& M, const RunK* run, bool scaled, const double* q,
                        const double* m, int32_t n_slots, double dt, double* H, float* H32);
 void launch_orient_batch(hipStream_t s, const double* pts, int64_t n, int32_t* out);
 void launch_math_batch(hipStream_t s, int which, const double* x, const double* y, int64_t n, double* out,
@@ -280,9 +280,21 @@ struct start_ctx {
         L.block = cfg.block == 128 && !L.walk ? 128 : 256;
         L.persistent = cfg.persistent ? 1 : 0;
         L.grid = n_cu * (1024 / L.block);  // 4 waves per SIMD x 4 SIMDs per CU
-        // per-lane run parameters unless the field is E_0 as given
-        L.batch = (runs.size() > 1 || d_E1 || runs[0].s0 != 1.0 || runs[0].s1 != 0.0) ? 1 : 0;
+        // per-lane run parameters for several runs; a single run whose field is
+        // not E_0 as given takes its increments from the push tables if every
+        // species of it has one.  Plates, 262,144 particles, 1,000 steps of
+        // s0 E_0 + s1 E_1: 4.95 -> 4.16 ms (no field of either basis, no run
+        // record and no division where a lane changes tet).
+        L.batch = runs.size() > 1 || (scaled_field() && !all_in_tables()) ? 1 : 0;
         return L;
+    }
+    // the field of a single run is not basis 0 as given
+    bool scaled_field() const { return runs.size() == 1 && (d_E1 || runs[0].s0 != 1.0 || runs[0].s1 != 0.0); }
+    bool all_in_tables() const
+    {
+        for (size_t s = 0; s < present.size(); ++s)
+            if (present[s] && species[s].push_slot < 0) return false;
+        return true;
     }
 };
 
@@ -761,8 +773,8 @@ int refresh_push_tables(start_ctx* c)
     if (c->n_push > 0) {
         std::vector<double> q, m;
         push_species(c, q, m);
-        launch_push_table(c->stream, c->d_E, c->d_E32, c->hm.n_tets, q.data(), m.data(), c->n_push, c->prm.dt, c->d_H,
-                          c->d_H32);
+        launch_push_table(c->stream, c->mesh_view(), c->d_runs, c->scaled_field(), q.data(), m.data(), c->n_push,
+                          c->prm.dt, c->d_H, c->d_H32);
         HIPCHECK(c, hipGetLastError());
     }
     c->push_dirty = false;
@@ -788,6 +800,7 @@ int ensure_second_basis(start_ctx* c)
     }
     c->d_E1 = E;
     c->d_E1_32 = E32;
+    c->push_dirty = true;
     drop_graphs(c);
     return START_OK;
 }
@@ -1046,7 +1059,9 @@ int begin_population(start_ctx* c, const std::vector<RunK>& rk, int64_t n, const
     } else {
         free_particles(c);
     }
+    c->push_dirty = c->push_dirty || c->scaled_field();
     c->runs = rk;
+    c->push_dirty = c->push_dirty || c->scaled_field();
     int rc = upload_runs(c);
     if (rc != START_OK) return rc;
     rc = alloc_run_outputs(c);
@@ -1752,7 +1767,7 @@ int start_set_tet_field_basis(start_ctx* c, int32_t which, const double* E)
     float* dE32 = which ? c->d_E1_32 : c->d_E32;
     HIPCHECK(c, hipMemcpyAsync(dE, E, sizeof(double) * 3 * T, hipMemcpyHostToDevice, c->stream));
     if (dE32) launch_e32(c->stream, dE, dE32, T);
-    if (which == 0) c->push_dirty = true;
+    if (which == 0 || c->scaled_field()) c->push_dirty = true;
     HIPCHECK(c, hipGetLastError());
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     return START_OK;
@@ -1796,11 +1811,12 @@ int start_set_node_potential_basis(start_ctx* c, int32_t which, const double* ph
     HIPCHECK(c, hipEventRecord(c->phi_copied, c->stream));
     c->phi_pending = true;
     std::vector<double> q, m;
-    if (which == 0) push_species(c, q, m);  // with the push tables of the new field
+    const bool tables = which == 0 && !c->scaled_field();  // with the push tables of the new field
+    if (tables) push_species(c, q, m);
     launch_field(c->stream, c->mesh_view(), c->d_phi, which ? c->d_E1 : c->d_E, which ? c->d_E1_32 : c->d_E32, q.data(),
                  m.data(), (int32_t)q.size(), c->prm.dt, c->d_H, c->d_H32);
     hipError_t e = hipGetLastError();
-    if (which == 0) c->push_dirty = e != hipSuccess || c->n_push == 0;
+    c->push_dirty = tables ? e != hipSuccess || c->n_push == 0 : c->push_dirty || c->scaled_field();
     if (e != hipSuccess) return fail(c, START_ERR_HIP, std::string("field from potential: ") + hipGetErrorString(e));
     return START_OK;
 }

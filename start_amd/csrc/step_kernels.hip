@@ -2536,18 +2536,22 @@ __global__ void field_kernel(DevMesh M, const double* __restrict__ phi, double* 
     push_rows(e, e32, t, M.n_tets, ps, dt, H, H32);
 }
 
-__global__ void push_table_kernel(const double* __restrict__ E, const float* __restrict__ E32, int64_t nt,
-                                  PushSlots ps, double dt, double* __restrict__ H, float* __restrict__ H32)
+// The increments of run 0's field, with run_field's operations where it is not
+// basis 0 as given.
+__global__ void push_table_kernel(DevMesh M, const RunK* __restrict__ run, int32_t scaled, PushSlots ps, double dt,
+                                  double* __restrict__ H, float* __restrict__ H32)
 {
     int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= nt) return;
+    if (t >= M.n_tets) return;
     double e[3];
-    float e32[3];
-    for (int c = 0; c < 3; ++c) {
-        e[c] = E[3 * t + c];
-        e32[c] = E32 ? E32[4 * t + c] : 0.0f;
+    float e32[3] = {0.0f, 0.0f, 0.0f};
+    if (scaled) run_field<double, true>(M, run, (int32_t)t, e[0], e[1], e[2]);
+    else run_field<double, false>(M, run, (int32_t)t, e[0], e[1], e[2]);
+    if (H32) {
+        if (scaled) run_field<float, true>(M, run, (int32_t)t, e32[0], e32[1], e32[2]);
+        else run_field<float, false>(M, run, (int32_t)t, e32[0], e32[1], e32[2]);
     }
-    push_rows(e, e32, t, nt, ps, dt, H, H32);
+    push_rows(e, e32, t, M.n_tets, ps, dt, H, H32);
 }
 
 static PushSlots push_slots(const double* q, const double* m, int32_t n_slots)
@@ -2561,12 +2565,12 @@ static PushSlots push_slots(const double* q, const double* m, int32_t n_slots)
     return ps;
 }
 
-void launch_push_table(hipStream_t s, const double* E, const float* E32, int64_t nt, const double* q,
+void launch_push_table(hipStream_t s, const DevMesh& M, const RunK* run, bool scaled, const double* q,
                        const double* m, int32_t n_slots, double dt, double* H, float* H32)
 {
-    if (nt > 0 && n_slots > 0)
-        push_table_kernel<<<(unsigned)((nt + 255) / 256), 256, 0, s>>>(E, E32, nt, push_slots(q, m, n_slots), dt, H,
-                                                                       H32);
+    if (M.n_tets > 0 && n_slots > 0)
+        push_table_kernel<<<(unsigned)((M.n_tets + 255) / 256), 256, 0, s>>>(M, run, scaled ? 1 : 0,
+                                                                             push_slots(q, m, n_slots), dt, H, H32);
 }
 
 __device__ inline float round_down(double x)
