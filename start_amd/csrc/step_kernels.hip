@@ -1601,7 +1601,7 @@ struct RareStep {
 // own values went to scratch memory, which is 100 MB over the chip and misses
 // the L2: up to 11 ms for 200 steps of 1M particles.  Called out of line
 // it was slower too, for the calling convention's saves.)
-template <typename R, bool kBatch, bool kWalk, bool kTrack>
+template <typename R, bool kBatch, bool kWalk, bool kTrack, bool kPlain>
 __device__ __forceinline__ RareStep rare_step(const StepArgs<R>& A, uint32_t row, uint32_t step, int32_t ks, int32_t remaining,
                                            bool go)
 {
@@ -1646,7 +1646,7 @@ __device__ __forceinline__ RareStep rare_step(const StepArgs<R>& A, uint32_t row
     }
     if (kTrack) track_start<R>(M, S, li, t_before, px, py, pz);
     if (!(x1 == px && y1 == py && z1 == pz)) {  // (a degenerate segment ends here, :188-190)
-        if (S.model != 0 && may_collide<R>(variate_word(S.seed, c.key, c.vid, step), c.ca, c.cb, s.v2))
+        if (!kPlain && S.model != 0 && may_collide<R>(variate_word(S.seed, c.key, c.vid, step), c.ca, c.cb, s.v2))
             collide(S, c, step, s);
         r.outcome = move_to<R, kWalk>(M, s, (s.f & kStrict) != 0, x1, y1, z1, r.lam, hit_tri);
     }
@@ -1692,21 +1692,26 @@ __device__ inline bool inside64(const DevMesh&, int32_t, double, double, double,
 // read-back, FP64: 3.31 -> 1.17 ms; of 16 runs of 1e4 to 4e5 particles on
 // 162k tets, mixed: 6.37 -> 3.10 ms.  Where one lane of nearly every wave
 // changes tet in every step the latency of the next record bounds it and the
-// gain is small: 4% on a run of 1M particles through a 374k-tet chamber, and
-// the launches of 4,096 waves between two plates are slower, 380 -> 450 us per
-// 50 steps, because a quarter of the waves waits for a second round.
+// gain is smaller: 16M particles on 3M tets, 10 steps, FP64 6.2 -> 4.5 ms,
+// mixed 7.3 -> 7.1 ms.
 // 3 waves per SIMD (168 registers): 4 waves put values of the loop into
 // scratch memory (1.47 ms), 2 waves hide too little of it (1.36 ms).
-template <typename R, int BS, int HashBits, bool kBatch, bool kWalk, bool kTrack>
+// kPlain: neither charge nor gas, without the charge sums, the hash and the
+// collision test in the loop's registers.  Ions between plates, where lanes
+// change tet all the time, 1,000 steps in launches of 50: 131,072 particles
+// 2,750 -> 2,210 us, 262,144 (4,096 waves, a quarter of which waits for a
+// second round) 4,150 -> 3,590 us; at 4 waves per SIMD 3,780 us.
+template <typename R, int BS, int HashBits, bool kBatch, bool kWalk, bool kTrack, bool kPlain>
 __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, int64_t n_active, uint32_t step0,
                                           unsigned int* blk_processed, int32_t* hk, double* hv, TetRows* s_rows)
 {
     constexpr int kSlots = 1 << HashBits;
     const DevMesh& M = A.M;
     const StepParams& S = A.S;
+    const bool has_charge = !kPlain && S.charge;
     const DevParticles<R>& P = A.P;
     if (threadIdx.x == 0) *blk_processed = 0u;
-    if (S.charge) {
+    if (has_charge) {
         for (int h = threadIdx.x; h < kSlots; h += BS) {
             hk[h] = -1;
             hv[h] = 0.0;
@@ -1794,7 +1799,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
             R x1, y1, z1;
             push_in(n, rec);
             end_point(S, pc.vid, pc.key, step, n, x1, y1, z1);
-            bool draw = S.model != 0;
+            bool draw = !kPlain && S.model != 0;
             if (draw) draw = may_collide<R>(variate_word(S.seed, pc.key, pc.vid, step), pc.ca, pc.cb, n.v2);
             Lam lam;
             rec.bary(x1, y1, z1, lam.l);
@@ -1818,7 +1823,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                         if (f < 0) inside = inside64(M, s.t, x1, y1, z1, lam.l);
                         if (f >= 0) {
                             int32_t code = (&rows->nbr.x)[f];
-                            if (S.charge && charge != 0.0) sink.flush_nodes(rows->node, base, charge);
+                            if (has_charge && charge != 0.0) sink.flush_nodes(rows->node, base, charge);
                             R nx = x1, ny = y1, nz = z1;
                             if constexpr (!std::is_same<R, double>::value) {
                                 double p1[3];
@@ -1858,7 +1863,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                             // particle-steps/s, so at 1.54e10 (collisions still
                             // in rare_step in both).
                             if (!inside && !settles) {
-                                if (f < 0 && S.charge && charge != 0.0) sink.flush_nodes(rows->node, base, charge);
+                                if (f < 0 && has_charge && charge != 0.0) sink.flush_nodes(rows->node, base, charge);
                                 double p0[3], p1[3];
                                 abs_pos(M, s.t, s.x, s.y, s.z, p0);
                                 abs_pos(M, s.t, x1, y1, z1, p1);
@@ -1916,10 +1921,12 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                 s.vy = n.vy;
                 s.vz = n.vz;
                 s.v2 = n.v2;
-                sink.a0 += lam.l[0];
-                sink.a1 += lam.l[1];
-                sink.a2 += lam.l[2];
-                sink.a3 += lam.l[3];
+                if (!kPlain) {
+                    sink.a0 += lam.l[0];
+                    sink.a1 += lam.l[1];
+                    sink.a2 += lam.l[2];
+                    sink.a3 += lam.l[3];
+                }
             }
             rare = rare && alive;
             if (__ballot(rare) != 0) break;
@@ -1930,17 +1937,17 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
         // lane's state goes through memory.
         if (alive) write_state();
         const int32_t t_before = s.t;
-        const RareStep r = rare_step<R, kBatch, kWalk, kTrack>(
+        const RareStep r = rare_step<R, kBatch, kWalk, kTrack, kPlain>(
             A, (uint32_t)(i0 + tid), step0 + (uint32_t)ks, ks,
             nsteps - ks, rare);
         asm volatile("" ::: "memory");
         if (rare) {
             const bool done = r.outcome != kDone;
-            if (S.charge && t_before >= 0 && (done || r.t != t_before)) {
+            if (has_charge && t_before >= 0 && (done || r.t != t_before)) {
                 if (r.outcome == kFrozenNow) sink.add((double)r.weight, r.lam.l);
                 sink.flush(M, t_before, base, charge);
             }
-            if (!done) sink.add((double)r.weight, r.lam.l);
+            if (!kPlain && !done) sink.add((double)r.weight, r.lam.l);
             if (done) {
                 const unsigned int taken = (unsigned int)ks + (r.outcome == kFrozenNow ? 0u : 1u);
                 if (taken) atomicAdd(blk_processed, taken);
@@ -1956,14 +1963,14 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
     }
     if (alive) write_state();
     if (!alive) sink.a0 = sink.a1 = sink.a2 = sink.a3 = 0.0;  // flushed when it stopped
-    if (S.charge) sink.flush_wave(M, s.t, base, charge);  // every lane is active here
+    if (has_charge) sink.flush_wave(M, s.t, base, charge);  // every lane is active here
     // processed particle-steps: LDS per block, one atomic per tile spread over slots
     const unsigned long long am = __ballot(alive);
     if ((threadIdx.x & 63) == 0 && am) atomicAdd(blk_processed, (unsigned int)__popcll(am) * (unsigned int)nsteps);
     __syncthreads();
     if (threadIdx.x == 0 && *blk_processed)
         atomicAdd(&A.cnt[kCntProcSlot0 + (tile & (kProcSlots - 1))], (unsigned long long)*blk_processed);
-    if (S.charge) {
+    if (has_charge) {
         for (int h = threadIdx.x; h < kSlots; h += BS) {
             int32_t node = hk[h];
             if (node >= 0) global_add_f64(&A.node_charge[node], hv[h]);
@@ -2115,7 +2122,8 @@ __device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, 
 // prefix is covered (one launch for every run of a batch, whatever their
 // sizes).  The charge of a tile is summed in LDS (node window and hash) and
 // flushed with one FP64 atomic per distinct node.
-template <typename R, int BS, bool kBatch, bool kPersistent, bool kWalk, bool kTrack = false, bool kWindow = false>
+template <typename R, int BS, bool kBatch, bool kPersistent, bool kWalk, bool kTrack = false, bool kWindow = false,
+          bool kPlain = false>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kWindow ? 4 : 3))) step_main(StepArgs<R> A)
 {
     const StepParams& S = A.S;
@@ -2159,8 +2167,8 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kWindow
                 single_tile<R, BS, kBits, kWin, kWalk>(A, blockIdx.x, n_active, step0, &blk_processed, hk, hv, wv,
                                                        &s_wbase);
             else
-                step_tile<R, BS, kBits, kBatch, kWalk, kTrack>(A, blockIdx.x, n_active, step0, &blk_processed, hk, hv,
-                                                               s_rows);
+                step_tile<R, BS, kBits, kBatch, kWalk, kTrack, kPlain>(A, blockIdx.x, n_active, step0, &blk_processed,
+                                                                       hk, hv, s_rows);
         }
         return;
     }
@@ -2169,7 +2177,8 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kWindow
         __syncthreads();
         const int64_t tile = s_tile;
         if (tile * BS >= n_active) break;  // queue drained: every workgroup exits here
-        step_tile<R, BS, kBits, kBatch, kWalk, kTrack>(A, tile, n_active, step0, &blk_processed, hk, hv, s_rows);
+        step_tile<R, BS, kBits, kBatch, kWalk, kTrack, kPlain>(A, tile, n_active, step0, &blk_processed, hk, hv,
+                                                               s_rows);
     }
 }
 
@@ -2896,6 +2905,14 @@ void launch_step(hipStream_t s, const DevMesh& M, const DevParticles<R>& P, cons
         else
             step_main<R, 256, false, false, false, false, true>
                 <<<grid, 256, 0, s>>>(A);
+    } else if (P.n > 0 && !S.charge && S.model == 0 && L.walk && !L.persistent) {
+        // neither charge nor gas (electrode optimisation and its adjoint, in
+        // its own launch shape): see step_tile
+        const unsigned grid = blocks_for(P.n, 256);
+        if (L.batch)
+            step_main<R, 256, true, false, true, false, false, true><<<grid, 256, 0, s>>>(A);
+        else
+            step_main<R, 256, false, false, true, false, false, true><<<grid, 256, 0, s>>>(A);
     } else if (P.n > 0) {
         const unsigned grid = L.persistent ? (unsigned)L.grid : blocks_for(P.n, L.block == 128 ? 128 : 256);
         // the multi-tet walk is instantiated for 256-thread workgroups only
