@@ -7,12 +7,15 @@
 // the step kernels then only cover the live prefix (n_active).
 //
 // The keys are small integers, so a counting sort places every row with one
-// count per key instead of sorting (key, index) pairs: rank (each row's place
-// among those of its key), the key counts' prefix sums, one scatter of every
-// array.  Four launches, bound by the scatter's memory traffic; a radix sort
-// of the pairs took some 20 passes of 6 us each.  With one sort each, 200
-// fused steps of 1M particles on 750k tets went from 1.17 to 1.09 ms, 100 steps
-// of 150,001 particles on 179k tets from 274 to 233 us.
+// count per key: rank (each row's place among those of its key), the key
+// counts' prefix sums, one scatter of every array.  Four launches, bound by the
+// scatter's memory traffic and, where rows are in no order, by the atomics of
+// the ranks; a library radix sort of (key, row) pairs took some 20 passes of
+// 6 us each.  With one sort each, 200 fused steps of 1M particles on 750k tets
+// went from 1.17 to 1.09 ms, 100 steps of 150,001 particles on 179k tets from
+// 274 to 233 us.
+// Populations of kRadixRows and more are radix sorted instead (below): their
+// ranks' atomics and scattered stores cost more than its passes.
 // The order of the rows of one key is not fixed (nothing depends on it but
 // the order in which charges are added).
 #include "kernels.h"
@@ -174,6 +177,263 @@ __global__ void place_kernel(DevParticles<R> src, R* __restrict__ x, R* __restri
     pidx[j] = src.pidx[s];
 }
 
+// ---------------------------------------------------------------------------
+// Large populations: radix sort of (key, row) by 11 bits a pass, two passes for
+// up to 4M tets, then a gather.  Five short launches a pass; the gather's random
+// reads bound it.  A sort in us, FP64, by a library radix sort and gather, by the
+// counting sort, by this one:
+//   rows on tets          unordered              nearly ordered
+//   1M on 374k        324    294    241      220    125    159
+//   2M on 3M          454    578    448      270    300    264
+//   2M on 750k        479    562    473      164     75    139
+//   8M on 3M        1,737  2,119  1,705    1,010  1,230    976
+//   8M on 750k      1,788  2,288  1,781      455    335    365
+//   16M on 3M       3,510  5,030  3,412    2,070  2,350  1,948
+//   24.6M on 750k   6,287  9,109  6,192    1,350  1,100  1,040
+// (nearly ordered: on 3M and 374k tets particles cross some two tets between
+// sorts, on 750k few do).  From 1.5M rows on it is never slower than the
+// library's, which the counting sort is where rows move; below, the counting
+// sort's four launches are.
+// ---------------------------------------------------------------------------
+constexpr int64_t kRadixRows = 1'500'000;
+constexpr int kDigitBits = 11, kDigits = 1 << kDigitBits;
+constexpr int kTileThreads = 1024, kTileWaves = kTileThreads / 64, kTileSteps = 8;
+constexpr int kTileRows = kTileThreads * kTileSteps;
+constexpr int kChunks = 32;  // of the tiles, for the prefix sums
+
+// The (key, row) pairs of a workgroup's tile: the rows as they are in the first
+// pass.  Wave w holds rows w * 512.. of it, 64 at a time: rows ascend with
+// (wave, step, lane).  Rows past the end repeat the last one.
+struct RadixIn {
+    const int32_t *tet, *flags;
+    const int2* pairs;
+    int64_t n;
+    int32_t n_tets, shift;
+    __device__ inline int32_t digit(int32_t key) const { return key >> shift & (kDigits - 1); }
+};
+template <bool kFirst>
+struct RadixTile {
+    int64_t first;
+    int rows;  // of the tile
+    int2 pair[kTileSteps];
+    __device__ inline int row(int step) const
+    {
+        return (threadIdx.x >> 6) * (64 * kTileSteps) + step * 64 + (threadIdx.x & 63);
+    }
+    __device__ inline void load(const RadixIn& in)
+    {
+        first = blockIdx.x * (int64_t)kTileRows;
+        rows = (int)min((int64_t)kTileRows, in.n - first);
+#pragma unroll
+        for (int i = 0; i < kTileSteps; ++i) {
+            const unsigned r = (unsigned)min(row(i), rows - 1);
+            pair[i] = kFirst ? make_int2(key_of((in.tet + first)[r], (in.flags + first)[r], in.n_tets), (int)(first + r))
+                             : (in.pairs + first)[r];
+        }
+    }
+};
+
+// rows per (tile, digit), and the settled rows per tile
+template <bool kFirst>
+__global__ void __launch_bounds__(kTileThreads, 8) radix_count_kernel(RadixIn in, int32_t* __restrict__ hist,
+                                                                      int32_t* __restrict__ settled)
+{
+    __shared__ int32_t count[kDigits];
+    RadixTile<kFirst> tile;
+    tile.load(in);
+    for (int d = threadIdx.x; d < kDigits; d += kTileThreads) count[d] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kTileSteps; ++i)
+        if (tile.row(i) < tile.rows) atomicAdd(&count[in.digit(tile.pair[i].x)], 1);
+    __syncthreads();
+    for (int d = threadIdx.x; d < kDigits; d += kTileThreads) hist[blockIdx.x * (int64_t)kDigits + d] = count[d];
+    if (kFirst) {
+        int s = 0;
+#pragma unroll
+        for (int i = 0; i < kTileSteps; ++i) s += __syncthreads_count(tile.row(i) < tile.rows && tile.pair[i].x == in.n_tets + 1);
+        if (threadIdx.x == 0) settled[blockIdx.x] = s;
+    }
+}
+
+// First row of every (tile, digit): by digit, then by tile.  A workgroup takes
+// 64 digits of a chunk of tiles.  sums: rows per (chunk, digit).
+constexpr int kChunkWaves = 4;
+__device__ inline int64_t chunk_first(int64_t tiles, int chunk) { return tiles * chunk / kChunks; }
+__global__ void __launch_bounds__(64 * kChunkWaves) digit_sums_kernel(const int32_t* __restrict__ hist, int64_t tiles,
+                                                                      int32_t* __restrict__ sums)
+{
+    __shared__ int32_t part[kChunkWaves][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, d = blockIdx.x * 64 + lane;
+    const int64_t a = chunk_first(tiles, blockIdx.y), b = chunk_first(tiles, blockIdx.y + 1);
+    int32_t v = 0;
+    for (int64_t t = a + wave; t < b; t += kChunkWaves) v += hist[t * kDigits + d];
+    part[wave][lane] = v;
+    __syncthreads();
+    if (wave == 0) sums[blockIdx.y * kDigits + d] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+}
+// sums -> first row of each (chunk, digit); one workgroup
+__global__ void __launch_bounds__(kDigits / 2) digit_bases_kernel(int32_t* __restrict__ sums)
+{
+    __shared__ int32_t s_wave[kDigits / 128];
+    const int d = 2 * threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int32_t c0[kChunks], c1[kChunks], t0 = 0, t1 = 0;
+#pragma unroll
+    for (int k = 0; k < kChunks; ++k) {
+        const int2 c = *(const int2*)&sums[k * kDigits + d];
+        c0[k] = c.x;
+        c1[k] = c.y;
+        t0 += c.x;
+        t1 += c.y;
+    }
+    int32_t upto = t0 + t1;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int32_t w = __shfl_up(upto, off);
+        if (lane >= off) upto += w;
+    }
+    if (lane == 63) s_wave[wave] = upto;
+    __syncthreads();
+    int32_t r0 = upto - t0 - t1;
+    for (int w = 0; w < wave; ++w) r0 += s_wave[w];
+    int32_t r1 = r0 + t0;
+#pragma unroll
+    for (int k = 0; k < kChunks; ++k) {
+        *(int2*)&sums[k * kDigits + d] = make_int2(r0, r1);
+        r0 += c0[k];
+        r1 += c1[k];
+    }
+}
+// hist -> first row, in place; a thread per (chunk, digit)
+__global__ void __launch_bounds__(64) digit_starts_kernel(int32_t* __restrict__ hist, int64_t tiles,
+                                                          const int32_t* __restrict__ sums)
+{
+    const int d = blockIdx.x * 64 + threadIdx.x;
+    const int64_t a = chunk_first(tiles, blockIdx.y), b = chunk_first(tiles, blockIdx.y + 1);
+    int32_t r = sums[blockIdx.y * kDigits + d];
+    int64_t t = a;
+    for (; t + 8 <= b; t += 8) {
+        int32_t c[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) c[q] = hist[(t + q) * kDigits + d];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            hist[(t + q) * kDigits + d] = r;
+            r += c[q];
+        }
+    }
+    for (; t < b; ++t) {
+        const int32_t c = hist[t * kDigits + d];
+        hist[t * kDigits + d] = r;
+        r += c;
+    }
+}
+
+// Every row to its place by the pass's digit, rows of one digit in the order
+// they had (start: the first row of each (tile, digit)).  Lanes of equal digit find each
+// other by one ballot per bit; the counters are a wave's own, so nothing is
+// added atomically.  The last pass leaves the rows alone.
+template <bool kFirst>
+__global__ void __launch_bounds__(kTileThreads, 8) radix_place_kernel(RadixIn in, const int32_t* __restrict__ start,
+                                                                      int2* __restrict__ pairs_out,
+                                                                      int32_t* __restrict__ rows_out)
+{
+    __shared__ uint16_t count[kTileWaves][kDigits];  // at most kTileRows
+    const int wave = threadIdx.x >> 6;
+    RadixTile<kFirst> tile;
+    tile.load(in);
+    int32_t at[kTileSteps];
+    for (int d = threadIdx.x; d < kTileWaves * kDigits / 2; d += kTileThreads) ((uint32_t*)count)[d] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kTileSteps; ++i) {
+        const int32_t d = in.digit(tile.pair[i].x);
+        const bool valid = tile.row(i) < tile.rows;
+        const unsigned long long live = __ballot(valid);
+        uint32_t lo = (uint32_t)live, hi = (uint32_t)(live >> 32);  // lanes of this digit
+#pragma unroll
+        for (int b = 0; b < kDigitBits; ++b) {
+            const uint32_t bit = (uint32_t)((int32_t)((uint32_t)d << (31 - b)) >> 31);  // in every place
+            const unsigned long long m = __ballot(bit);
+            lo &= ~((uint32_t)m ^ bit);
+            hi &= ~((uint32_t)(m >> 32) ^ bit);
+        }
+        const int before = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+        // (a wave's LDS accesses keep their order)
+        const int32_t c = count[wave][d];
+        at[i] = c + before;
+        if (valid && before == 0) count[wave][d] = (uint16_t)(c + __popc(lo) + __popc(hi));
+        asm volatile("" ::: "memory");
+    }
+    __syncthreads();
+    for (int d = threadIdx.x; d < kDigits; d += kTileThreads) {
+        uint16_t c[kTileWaves], sum = 0;  // of the earlier waves
+#pragma unroll
+        for (int w = 0; w < kTileWaves; ++w) c[w] = count[w][d];
+#pragma unroll
+        for (int w = 0; w < kTileWaves; ++w) {
+            count[w][d] = sum;
+            sum += c[w];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kTileSteps; ++i) {
+        const unsigned d = (unsigned)in.digit(tile.pair[i].x);
+        at[i] += (start + blockIdx.x * (int64_t)kDigits)[d] + count[wave][d];
+    }
+#pragma unroll
+    for (int i = 0; i < kTileSteps; ++i) {
+        // (a place past the end: only if an earlier launch failed)
+        if (tile.row(i) >= tile.rows || (unsigned)at[i] >= (uint64_t)in.n) continue;
+        if (pairs_out) pairs_out[(unsigned)at[i]] = tile.pair[i];
+        else rows_out[(unsigned)at[i]] = tile.pair[i].y;
+    }
+}
+
+// Row perm[j] to j, two arrays at a time (with all ten loads in flight the
+// lines of a wave drive each other out of the caches: 1,745 against 1,574 us
+// for 16M nearly ordered rows).  The live rows lead: all but the settled ones
+// of the tiles.
+template <typename R>
+__global__ void __launch_bounds__(256) gather_rows_kernel(DevParticles<R> src, R* __restrict__ x, R* __restrict__ y,
+                                                          R* __restrict__ z, double* __restrict__ vx,
+                                                          double* __restrict__ vy, double* __restrict__ vz,
+                                                          int32_t* __restrict__ tet, int32_t* __restrict__ flags,
+                                                          int32_t* __restrict__ hit, uint32_t* __restrict__ pidx,
+                                                          const int32_t* __restrict__ perm, int64_t n,
+                                                          const int32_t* __restrict__ settled, int64_t tiles,
+                                                          int64_t* __restrict__ n_active)
+{
+    const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (j < n) {
+        const int64_t s = min((int64_t)(uint32_t)perm[j], n - 1);
+        x[j] = src.x[s];
+        y[j] = src.y[s];
+        asm volatile("" ::: "memory");
+        z[j] = src.z[s];
+        vx[j] = src.vx[s];
+        asm volatile("" ::: "memory");
+        vy[j] = src.vy[s];
+        vz[j] = src.vz[s];
+        asm volatile("" ::: "memory");
+        tet[j] = src.tet[s];
+        flags[j] = src.flags[s];
+        asm volatile("" ::: "memory");
+        hit[j] = src.hit[s];
+        pidx[j] = src.pidx[s];
+    }
+    if (blockIdx.x == 0) {
+        __shared__ int32_t part[4];
+        int32_t v = 0;
+        for (int64_t t = threadIdx.x; t < tiles; t += 256) v += settled[t];
+        v = wave_sum(v);
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+        __syncthreads();
+        if (threadIdx.x == 0) *n_active = n - ((part[0] + part[1]) + (part[2] + part[3]));
+    }
+}
+
 // Scratch of the sort besides the ranks, in int32: the key counts (zero
 // before the first sort), the key starts, the workgroup sums.
 size_t sort_scratch_len(int64_t n_tets)
@@ -186,10 +446,42 @@ size_t sort_zeroed_len(int64_t n_tets) { return (size_t)padded_keys(n_tets); }
 template <typename R>
 hipError_t sort_particles(hipStream_t s, const DevParticles<R>& P, R* x, R* y, R* z, double* vx, double* vy, double* vz,
                           int32_t* tet, int32_t* flags, int32_t* hit, uint32_t* pidx, int32_t* rank, int32_t* scratch,
-                          int32_t n_tets, int64_t* n_active)
+                          WorkItem* work, int32_t n_tets, int64_t* n_active)
 {
     const int64_t n = P.n;
     if (n == 0) return hipSuccess;
+    if (n >= kRadixRows) {
+        const int64_t tiles = (n + kTileRows - 1) / kTileRows;
+        // pairs (two sets), counts and their sums in the work list's rows
+        static_assert(kRadixRows * sizeof(WorkItem) >=
+                          kRadixRows * 2 * sizeof(int2) +
+                              (kRadixRows / kTileRows + 1) * (kDigits + 1) * sizeof(int32_t) +
+                              kDigits * kChunks * sizeof(int32_t) && sizeof(WorkItem) >= 2 * sizeof(int2) + 2,
+                      "scratch of the radix sort");
+        int2* pairs[2] = {(int2*)work, (int2*)work + n};
+        int32_t *hist = (int32_t*)(pairs[1] + n), *sums = hist + kDigits * tiles, *settled = sums + kDigits * kChunks;
+        int32_t* const perm = rank;
+        const unsigned tb = (unsigned)tiles;
+        const dim3 parts(kDigits / 64, kChunks);
+        RadixIn in{P.tet, P.flags, nullptr, n, n_tets, 0};
+        for (int set = 0;; set ^= 1) {
+            const bool first = in.shift == 0, last = ((int64_t)n_tets + 1) >> in.shift < kDigits;
+            int2* const out = last ? nullptr : pairs[set];
+            if (first) radix_count_kernel<true><<<tb, kTileThreads, 0, s>>>(in, hist, settled);
+            else radix_count_kernel<false><<<tb, kTileThreads, 0, s>>>(in, hist, settled);
+            digit_sums_kernel<<<parts, 64 * kChunkWaves, 0, s>>>(hist, tiles, sums);
+            digit_bases_kernel<<<1, kDigits / 2, 0, s>>>(sums);
+            digit_starts_kernel<<<parts, 64, 0, s>>>(hist, tiles, sums);
+            if (first) radix_place_kernel<true><<<tb, kTileThreads, 0, s>>>(in, hist, out, perm);
+            else radix_place_kernel<false><<<tb, kTileThreads, 0, s>>>(in, hist, out, perm);
+            if (last) break;
+            in.pairs = out;
+            in.shift += kDigitBits;
+        }
+        gather_rows_kernel<R><<<(unsigned)((n + 255) / 256), 256, 0, s>>>(P, x, y, z, vx, vy, vz, tet, flags, hit, pidx,
+                                                                           perm, n, settled, tiles, n_active);
+        return hipGetLastError();
+    }
     const int64_t keys = padded_keys(n_tets);
     int32_t *count = scratch, *start = scratch + keys, *sums = scratch + 2 * keys;
     const unsigned nb = (unsigned)((n + 255) / 256), kb = (unsigned)(keys / kScan);
@@ -202,9 +494,9 @@ hipError_t sort_particles(hipStream_t s, const DevParticles<R>& P, R* x, R* y, R
 
 template hipError_t sort_particles<double>(hipStream_t, const DevParticles<double>&, double*, double*, double*,
                                            double*, double*, double*, int32_t*, int32_t*, int32_t*, uint32_t*,
-                                           int32_t*, int32_t*, int32_t, int64_t*);
+                                           int32_t*, int32_t*, WorkItem*, int32_t, int64_t*);
 template hipError_t sort_particles<float>(hipStream_t, const DevParticles<float>&, float*, float*, float*, double*,
                                           double*, double*, int32_t*, int32_t*, int32_t*, uint32_t*, int32_t*,
-                                          int32_t*, int32_t, int64_t*);
+                                          int32_t*, WorkItem*, int32_t, int64_t*);
 
 }  // namespace sg

@@ -62,7 +62,7 @@ size_t sort_zeroed_len(int64_t n_tets);
 template <typename R>
 hipError_t sort_particles(hipStream_t s, const DevParticles<R>& P, R* x, R* y, R* z, double* vx, double* vy, double* vz,
                           int32_t* tet, int32_t* flags, int32_t* hit, uint32_t* pidx, int32_t* rank, int32_t* scratch,
-                          int32_t n_tets, int64_t* n_active);
+                          WorkItem* work, int32_t n_tets, int64_t* n_active);
 }  // namespace sg
 
 using namespace sg;
@@ -432,7 +432,7 @@ hipError_t sort_typed(start_ctx* c)
 {
     PBuf& B = c->B;
     return sort_particles<R>(c->stream, c->view<R>(), (R*)B.x, (R*)B.y, (R*)B.z, (double*)B.vx, (double*)B.vy, (double*)B.vz, B.tet,
-                             B.flags, B.hit, B.pidx, c->d_rank, c->d_sort, (int32_t)c->hm.n_tets, c->d_nactive);
+                             B.flags, B.hit, B.pidx, c->d_rank, c->d_sort, c->d_wl, (int32_t)c->hm.n_tets, c->d_nactive);
 }
 
 int sort_now(start_ctx* c)
