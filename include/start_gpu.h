@@ -227,8 +227,9 @@ int start_read_tri_counts_runs(start_ctx* ctx, uint64_t* out /* n_runs*n_tris, r
 /* ---- launch configuration and the autotuner ---- */
 typedef struct start_launch_cfg {
     int32_t steps_per_launch; /* steps fused per launch, >= 1                                */
-    int32_t block;            /* threads per workgroup: 128 or 256                            */
-    int32_t persistent;       /* 1: a grid sized to the chip pulls particle tiles from a queue */
+    int32_t block;            /* threads per workgroup: 128 or 256 (single steps: 256)        */
+    int32_t persistent;       /* 1: a grid sized to the chip pulls particle tiles from a queue
+                                 (launches of several steps)                                  */
     int32_t sort_interval;    /* steps between sorts by tet; 0 = never                        */
     int32_t graph;            /* 1: the launches between two sorts are captured once in a
                                  hipGraph and replayed                                        */

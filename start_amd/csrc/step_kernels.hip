@@ -745,7 +745,10 @@ struct RegSink {
     // active: lanes of one run of equal (tet, run offset) -- neighbours in the
     // tet-sorted order -- sum their four weights into the run's first lane
     // (segmented Hillis-Steele over the wavefront), which alone goes to the
-    // inner sink.  One LDS insertion per run instead of one per particle.
+    // inner sink.  One LDS insertion per run instead of one per particle; per
+    // 2^kRounds particles of a run with fewer rounds, which single steps of a
+    // batch take (its runs are short: 109 -> 107 us with 4 of them).
+    template <int kRounds = 6>
     __device__ void flush_wave(const DevMesh& M, int32_t cur, int32_t base, double q)
     {
         if (q == 0.0) cur = -1;
@@ -759,7 +762,7 @@ struct RegSink {
         const unsigned long long hm = __ballot(head);
         const int seg = __popcll(hm & (~0ull >> (63 - lane)));  // runs starting at or below this lane
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
+        for (int d = 1; d < 1 << kRounds; d <<= 1) {
             const int sd = __shfl_down(seg, d);
             const double b0 = __shfl_down(a0, d), b1 = __shfl_down(a1, d), b2 = __shfl_down(a2, d),
                          b3 = __shfl_down(a3, d);
@@ -770,7 +773,8 @@ struct RegSink {
                 a3 += b3;
             }
         }
-        if (!head) cur = -1;  // summed into the run's first lane
+        const int start = 63 - __builtin_clzll(hm & (~0ull >> (63 - lane)));
+        if (((lane - start) & ((1 << kRounds) - 1)) != 0) cur = -1;
         flush(M, cur, base, 1.0);
     }
     // flush_wave with the node window of an LDS sink, when no charge has gone
@@ -1979,14 +1983,15 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
     __syncthreads();  // the LDS table and counter are reused by the next tile
 }
 
-// One tile of a single-step launch of one simulation: each particle's step in
-// registers from load to store.  All charge goes to LDS in the flush at the
-// end of the tile, into a window of consecutive nodes (flush_wave_window).
+// One tile of a single-step launch: each particle's step in registers from load
+// to store.  All charge goes to LDS in the flush at the end of the tile: that of
+// one simulation into a window of consecutive nodes (flush_wave_window), a
+// batch's, whose runs are interleaved, into the hash.
 // HBM and the charge atomics bound it: 227 B per particle-step.  1M particles
 // on 750k tets: FP64 53.4 -> 52.6 us, mixed 57.8 -> 45.0 us; 4M particles FP64
 // 211 -> 183 us.  4 workgroups per CU, no scratch memory; a fifth (half the
 // hash, 96 registers) was slower, 55.5 and 193 us.
-template <typename R, int BS, int HashBits, int Win, bool kWalk>
+template <typename R, int BS, int HashBits, int Win, bool kBatch, bool kWalk, bool kTrack>
 __device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, int64_t n_active, uint32_t step,
                                             unsigned int* blk_processed, int32_t* hk, double* hv, double* wv,
                                             int32_t* s_wbase)
@@ -2019,6 +2024,7 @@ __device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, 
     Lam lam;
     lam.l[0] = lam.l[1] = lam.l[2] = lam.l[3] = 0.0;
     const SpeciesK* kp = A.sp;
+    const RunK* rk = S.runs;
     uint32_t vid = 0;
     if (i0 + tid < n_active) {
         s.f = (P.flags + i0)[tid];
@@ -2029,19 +2035,20 @@ __device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, 
         s.vx = (P.vx + i0)[tid];
         s.vy = (P.vy + i0)[tid];
         s.vz = (P.vz + i0)[tid];
-        vid = (P.pidx + i0)[tid] - S.runs->first;
+        if (kBatch) rk = S.runs + ((uint32_t)s.f >> kRunShift);
+        vid = (P.pidx + i0)[tid] - rk->first;
         if (!(s.f & kSettled)) {
             kp = A.sp + ((s.f >> kSpeciesShift) & 0xff);
             charge = kp->charge;
             s.set_v2();
             TetRec<R> rec;
-            rec.template load<false>(M, S, *kp, S.runs, s.t);
+            rec.template load<kBatch>(M, S, *kp, rk, s.t);
             if (frozen_in_tet(M, S, s)) {
                 rec.bary(s.x, s.y, s.z, lam.l);
                 cur = s.t;
             } else {
                 taken = true;
-                const PConst pc = particle_const(S, kp, S.runs, vid);
+                const PConst pc = particle_const(S, kp, rk, vid);
                 const double tau = tau_of<R>(M);
                 push_in(s, rec);
                 end_point(S, vid, pc.key, step, s, x1, y1, z1);
@@ -2050,6 +2057,7 @@ __device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, 
                 rare = draw || !((s.f & kStrict) && lam.l[0] > tau && lam.l[1] > tau && lam.l[2] > tau &&
                                  lam.l[3] > tau);
                 if (!rare) {
+                    if (kTrack) track_start<R>(M, S, vid + rk->first, s.t, s.x, s.y, s.z);
                     (P.x + i0)[tid] = x1;
                     (P.y + i0)[tid] = y1;
                     (P.z + i0)[tid] = z1;
@@ -2072,8 +2080,9 @@ __device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, 
             const R px = s.x, py = s.y, pz = s.z;
             int outcome = kDone;
             int32_t hit_tri = -1;
+            if (kTrack) track_start<R>(M, S, vid + rk->first, t_in, px, py, pz);
             if (!(x1 == px && y1 == py && z1 == pz)) {  // (a degenerate segment ends here, :188-190)
-                if (draw) collide(S, PConst{kp, S.runs, vid, S.runs->key, 0.0f, 0.0f}, step, s);
+                if (draw) collide(S, PConst{kp, rk, vid, rk->key, 0.0f, 0.0f}, step, s);
                 outcome = move_to<R, kWalk>(M, s, (s.f & kStrict) != 0, x1, y1, z1, lam, hit_tri);
             }
             const uint32_t row = (uint32_t)(i0 + tid);
@@ -2089,15 +2098,18 @@ __device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, 
             }
             if (outcome == kDone) cur = s.t;
             else
-                finish_rare<R, false>(A, outcome, row, vid + S.runs->first, S.runs, s, t_in, px, py, pz, step, 0,
-                                      hit_tri);
+                finish_rare<R, kTrack>(A, outcome, row, vid + rk->first, rk, s, t_in, px, py, pz, step, 0, hit_tri);
         }
     }
     sink.a0 = lam.l[0];
     sink.a1 = lam.l[1];
     sink.a2 = lam.l[2];
     sink.a3 = lam.l[3];
-    if (S.charge) sink.flush_wave_window(M, cur, 0, charge, s_wbase);  // every lane is active here
+    if (S.charge) {  // every lane is active here
+        const int32_t base = kBatch ? (int32_t)rk->node_base : 0;
+        if constexpr (Win > 0) sink.flush_wave_window(M, cur, base, charge, s_wbase);
+        else sink.template flush_wave<2>(M, cur, base, charge);
+    }
     const unsigned long long am = __ballot(taken);
     if ((threadIdx.x & 63) == 0 && am) atomicAdd(blk_processed, (unsigned int)__popcll(am));
     __syncthreads();
@@ -2122,21 +2134,20 @@ __device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, 
 // prefix is covered (one launch for every run of a batch, whatever their
 // sizes).  The charge of a tile is summed in LDS (node window and hash) and
 // flushed with one FP64 atomic per distinct node.
-template <typename R, int BS, bool kBatch, bool kPersistent, bool kWalk, bool kTrack = false, bool kWindow = false,
+template <typename R, int BS, bool kBatch, bool kPersistent, bool kWalk, bool kTrack = false, bool kSingle = false,
           bool kPlain = false>
-__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kWindow ? 4 : 3))) step_main(StepArgs<R> A)
+__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kSingle ? 4 : 3))) step_main(StepArgs<R> A)
 {
     const StepParams& S = A.S;
     unsigned long long* const cnt = A.cnt;
-    // kWindow (single-step launches of one simulation, 256 threads): a
-    // 3,072-node window (24 KB) and a 1,024-slot hash (12 KB), 36 KB in all,
-    // so that four workgroups (the 16 waves the 128-VGPR budget allows) share
-    // a CU's 160 KB.  Otherwise the hash alone, 8 slots per thread: fused
-    // launches add to LDS while they step, and batches interleave their runs
-    // in the tet order.  (The window variant run fused was 5% slower on the
+    // Single-step launches (256 threads) of one simulation: a 3,072-node window
+    // (24 KB) and a 1,024-slot hash (12 KB), 36 KB in all, so that four
+    // workgroups (the 16 waves the 128-VGPR budget allows) share a CU's 160 KB.
+    // Otherwise the hash alone, 8 slots per thread: fused launches add to LDS
+    // while they step, and batches interleave their runs in the tet order.  (The window variant run fused was 5% slower on the
     // 3M-tet chamber, whose node layers lie 6,600 ids apart.)
-    static_assert(!kWindow || (BS == 256 && !kBatch), "the window is for 256-thread single-run launches");
-    constexpr int kWin = kWindow ? 3072 : 0;
+    static_assert(!kSingle || (BS == 256 && !kPersistent), "single steps: 256 threads, a workgroup per tile");
+    constexpr int kWin = kSingle && !kBatch ? 3072 : 0;
     constexpr int kBits = kWin > 0 ? 10 : (BS == 256 ? 11 : 10);
     __shared__ unsigned int blk_processed;
     __shared__ int64_t s_tile;
@@ -2144,7 +2155,7 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kWindow
     __shared__ int32_t hk[1 << kBits];
     __shared__ double hv[1 << kBits];
     __shared__ double wv[kWin > 0 ? kWin : 1];
-    __shared__ TetRows s_rows[kWin > 0 ? 1 : BS];
+    __shared__ TetRows s_rows[kSingle ? 1 : BS];
     const uint32_t step0 = (uint32_t)cnt[kCntStep + S.work_slot];
     {
         // clear the next launch's charge buffers and counters, and give it its first step
@@ -2163,9 +2174,9 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kWindow
     if (!kPersistent) {
         if ((int64_t)blockIdx.x * BS < n_active)  // else the whole block is past the live particles
         {
-            if constexpr (kWindow)
-                single_tile<R, BS, kBits, kWin, kWalk>(A, blockIdx.x, n_active, step0, &blk_processed, hk, hv, wv,
-                                                       &s_wbase);
+            if constexpr (kSingle)
+                single_tile<R, BS, kBits, kWin, kBatch, kWalk, kTrack>(A, blockIdx.x, n_active, step0, &blk_processed,
+                                                                       hk, hv, wv, &s_wbase);
             else
                 step_tile<R, BS, kBits, kBatch, kWalk, kTrack, kPlain>(A, blockIdx.x, n_active, step0, &blk_processed,
                                                                        hk, hv, s_rows);
@@ -2884,7 +2895,27 @@ void launch_step(hipStream_t s, const DevMesh& M, const DevParticles<R>& P, cons
                  unsigned long long* tri_count, const StepLaunch& L, hipEvent_t ev_mid)
 {
     const StepArgs<R> A{M, P, S, sp, node_charge, wl, cnt, tri_count};
-    if (P.n > 0 && S.trk_slot) {
+    if (P.n > 0 && S.nsteps == 1) {
+        // single steps: 256 threads and a workgroup per tile, whatever shape the
+        // fused launches have.  1M particles on 750k tets, in us, FP64 and mixed,
+        // against step_tile in the shape asked for: a batch of 4 runs 107 and
+        // 102 (122, 117); with movement records 70 and 70 (95, 109); block 128
+        // without the walk 51 and 46 (75, 69); persistent 52 and 46 (117, 117)
+        const unsigned grid = blocks_for(P.n, 256);
+        switch ((S.trk_slot ? 4 : 0) + (L.batch ? 2 : 0) + (L.walk ? 1 : 0)) {
+#define SG_STEP_SINGLE(T_, B_, W_) \
+    step_main<R, 256, B_, false, W_, T_, true><<<grid, 256, 0, s>>>(A)
+        case 0: SG_STEP_SINGLE(false, false, false); break;
+        case 1: SG_STEP_SINGLE(false, false, true); break;
+        case 2: SG_STEP_SINGLE(false, true, false); break;
+        case 3: SG_STEP_SINGLE(false, true, true); break;
+        case 4: SG_STEP_SINGLE(true, false, false); break;
+        case 5: SG_STEP_SINGLE(true, false, true); break;
+        case 6: SG_STEP_SINGLE(true, true, false); break;
+        default: SG_STEP_SINGLE(true, true, true); break;
+#undef SG_STEP_SINGLE
+        }
+    } else if (P.n > 0 && S.trk_slot) {
         // movement records: the tracking variants (256-thread workgroups, one per tile)
         const unsigned grid = blocks_for(P.n, 256);
         switch ((L.batch ? 2 : 0) + (L.walk ? 1 : 0)) {
@@ -2896,15 +2927,6 @@ void launch_step(hipStream_t s, const DevMesh& M, const DevParticles<R>& P, cons
         default: SG_STEP_TRACK(true, true); break;
 #undef SG_STEP_TRACK
         }
-    } else if (P.n > 0 && S.nsteps == 1 && !L.persistent && !L.batch && (L.walk || L.block != 128)) {
-        // single-step launches of one simulation: the node-window variants
-        const unsigned grid = blocks_for(P.n, 256);
-        if (L.walk)
-            step_main<R, 256, false, false, true, false, true>
-                <<<grid, 256, 0, s>>>(A);
-        else
-            step_main<R, 256, false, false, false, false, true>
-                <<<grid, 256, 0, s>>>(A);
     } else if (P.n > 0 && !S.charge && S.model == 0 && L.walk && !L.persistent) {
         // neither charge nor gas (electrode optimisation and its adjoint, in
         // its own launch shape): see step_tile
