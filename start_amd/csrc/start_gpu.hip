@@ -279,7 +279,7 @@ struct start_ctx {
         L.walk = cfg.walk ? 1 : 0;
         L.block = cfg.block == 128 && !L.walk ? 128 : 256;
         L.persistent = cfg.persistent ? 1 : 0;
-        L.grid = n_cu * (1024 / L.block);  // 4 waves per SIMD x 4 SIMDs per CU
+        L.grid = n_cu * (768 / L.block);  // all that is resident: 3 waves on each of the 4 SIMDs of a CU
         // per-lane run parameters for several runs; a single run whose field is
         // not E_0 as given takes its increments from the push tables if every
         // species of it has one.  Plates, 262,144 particles, 1,000 steps of
