@@ -1014,6 +1014,7 @@ __device__ inline int walk64(const DevMesh& M, int32_t t, const double* p0, cons
     return kWalkUnsure;
 }
 
+constexpr int32_t kDeferredLane = -1;  // a lane's flags once its particle has deferred
 enum StepOutcome { kDone = 0, kSettledNow = 1, kDeferNow = 2, kFrozenNow = 3 };
 
 // settle record for the adjoint
@@ -1129,9 +1130,17 @@ __device__ inline PConst particle_const(const StepParams& S, const SpeciesK* k, 
     return PConst{k, rk, vid, rk->key, k->coll_a + rk->log2_conc + S.log2_dt, k->coll_b};
 }
 
-// face codes and nodes of a particle's tet
-struct TetRows {
-    int4 nbr, node;
+// face codes and nodes of a particle's tet; of a lane whose particle deferred,
+// the deferred step
+struct Deferral {
+    double x0[3];
+    int32_t t0, k;
+};
+union TetRows {
+    struct {
+        int4 nbr, node;
+    };
+    Deferral deferral;
 };
 
 // The record of one tet as a particle's step uses it: the barycentric map
@@ -1544,13 +1553,36 @@ struct StepArgs {
     unsigned long long* cnt;
     unsigned long long* tri_count;
 };
-// A particle that settled (flags, hit, counters, records) or deferred (work
-// list) in a step from px, py, pz in tet t_before; s: its state after it, which
-// the caller has stored.
+// To the work list: one atomic for the lanes that come together.
+template <typename R>
+__device__ inline void append_work(const StepArgs<R>& A, uint32_t row, const Deferral& d)
+{
+    const unsigned long long dm = __ballot(true);
+    const int lane = __lane_id();
+    const int leader = __ffsll((long long)dm) - 1;
+    unsigned int slot = 0u;
+    if (lane == leader)
+        slot = (unsigned int)atomicAdd(&A.cnt[kCntWork + 2 * A.S.work_slot], (unsigned long long)__popcll(dm));
+    slot = __shfl(slot, leader);
+    WorkItem it;
+    it.x0 = d.x0[0];
+    it.y0 = d.x0[1];
+    it.z0 = d.x0[2];
+    it.i = (int32_t)row;
+    it.t0 = d.t0;
+    it.k = d.k;
+    it.pad = 0;
+    A.wl[slot + (unsigned)__popcll(dm & ((1ull << lane) - 1ull))] = it;
+}
+
+// A particle that settled (flags, hit, counters, records) or deferred (to
+// `stage`, for the work list at the end of the tile, or to the list itself) in a
+// step from px, py, pz in tet t_before; s: its state after it, which the caller
+// has stored.
 template <typename R, bool kTrack>
 __device__ inline void finish_rare(const StepArgs<R>& A, int outcome, uint32_t row, uint32_t li, const RunK* rk,
                                    const PState<R>& s, int32_t t_before, R px, R py, R pz, uint32_t step, int32_t ks,
-                                   int32_t hit_tri)
+                                   int32_t hit_tri, TetRows* stage)
 {
     const StepParams& S = A.S;
     if (outcome == kSettledNow) {
@@ -1566,25 +1598,12 @@ __device__ inline void finish_rare(const StepArgs<R>& A, int outcome, uint32_t r
         }
         return;
     }
-    // work list: one atomic for the lanes that defer together
-    const unsigned long long dm = __ballot(true);
-    const int lane = __lane_id();
-    const int leader = __ffsll((long long)dm) - 1;
-    unsigned int slot = 0u;
-    if (lane == leader)
-        slot = (unsigned int)atomicAdd(&A.cnt[kCntWork + 2 * S.work_slot], (unsigned long long)__popcll(dm));
-    slot = __shfl(slot, leader);
-    double a[3];
-    abs_pos(A.M, t_before, px, py, pz, a);
-    WorkItem it;
-    it.x0 = a[0];
-    it.y0 = a[1];
-    it.z0 = a[2];
-    it.i = (int32_t)row;
-    it.t0 = t_before;
-    it.k = ks;
-    it.pad = 0;
-    A.wl[slot + (unsigned)__popcll(dm & ((1ull << lane) - 1ull))] = it;
+    Deferral d;
+    abs_pos(A.M, t_before, px, py, pz, d.x0);
+    d.t0 = t_before;
+    d.k = ks;
+    if (stage) stage->deferral = d;
+    else append_work(A, row, d);
 }
 
 // What a rare step left: the owner, the outcome, and the charge weights lam,
@@ -1607,7 +1626,7 @@ struct RareStep {
 // it was slower too, for the calling convention's saves.)
 template <typename R, bool kBatch, bool kWalk, bool kTrack, bool kPlain>
 __device__ __forceinline__ RareStep rare_step(const StepArgs<R>& A, uint32_t row, uint32_t step, int32_t ks, int32_t remaining,
-                                           bool go)
+                                           bool go, TetRows* stage)
 {
     RareStep r{{{0.0, 0.0, 0.0, 0.0}}, -1, kDone, 0};
     if (!go) return r;
@@ -1665,7 +1684,7 @@ __device__ __forceinline__ RareStep rare_step(const StepArgs<R>& A, uint32_t row
     if (s.t != t_before) P.tet[row] = s.t;
     if (s.t < 0 && t_before >= 0) P.flags[row] = s.f & ~kStrict;
     if (r.outcome != kDone)
-        finish_rare<R, kTrack>(A, r.outcome, row, li, rk, s, t_before, px, py, pz, step, ks, hit_tri);
+        finish_rare<R, kTrack>(A, r.outcome, row, li, rk, s, t_before, px, py, pz, step, ks, hit_tri, stage);
     return r;
 }
 
@@ -1812,7 +1831,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                 // (a degenerate segment ends before the collision, :188-190)
                 if (alive && draw && !rare && !(x1 == s.x && y1 == s.y && z1 == s.z)) collide(S, pc, step, n);
             }
-            bool settles = false;
+            bool settles = false, defers = false;
             if (__ballot(alive && (rare || !inside)) != 0) {
                 if (alive && !rare && !inside) {
                     if (s.t < 0) {
@@ -1824,6 +1843,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                         int fneg = 0;
                         int f = kFar ? exit_face(tau, lam.l, [&](double* l0) { rec.bary(s.x, s.y, s.z, l0); })
                                      : (classify(lam.l, tau, fneg) == kOneFace ? fneg : (int)kNoFace);
+                        const bool one_face = f >= 0;
                         if (f < 0) inside = inside64(M, s.t, x1, y1, z1, lam.l);
                         if (f >= 0) {
                             int32_t code = (&rows->nbr.x)[f];
@@ -1857,6 +1877,19 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                             } else if (f >= 0 && code <= -2) {
                                 settles = true;  // on triangle -2 - code
                                 s.f = code;
+                            }
+                        }
+                        if constexpr (!kWalk) {
+                            // Deferred, as relocate() has it: what is neither
+                            // certified nor an exit through an open face (f is
+                            // then still that face).  Without the walk most
+                            // long segments are (10 steps of 1M particles, dt
+                            // 1e-6 in 1 cm tets: 942 -> 499 us against
+                            // rare_step).
+                            const bool known = std::is_same<R, double>::value || one_face;
+                            if (!inside && !settles && f < 0 && known && !(x1 == s.x && y1 == s.y && z1 == s.z)) {
+                                defers = true;
+                                if (!one_face && has_charge && charge != 0.0) sink.flush_nodes(rows->node, base, charge);
                             }
                         }
                         if constexpr (kWalk && !std::is_same<R, double>::value) {
@@ -1896,11 +1929,11 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                 }
                 rare = rare || !inside;
             }
-            if (kTrack && alive && (!rare || settles)) track_start<R>(M, S, vid + rk->first, t0, s.x, s.y, s.z);
-            if (__builtin_expect(__ballot(settles) != 0, 0)) {
-                if (settles) {
+            if (kTrack && alive && (!rare || settles || defers)) track_start<R>(M, S, vid + rk->first, t0, s.x, s.y, s.z);
+            if (__builtin_expect(__ballot(settles || defers) != 0, 0)) {
+                if (settles || defers) {
                     const R px = s.x, py = s.y, pz = s.z;
-                    const int32_t tri = -2 - s.f;
+                    const int32_t tri = settles ? -2 - s.f : -1;
                     s.f = (P.flags + i0)[tid];
                     s.x = x1;  // in the frame of the owner it leaves
                     s.y = y1;
@@ -1909,12 +1942,19 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                     s.vy = n.vy;
                     s.vz = n.vz;
                     write_state();
-                    finish_rare<R, kTrack>(A, kSettledNow, (uint32_t)(i0 + tid), vid + rk->first, rk, s, t0, px, py,
-                                           pz, step, ks, tri);
+                    finish_rare<R, kTrack>(A, settles ? kSettledNow : kDeferNow, (uint32_t)(i0 + tid), vid + rk->first,
+                                           rk, s, t0, px, py, pz, step, ks, tri, rows);
                     atomicAdd(blk_processed, (unsigned int)ks + 1u);
                     alive = false;
+                    if (defers) s.f = kDeferredLane;
                     s.t = -1;
                     rec.template load<kBatch>(M, S, k, rk, -1, rows);
+                }
+                if constexpr (!kWalk) {
+                    if (__ballot(alive) == 0) {  // a wave can defer as a whole
+                        ks = nsteps;
+                        break;
+                    }
                 }
             }
             if (!rare) {
@@ -1943,7 +1983,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
         const int32_t t_before = s.t;
         const RareStep r = rare_step<R, kBatch, kWalk, kTrack, kPlain>(
             A, (uint32_t)(i0 + tid), step0 + (uint32_t)ks, ks,
-            nsteps - ks, rare);
+            nsteps - ks, rare, rows);
         asm volatile("" ::: "memory");
         if (rare) {
             const bool done = r.outcome != kDone;
@@ -1956,6 +1996,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
                 const unsigned int taken = (unsigned int)ks + (r.outcome == kFrozenNow ? 0u : 1u);
                 if (taken) atomicAdd(blk_processed, taken);
                 alive = false;
+                if (r.outcome == kDeferNow) s.f = kDeferredLane;
             }
             s.t = done ? -1 : r.t;
         }
@@ -1966,6 +2007,10 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
         ++ks;
     }
     if (alive) write_state();
+    // The particles that deferred, of all steps together: where most of them do
+    // (10 steps of 1M particles, no walk), the wave's atomics in every step, all
+    // to one address, took 1.0 of 1.95 ms.
+    if (s.f == kDeferredLane) append_work(A, (uint32_t)(i0 + tid), rows->deferral);
     if (!alive) sink.a0 = sink.a1 = sink.a2 = sink.a3 = 0.0;  // flushed when it stopped
     if (has_charge) sink.flush_wave(M, s.t, base, charge);  // every lane is active here
     // processed particle-steps: LDS per block, one atomic per tile spread over slots
@@ -2098,7 +2143,8 @@ __device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, 
             }
             if (outcome == kDone) cur = s.t;
             else
-                finish_rare<R, kTrack>(A, outcome, row, vid + rk->first, rk, s, t_in, px, py, pz, step, 0, hit_tri);
+                finish_rare<R, kTrack>(A, outcome, row, vid + rk->first, rk, s, t_in, px, py, pz, step, 0, hit_tri,
+                                       nullptr);
         }
     }
     sink.a0 = lam.l[0];
@@ -2245,8 +2291,13 @@ __global__ void __launch_bounds__(64) step_resolve(DevMesh M, DevParticles<R> P,
     const uint32_t step0 = (uint32_t)cnt[kCntStep + S.work_slot];
     // Items go to the waves in turn: lanes of one wave wait for each other's
     // exact work (10 us and more an item), waves do not.  16 runs of 1e4 to 4e5
-    // particles, mixed, 200 steps, 123 items: 640-860 -> 390 us.
-    for (uint64_t w = blockIdx.x + (uint64_t)gridDim.x * threadIdx.x; w < nw; w += (uint64_t)gridDim.x * blockDim.x) {
+    // particles, mixed, 200 steps, 123 items: 640-860 -> 390 us.  A list that
+    // fills the lanes is taken in order (2.3M items over 6 launches: 8.9 -> 8.2
+    // ms; the rows of neighbouring items are neighbours).
+    const uint64_t lanes = (uint64_t)gridDim.x * blockDim.x;
+    const uint64_t first = nw < lanes ? blockIdx.x + (uint64_t)gridDim.x * threadIdx.x
+                                      : blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+    for (uint64_t w = first; w < nw; w += lanes) {
         RegSink<GlobalSink> sink{GlobalSink{node_charge}, 0.0, 0.0, 0.0, 0.0};
         WorkItem it = wl[w];
         int64_t i = it.i;
