@@ -43,9 +43,13 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, GB/s
-# VALU issue rate: 256 CUs x 4 SIMDs, one wave64 instruction per SIMD every 4
-# cycles (16 lanes) at the 2.4 GHz peak engine clock, in wave-instructions/s
-VALU_PEAK = 256 * 4 * 2.4e9 / 4
+# VALU issue rate: 256 CUs x 4 SIMDs at the 2.4 GHz peak engine clock, one
+# wave64 instruction per SIMD every 2 cycles, in wave-instructions/s.  Measured
+# with every SIMD full: two-operand 32-bit instructions (add, multiply, shift,
+# logic, move) one every 2.2-2.5 cycles; FMA, compares, 32-bit integer products
+# and FP64 one every 4.1-5.1.  The kernels mix both, so this bounds them, and
+# one every 4 cycles does not (the batched sweep has exceeded it).
+VALU_PEAK = 256 * 4 * 2.4e9 / 2
 # algorithmic bytes per particle-step of the streaming step:
 #   2*(3s + 3*8 + 8) particle state (positions in s bytes, velocities FP64)
 #   + (3 s_E + 12 s_G + 16 + 16) tet record + 4*8 charge

@@ -126,22 +126,6 @@ __device__ inline uint32_t hash3(uint32_t a, uint32_t b, uint32_t c)
     return h;
 }
 
-// B = 0 push: v = (v + h) + h, h = (((E*q)/m)*dt)/2 per component; skipped when
-// dt == 0 or E == 0 exactly (Particle.cpp:199-207).  h in R, the velocity
-// (always FP64 state) accumulated in V.
-template <typename R, typename V>
-__device__ inline void push(R ex, R ey, R ez, R q, R m, R dt, V& vx, V& vy, V& vz)
-{
-    if (dt == R(0)) return;
-    if (ex == R(0) && ey == R(0) && ez == R(0)) return;
-    V hx = (V)((((ex * q) / m) * dt) / R(2));
-    V hy = (V)((((ey * q) / m) * dt) / R(2));
-    V hz = (V)((((ez * q) / m) * dt) / R(2));
-    vx = (vx + hx) + hx;
-    vy = (vy + hy) + hy;
-    vz = (vz + hz) + hz;
-}
-
 template <typename R>
 struct CollideK {
     R sigma_hs, vhs_c, two_kt, m_r, vhs_exp, mass_cp, mass_ct, inv_alpha;

@@ -2548,9 +2548,10 @@ __global__ void node_density_bary_kernel(const double* __restrict__ q, const dou
     if (written) written[n] = 1;
 }
 
-// Push increments h = (((E*q)/m)*dt)/2 of field basis 0 for each charged
-// species slot (push<R>'s arithmetic, FP64 from E and FP32 from the FP32 field),
-// -0 where push<R> returns early (dt == 0 or E == 0 exactly).
+// Push increments h = (((E*q)/m)*dt)/2 of a single run's field for each charged
+// species slot (TetRec::load_h's arithmetic, FP64 from E and FP32 from the FP32
+// field), -0 where the push is skipped (dt == 0 or E == 0 exactly,
+// Particle.cpp:199-207).
 struct PushSlots {
     double q[kMaxPushSlots], m[kMaxPushSlots];
     int32_t n;
