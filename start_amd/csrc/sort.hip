@@ -14,8 +14,8 @@
 // 6 us each.  With one sort each, 200 fused steps of 1M particles on 750k tets
 // went from 1.17 to 1.09 ms, 100 steps of 150,001 particles on 179k tets from
 // 274 to 233 us.
-// Populations of kRadixRows and more are radix sorted instead (below): their
-// ranks' atomics and scattered stores cost more than its passes.
+// Large populations whose ranks' atomics and scattered stores cost more are
+// radix sorted instead (below).
 // The order of the rows of one key is not fixed (nothing depends on it but
 // the order in which charges are added).
 #include "kernels.h"
@@ -179,23 +179,30 @@ __global__ void place_kernel(DevParticles<R> src, R* __restrict__ x, R* __restri
 
 // ---------------------------------------------------------------------------
 // Large populations: radix sort of (key, row) by 11 bits a pass, two passes for
-// up to 4M tets, then a gather.  Five short launches a pass; the gather's random
+// up to 4M tets, then a gather.  Four short launches a pass; the gather's random
 // reads bound it.  A sort in us, FP64, by a library radix sort and gather, by the
 // counting sort, by this one:
 //   rows on tets          unordered              nearly ordered
-//   1M on 374k        324    294    241      220    125    159
-//   2M on 3M          454    578    448      270    300    264
-//   2M on 750k        479    562    473      164     75    139
-//   8M on 3M        1,737  2,119  1,705    1,010  1,230    976
-//   8M on 750k      1,788  2,288  1,781      455    335    365
-//   16M on 3M       3,510  5,030  3,412    2,070  2,350  1,948
-//   24.6M on 750k   6,287  9,109  6,192    1,350  1,100  1,040
-// (nearly ordered: on 3M and 374k tets particles cross some two tets between
-// sorts, on 750k few do).  From 1.5M rows on it is never slower than the
-// library's, which the counting sort is where rows move; below, the counting
-// sort's four launches are.
+//   1M on 374k        324    294    225      220    125    143
+//   2M on 3M          461    578    432      271    300    250
+//   2M on 750k        480    562    455      164     75    123
+//   4M on 720k        860  1,199    845      466    575    440
+//   4M on 750k        910    890    882      240    153    201
+//   8M on 3M        1,737  2,119  1,690    1,010  1,230    960
+//   8M on 750k      1,788  2,288  1,765      455    335    350
+//   16M on 3M       3,500  5,030  3,400    2,090  2,350  1,940
+//   24.6M on 750k   6,300  9,109  6,190    1,355  1,100  1,030
+// (nearly ordered: on 3M, 720k and 374k tets particles cross some two tets
+// between sorts, on 750k few do.)  Where the rows are new (in no order), 1M of
+// them suffice; where fewer than two share a tet, every row is a run of its own
+// to the counting sort, and 1.5M do; else it is the rows that moved, which the
+// host does not know, and from 4M on this one is taken as the library's was.
 // ---------------------------------------------------------------------------
-constexpr int64_t kRadixRows = 1'500'000;
+constexpr int64_t kRadixRows = 1'000'000;
+static bool use_radix(int64_t n, int64_t n_tets, bool unordered)
+{
+    return n >= 4 * kRadixRows || (unordered && n >= kRadixRows) || (2 * n >= 3 * kRadixRows && n < 2 * n_tets);
+}
 constexpr int kDigitBits = 11, kDigits = 1 << kDigitBits;
 constexpr int kTileThreads = 1024, kTileWaves = kTileThreads / 64, kTileSteps = 8;
 constexpr int kTileRows = kTileThreads * kTileSteps;
@@ -256,8 +263,7 @@ __global__ void __launch_bounds__(kTileThreads, 8) radix_count_kernel(RadixIn in
     }
 }
 
-// First row of every (tile, digit): by digit, then by tile.  A workgroup takes
-// 64 digits of a chunk of tiles.  sums: rows per (chunk, digit).
+// A workgroup takes 64 digits of a chunk of tiles.  sums: rows per (chunk, digit).
 constexpr int kChunkWaves = 4;
 __device__ inline int64_t chunk_first(int64_t tiles, int chunk) { return tiles * chunk / kChunks; }
 __global__ void __launch_bounds__(64 * kChunkWaves) digit_sums_kernel(const int32_t* __restrict__ hist, int64_t tiles,
@@ -272,45 +278,19 @@ __global__ void __launch_bounds__(64 * kChunkWaves) digit_sums_kernel(const int3
     __syncthreads();
     if (wave == 0) sums[blockIdx.y * kDigits + d] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
 }
-// sums -> first row of each (chunk, digit); one workgroup
-__global__ void __launch_bounds__(kDigits / 2) digit_bases_kernel(int32_t* __restrict__ sums)
-{
-    __shared__ int32_t s_wave[kDigits / 128];
-    const int d = 2 * threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int32_t c0[kChunks], c1[kChunks], t0 = 0, t1 = 0;
-#pragma unroll
-    for (int k = 0; k < kChunks; ++k) {
-        const int2 c = *(const int2*)&sums[k * kDigits + d];
-        c0[k] = c.x;
-        c1[k] = c.y;
-        t0 += c.x;
-        t1 += c.y;
-    }
-    int32_t upto = t0 + t1;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int32_t w = __shfl_up(upto, off);
-        if (lane >= off) upto += w;
-    }
-    if (lane == 63) s_wave[wave] = upto;
-    __syncthreads();
-    int32_t r0 = upto - t0 - t1;
-    for (int w = 0; w < wave; ++w) r0 += s_wave[w];
-    int32_t r1 = r0 + t0;
-#pragma unroll
-    for (int k = 0; k < kChunks; ++k) {
-        *(int2*)&sums[k * kDigits + d] = make_int2(r0, r1);
-        r0 += c0[k];
-        r1 += c1[k];
-    }
-}
-// hist -> first row, in place; a thread per (chunk, digit)
+// hist -> place of a tile's rows among those of the digit, in place (a thread
+// per chunk and digit); totals: rows of the digit
 __global__ void __launch_bounds__(64) digit_starts_kernel(int32_t* __restrict__ hist, int64_t tiles,
-                                                          const int32_t* __restrict__ sums)
+                                                          const int32_t* __restrict__ sums,
+                                                          int32_t* __restrict__ totals)
 {
     const int d = blockIdx.x * 64 + threadIdx.x;
     const int64_t a = chunk_first(tiles, blockIdx.y), b = chunk_first(tiles, blockIdx.y + 1);
-    int32_t r = sums[blockIdx.y * kDigits + d];
+    int32_t before[kChunks], r = 0;
+#pragma unroll
+    for (int k = 0; k < kChunks; ++k) before[k] = sums[k * kDigits + d];
+#pragma unroll
+    for (int k = 0; k < kChunks; ++k) r += k < (int)blockIdx.y ? before[k] : 0;
     int64_t t = a;
     for (; t + 8 <= b; t += 8) {
         int32_t c[8];
@@ -327,21 +307,42 @@ __global__ void __launch_bounds__(64) digit_starts_kernel(int32_t* __restrict__ 
         hist[t * kDigits + d] = r;
         r += c;
     }
+    if (blockIdx.y == kChunks - 1) totals[d] = r;
 }
 
 // Every row to its place by the pass's digit, rows of one digit in the order
-// they had (start: the first row of each (tile, digit)).  Lanes of equal digit find each
-// other by one ballot per bit; the counters are a wave's own, so nothing is
-// added atomically.  The last pass leaves the rows alone.
+// they had (start: places of the tiles' rows within the digit).  Lanes of equal
+// digit find each other by one ballot per bit; the counters are a wave's own, so
+// nothing is added atomically.  The last pass leaves the rows alone.
 template <bool kFirst>
 __global__ void __launch_bounds__(kTileThreads, 8) radix_place_kernel(RadixIn in, const int32_t* __restrict__ start,
+                                                                      const int32_t* __restrict__ totals,
                                                                       int2* __restrict__ pairs_out,
                                                                       int32_t* __restrict__ rows_out)
 {
     __shared__ uint16_t count[kTileWaves][kDigits];  // at most kTileRows
-    const int wave = threadIdx.x >> 6;
+    __shared__ int32_t base[kDigits], s_wave[kTileWaves];
+    static_assert(kDigits == 2 * kTileThreads, "two digits a thread");
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     RadixTile<kFirst> tile;
     tile.load(in);
+    {
+        // first row of each digit
+        const int2 c = ((const int2*)totals)[threadIdx.x];
+        int32_t upto = c.x + c.y;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int32_t w = __shfl_up(upto, off);
+            if (lane >= off) upto += w;
+        }
+        if (lane == 63) s_wave[wave] = upto;
+        __syncthreads();
+        int32_t r = upto - c.x - c.y;
+#pragma unroll
+        for (int w = 0; w < kTileWaves; ++w) r += w < wave ? s_wave[w] : 0;
+        base[2 * threadIdx.x] = r;
+        base[2 * threadIdx.x + 1] = r + c.x;
+    }
     int32_t at[kTileSteps];
     for (int d = threadIdx.x; d < kTileWaves * kDigits / 2; d += kTileThreads) ((uint32_t*)count)[d] = 0u;
     __syncthreads();
@@ -380,7 +381,7 @@ __global__ void __launch_bounds__(kTileThreads, 8) radix_place_kernel(RadixIn in
 #pragma unroll
     for (int i = 0; i < kTileSteps; ++i) {
         const unsigned d = (unsigned)in.digit(tile.pair[i].x);
-        at[i] += (start + blockIdx.x * (int64_t)kDigits)[d] + count[wave][d];
+        at[i] += (start + blockIdx.x * (int64_t)kDigits)[d] + base[d] + count[wave][d];
     }
 #pragma unroll
     for (int i = 0; i < kTileSteps; ++i) {
@@ -446,20 +447,21 @@ size_t sort_zeroed_len(int64_t n_tets) { return (size_t)padded_keys(n_tets); }
 template <typename R>
 hipError_t sort_particles(hipStream_t s, const DevParticles<R>& P, R* x, R* y, R* z, double* vx, double* vy, double* vz,
                           int32_t* tet, int32_t* flags, int32_t* hit, uint32_t* pidx, int32_t* rank, int32_t* scratch,
-                          WorkItem* work, int32_t n_tets, int64_t* n_active)
+                          WorkItem* work, int32_t n_tets, bool unordered, int64_t* n_active)
 {
     const int64_t n = P.n;
     if (n == 0) return hipSuccess;
-    if (n >= kRadixRows) {
+    if (use_radix(n, n_tets, unordered)) {
         const int64_t tiles = (n + kTileRows - 1) / kTileRows;
         // pairs (two sets), counts and their sums in the work list's rows
         static_assert(kRadixRows * sizeof(WorkItem) >=
                           kRadixRows * 2 * sizeof(int2) +
                               (kRadixRows / kTileRows + 1) * (kDigits + 1) * sizeof(int32_t) +
-                              kDigits * kChunks * sizeof(int32_t) && sizeof(WorkItem) >= 2 * sizeof(int2) + 2,
+                              kDigits * (kChunks + 1) * sizeof(int32_t) && sizeof(WorkItem) >= 2 * sizeof(int2) + 2,
                       "scratch of the radix sort");
         int2* pairs[2] = {(int2*)work, (int2*)work + n};
-        int32_t *hist = (int32_t*)(pairs[1] + n), *sums = hist + kDigits * tiles, *settled = sums + kDigits * kChunks;
+        int32_t *hist = (int32_t*)(pairs[1] + n), *sums = hist + kDigits * tiles, *totals = sums + kDigits * kChunks,
+                *settled = totals + kDigits;
         int32_t* const perm = rank;
         const unsigned tb = (unsigned)tiles;
         const dim3 parts(kDigits / 64, kChunks);
@@ -470,10 +472,9 @@ hipError_t sort_particles(hipStream_t s, const DevParticles<R>& P, R* x, R* y, R
             if (first) radix_count_kernel<true><<<tb, kTileThreads, 0, s>>>(in, hist, settled);
             else radix_count_kernel<false><<<tb, kTileThreads, 0, s>>>(in, hist, settled);
             digit_sums_kernel<<<parts, 64 * kChunkWaves, 0, s>>>(hist, tiles, sums);
-            digit_bases_kernel<<<1, kDigits / 2, 0, s>>>(sums);
-            digit_starts_kernel<<<parts, 64, 0, s>>>(hist, tiles, sums);
-            if (first) radix_place_kernel<true><<<tb, kTileThreads, 0, s>>>(in, hist, out, perm);
-            else radix_place_kernel<false><<<tb, kTileThreads, 0, s>>>(in, hist, out, perm);
+            digit_starts_kernel<<<parts, 64, 0, s>>>(hist, tiles, sums, totals);
+            if (first) radix_place_kernel<true><<<tb, kTileThreads, 0, s>>>(in, hist, totals, out, perm);
+            else radix_place_kernel<false><<<tb, kTileThreads, 0, s>>>(in, hist, totals, out, perm);
             if (last) break;
             in.pairs = out;
             in.shift += kDigitBits;
@@ -494,9 +495,11 @@ hipError_t sort_particles(hipStream_t s, const DevParticles<R>& P, R* x, R* y, R
 
 template hipError_t sort_particles<double>(hipStream_t, const DevParticles<double>&, double*, double*, double*,
                                            double*, double*, double*, int32_t*, int32_t*, int32_t*, uint32_t*,
-                                           int32_t*, int32_t*, WorkItem*, int32_t, int64_t*);
+                                           int32_t*, int32_t*, WorkItem*, int32_t, bool,
+                                           int64_t*);
 template hipError_t sort_particles<float>(hipStream_t, const DevParticles<float>&, float*, float*, float*, double*,
                                           double*, double*, int32_t*, int32_t*, int32_t*, uint32_t*, int32_t*,
-                                          int32_t*, WorkItem*, int32_t, int64_t*);
+                                          int32_t*, WorkItem*, int32_t, bool,
+                                           int64_t*);
 
 }  // namespace sg

@@ -62,7 +62,7 @@ size_t sort_zeroed_len(int64_t n_tets);
 template <typename R>
 hipError_t sort_particles(hipStream_t s, const DevParticles<R>& P, R* x, R* y, R* z, double* vx, double* vy, double* vz,
                           int32_t* tet, int32_t* flags, int32_t* hit, uint32_t* pidx, int32_t* rank, int32_t* scratch,
-                          WorkItem* work, int32_t n_tets, int64_t* n_active);
+                          WorkItem* work, int32_t n_tets, bool unordered, int64_t* n_active);
 }  // namespace sg
 
 using namespace sg;
@@ -427,18 +427,19 @@ void free_particles(start_ctx* c)
 }
 
 // sort by owning tet, settled particles last, then swap the buffer sets
+// (unordered: the rows are as the caller loaded them)
 template <typename R>
-hipError_t sort_typed(start_ctx* c)
+hipError_t sort_typed(start_ctx* c, bool unordered)
 {
     PBuf& B = c->B;
     return sort_particles<R>(c->stream, c->view<R>(), (R*)B.x, (R*)B.y, (R*)B.z, (double*)B.vx, (double*)B.vy, (double*)B.vz, B.tet,
-                             B.flags, B.hit, B.pidx, c->d_rank, c->d_sort, c->d_wl, (int32_t)c->hm.n_tets, c->d_nactive);
+                             B.flags, B.hit, B.pidx, c->d_rank, c->d_sort, c->d_wl, (int32_t)c->hm.n_tets, unordered, c->d_nactive);
 }
 
-int sort_now(start_ctx* c)
+int sort_now(start_ctx* c, bool unordered = false)
 {
     if (c->n == 0 || !c->B.x) return START_OK;
-    hipError_t e = c->mixed ? sort_typed<float>(c) : sort_typed<double>(c);
+    hipError_t e = c->mixed ? sort_typed<float>(c, unordered) : sort_typed<double>(c, unordered);
     if (e != hipSuccess) return fail(c, START_ERR_HIP, std::string("particle sort: ") + hipGetErrorString(e));
     std::swap(c->A, c->B);
     c->last_sort = c->step;
@@ -1516,7 +1517,7 @@ int start_load_batch(start_ctx* c, int32_t n_runs, const start_run_desc* runs, c
     rc = upload_rows(c, 0, n, x, y, z, vx, vy, vz, species);
     if (rc != START_OK) return rc;
     if (c->cfg.sort_interval > 0) {
-        int rc2 = sort_now(c);
+        int rc2 = sort_now(c, true);
         if (rc2 != START_OK) return rc2;
     }
     return check_kernel_errors(c);

@@ -1,8 +1,9 @@
-"""The sort of large populations at the size where its method changes and with
-a partial last tile (8,192 rows), for one, two and three passes over the key
-bits: the same run never sorted takes every particle to the same state, bit
-for bit (each row moved exactly once), the same number of steps (the live
-prefix holds every particle that moves), and the same charge."""
+"""The sort of large populations at the sizes where its method changes (1M
+rows as loaded, 1.5M with fewer than two a tet, 4M) and with a partial last
+tile (8,192 rows), for one, two and three passes over the key bits: the same
+run never sorted takes every particle to the same state, bit for bit (each row
+moved exactly once), the same number of steps (the live prefix holds every
+particle that moves), and the same charge."""
 from __future__ import annotations
 
 import numpy as np
@@ -15,9 +16,10 @@ from start_amd.species import E_CHARGE
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,cells,precision", [(1_499_999, 12, "fp64"), (1_500_000, 12, "fp64"),
-                                               (1_507_329, 12, "mixed"), (1_500_001, 6, "mixed"),
-                                               (1_500_001, 89, "fp64")])
+@pytest.mark.parametrize("n,cells,precision", [(999_999, 12, "fp64"), (1_000_000, 12, "fp64"),
+                                               (1_007_617, 12, "mixed"), (1_000_001, 6, "mixed"),
+                                               (1_499_999, 51, "mixed"), (1_500_000, 51, "fp64"),
+                                               (1_500_001, 89, "fp64"), (4_000_001, 12, "mixed")])
 def test_sorted_run_equals_the_unsorted_one(n, cells, precision):
     w = workloads.large_box(n_particles=n, cells=cells)
     w.dt = 4e-5 / cells  # a part settles between the sorts
