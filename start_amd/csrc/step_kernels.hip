@@ -1368,21 +1368,25 @@ __device__ inline Relocated<R> relocate(const DevMesh& M, int32_t t, int32_t vne
 
 // Frozen this step and every later one of the launch (nothing changes its
 // state; it still carries charge): 2. |v| < 10 m/s or 3. outside the expanded
-// bbox (ParticleDynamicsProcessor.cpp:166-176).  NaN and infinite positions are
-// outside it.
+// bbox (ParticleDynamicsProcessor.cpp:166-176).  Where the expanded bbox holds
+// every node, a finite point in a tet is inside it.
+template <typename R>
+__device__ inline bool frozen_finite(const DevMesh& M, const StepParams& S, const PState<R>& s)
+{
+    return too_slow(s.v2) || ((s.t < 0 || !S.bbox_covers) && !in_bbox_at(M, S, s.t, s.x, s.y, s.z));
+}
+// A NaN or infinite point, which the exact predicates can give an owner, is
+// outside the bbox.  The common step does without this test: such a point ends
+// its step nowhere certain, and comes here with the rare ones.
+template <typename R>
+__device__ inline bool not_finite(const PState<R>& s)
+{
+    return !((s.x - s.x) + (s.y - s.y) + (s.z - s.z) == R(0));
+}
 template <typename R>
 __device__ inline bool is_frozen(const DevMesh& M, const StepParams& S, const PState<R>& s)
 {
-    return too_slow(s.v2) || !in_bbox_at(M, S, s.t, s.x, s.y, s.z);
-}
-// The same for the common step of a particle, which the expanded bbox does not
-// concern where it holds every node: a finite point in a tet is inside it, and
-// a NaN or infinite one (which the exact predicates can give an owner) ends its
-// step nowhere certain and so comes to is_frozen.
-template <typename R>
-__device__ inline bool frozen_in_tet(const DevMesh& M, const StepParams& S, const PState<R>& s)
-{
-    return too_slow(s.v2) || ((s.t < 0 || !S.bbox_covers) && !in_bbox_at(M, S, s.t, s.x, s.y, s.z));
+    return frozen_finite(M, S, s) || not_finite(s);
 }
 
 // 4. push with the owning tet's field (ParticleDynamicsProcessor.cpp:179-180);
@@ -1474,7 +1478,7 @@ template <typename R, typename Sink>
 __device__ inline bool plain_step(const DevMesh& M, const StepParams& S, const PConst& c, uint32_t step, PState<R>& s,
                                   const TetRec<R>& rec, Sink& sink)
 {
-    if (frozen_in_tet(M, S, s)) return false;
+    if (frozen_finite(M, S, s)) return false;
     PState<R> n = s;
     push_in(n, rec);
     R x1, y1, z1;
@@ -2088,7 +2092,7 @@ __device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, 
             s.set_v2();
             TetRec<R> rec;
             rec.template load<kBatch>(M, S, *kp, rk, s.t);
-            if (frozen_in_tet(M, S, s)) {
+            if (frozen_finite(M, S, s)) {
                 rec.bary(s.x, s.y, s.z, lam.l);
                 cur = s.t;
             } else {
@@ -2116,7 +2120,7 @@ __device__ __forceinline__ void single_tile(const StepArgs<R>& A, int64_t tile, 
     }
     // collisions and segments that leave the tet
     if (__ballot(rare) != 0) {
-        if (rare && !in_bbox_at(M, S, s.t, s.x, s.y, s.z)) {  // (only a NaN or infinite point: frozen)
+        if (rare && not_finite(s)) {  // frozen
             bary_at(M, s.t, s.x, s.y, s.z, lam.l);
             cur = s.t;
             taken = false;
