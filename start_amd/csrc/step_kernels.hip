@@ -1831,12 +1831,12 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
             Lam lam;
             rec.bary(x1, y1, z1, lam.l);
             bool inside = strict && lam.l[0] > tau && lam.l[1] > tau && lam.l[2] > tau && lam.l[3] > tau;
-            if (__ballot(alive && draw && !rare) != 0) {
-                // (a degenerate segment ends before the collision, :188-190)
-                if (alive && draw && !rare && !(x1 == s.x && y1 == s.y && z1 == s.z)) collide(S, pc, step, n);
-            }
             bool settles = false, defers = false;
-            if (__ballot(alive && (rare || !inside)) != 0) {
+            if (__ballot(alive && (rare || draw || !inside)) != 0) {
+                if (__ballot(alive && draw && !rare) != 0) {
+                    // (a degenerate segment ends before the collision, :188-190)
+                    if (alive && draw && !rare && !(x1 == s.x && y1 == s.y && z1 == s.z)) collide(S, pc, step, n);
+                }
                 if (alive && !rare && !inside) {
                     if (s.t < 0) {
                         inside = in_bbox_at(M, S, s.t, s.x, s.y, s.z) && stays_outside(M, s, x1, y1, z1);
