@@ -1712,15 +1712,15 @@ __device__ inline bool inside64(const DevMesh&, int32_t, double, double, double,
 // list with the step it stopped at.  Called with a block-uniform tile.
 // kTrack: movement records on (S.trk_slot set), a kernel variant of its own so
 // that the streaming kernels without them carry none of their code.
-// What bounds a fused launch is VALU issue: a common step is about 150 vector
-// instructions, against 525 when every step read the record again, took an
-// FP32 pow and two square roots for the collision test and ran through the
-// code of the rare cases.  200 steps of 1M particles on 750k tets with their
-// read-back, FP64: 3.31 -> 1.17 ms; of 16 runs of 1e4 to 4e5 particles on
-// 162k tets, mixed: 6.37 -> 3.10 ms.  Where one lane of nearly every wave
+// What bounds a fused launch is the issue and latency of its instructions: a
+// step is about 140 vector instructions (mixed 210), against 525 when every
+// step read the record again, took an FP32 pow and two square roots for the
+// collision test and ran through the code of the rare cases.  200 steps of 1M
+// particles on 750k tets with their read-back, FP64: 3.31 -> 1.00 ms; of 16
+// runs of 1e4 to 4e5 particles on 162k tets, mixed: 6.37 -> 2.42 ms.  Where one lane of nearly every wave
 // changes tet in every step the latency of the next record bounds it and the
-// gain is smaller: 16M particles on 3M tets, 10 steps, FP64 6.2 -> 4.5 ms,
-// mixed 7.3 -> 7.1 ms.
+// gain is smaller: 200 steps of 16M particles on 3M tets, FP64 2.0e10 -> 2.6e10
+// particle-steps/s, mixed 1.71e10 -> 1.77e10.
 // 3 waves per SIMD (168 registers): 4 waves put values of the loop into
 // scratch memory (1.47 ms), 2 waves hide too little of it (1.36 ms).
 // kPlain: neither charge nor gas, without the charge sums, the hash and the
@@ -2036,7 +2036,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<R>& A, int64_t tile, in
 // to store.  All charge goes to LDS in the flush at the end of the tile: that of
 // one simulation into a window of consecutive nodes (flush_wave_window), a
 // batch's, whose runs are interleaved, into the hash.
-// HBM and the charge atomics bound it: 227 B per particle-step.  1M particles
+// HBM and the charge atomics bound it: 219 B per particle-step, mixed 158.  1M particles
 // on 750k tets: FP64 53.4 -> 52.6 us, mixed 57.8 -> 45.0 us; 4M particles FP64
 // 211 -> 183 us.  4 workgroups per CU, no scratch memory; a fifth (half the
 // hash, 96 registers) was slower, 55.5 and 193 us.
@@ -2194,8 +2194,9 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kSingle
     // (24 KB) and a 1,024-slot hash (12 KB), 36 KB in all, so that four
     // workgroups (the 16 waves the 128-VGPR budget allows) share a CU's 160 KB.
     // Otherwise the hash alone, 8 slots per thread: fused launches add to LDS
-    // while they step, and batches interleave their runs in the tet order.  (The window variant run fused was 5% slower on the
-    // 3M-tet chamber, whose node layers lie 6,600 ids apart.)
+    // while they step, and batches interleave their runs in the tet order.  (The
+    // window run fused was 5% slower on the 3M-tet chamber, whose node layers lie
+    // 6,600 ids apart.)
     static_assert(!kSingle || (BS == 256 && !kPersistent), "single steps: 256 threads, a workgroup per tile");
     constexpr int kWin = kSingle && !kBatch ? 3072 : 0;
     constexpr int kBits = kWin > 0 ? 10 : (BS == 256 ? 11 : 10);
